@@ -138,13 +138,13 @@ SINGLE_ANCHOR_TILES = (
 )
 
 # 16-wave tiles (4 waves per SIMD): offered when the operand chunks leave the
-# registers for it (no full-size gathered prologue operands) -- measured on
-# MI355X with direct-to-LDS loads: 4096^3 977.7 -> 968.0 us (2x8 waves of
-# 128x32), C4 X @ W1 2650 -> 2609 us, C5 S 287.2 -> 283.6 us, C5 P @ V
-# 280.3 -> 274.2 us (256x128 as 4x4 waves of 64x32).  4x4 waves of 64x64 on
-# 256x256 were slower than 2x8 (987 us).
+# registers for it (no full-size gathered prologue operands).  4x4 waves of
+# 64x64 on 256x256: a wave splits the operand fragments it multiplies into
+# bf16 parts, (64 + 64) x 32 elements a chunk for square wave tiles against
+# (128 + 32) x 32 for 2x8 waves of 128x32 (measured on MI355X, 4096^3: 750
+# against 787 us; 8 waves of 128x64 731 us).
 WIDE_TILES = (
-    TileConfig(256, 256, 32, 2, 8),
+    TileConfig(256, 256, 32, 4, 4),
     TileConfig(256, 128, 32, 4, 4),
 )
 

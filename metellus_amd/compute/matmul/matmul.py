@@ -1,4 +1,4 @@
-"""Matmul fragments for gfx950: fp32 MFMA mainloop with register epilogues.
+"""Matmul fragments for gfx950: MFMA mainloop with register epilogues.
 
 Same fragment roles as the reference (reference:
 src/compute/matmul/matmul.py:12-369) -- tile mapping, thread index, setup,
@@ -341,10 +341,15 @@ class MatmulSetupFragment:
 
 @dataclass(frozen=True)
 class MatmulComputeFragment:
-    """MFMAs over the LDS k-chunk in buffer ``stage`` (set by the mainloop)."""
+    """MFMAs over the LDS k-chunk in buffer ``stage`` (set by the mainloop).
+    ``split``: fp32 operands as three bf16 parts on the bf16 matrix cores
+    (``mt_mfma_tile``; a ``MatmulExactRetryFragment`` follows the mainloop);
+    without it, fp32 MFMAs (``mt_mfma_tile_f32``), which need nothing after
+    them -- the default for kernels composed by hand."""
 
     config: MatmulConfig
     accumulator_suffix: str = ""
+    split: bool = False
     name: str = "matmul_compute"
     kind: str = "compute"
 
@@ -352,10 +357,9 @@ class MatmulComputeFragment:
                      held: tuple[str, str] | None = None) -> str:
         """MFMAs over LDS buffer ``stage`` of double-buffered tiles, or over
         single-buffered tiles when ``stage`` is None; ``hook`` names a
-        callable run at each group of 4 k-steps (``mt_mfma_tile``).
-        ``held`` = (group variable, has-held expression): the chunk's last
-        group of 4 k-steps is carried to the next chunk
-        (``mt_mfma_tile_held``; no hook)."""
+        callable run before the reads of each group of 8 k's (``mt_mfma_tile``).
+        ``held`` = (group variable, has-held expression): a long mainloop's
+        chunk (``mt_mfma_tile_held``; no hook)."""
         t = self.config.tile
         at, bt = self.config.a_tile_name, self.config.b_tile_name
         a_ptr = f"&{at}[{stage}][wave_m0][0]" if stage is not None else f"&{at}[wave_m0][0]"
@@ -368,6 +372,13 @@ class MatmulComputeFragment:
             aswz = "true" if t.a_layout == "swz" else "false"
             bnm = "true" if t.b_layout == "nswz" else "false"
             flags = f", {aswz}, {bnm}"
+        if not self.split:
+            if held is not None or hook is not None:
+                raise ValueError("a load hook or a held group needs the split form")
+            return (
+                f"mt_mfma_tile_f32<{t.WM}, {t.WN}, {t.tile_K}, {t.lda}, {t.ldb}{flags}>"
+                f"({a_ptr}, {b_ptr}, acc{self.accumulator_suffix}, lane);"
+            )
         if hook is not None and not flags:
             flags = ", false, false"
         if held is not None:
@@ -384,13 +395,12 @@ class MatmulComputeFragment:
         )
 
     def render_held_decl(self, var: str) -> str:
-        """Zeroed: after a k loop that ran no chunk its flush adds 0 * 0 to
-        accumulators that still hold +0."""
+        """What one chunk leaves to the next (nothing, ``mt_mfma_group``)."""
         t = self.config.tile
         return f"mt_mfma_group<{t.WM}, {t.WN}> {var} = {{}};"
 
     def render_held_flush(self, var: str) -> str:
-        """The last chunk's held group, after the k loop."""
+        """Runs what the last chunk left, after the k loop."""
         t = self.config.tile
         return f"mt_mfma_group_run<{t.WM}, {t.WN}>({var}, acc{self.accumulator_suffix});"
 
@@ -406,6 +416,59 @@ class MatmulComputeFragment:
             TgmemAccess(self.config.a_tile_name, "read", _prod(a_shape), a_shape),
             TgmemAccess(self.config.b_tile_name, "read", _prod(b_shape), b_shape),
         )
+
+
+@dataclass(frozen=True)
+class MatmulExactRetryFragment:
+    """After a split mainloop: a wave whose accumulators hold a NaN or a
+    vanishingly small value (``mt_mfma_retry``) computes its blocks again with
+    fp32 MFMAs on operands read from global memory (``mt_mfma_exact``), over
+    the chunks this workgroup walked.  ``a`` / ``b`` are (parameter, row
+    stride, col stride, prologue lambda over (raw, row, col) or None)."""
+
+    config: MatmulConfig
+    a: tuple[str, int, int, str | None]
+    b: tuple[str, int, int, str | None]
+    accumulator_suffix: str = ""
+    persistent: bool = False
+    name: str = "matmul_exact_retry"
+    kind: str = "compute"
+
+    @staticmethod
+    def _operand(label: str, operand: tuple, rows: str, cols: str) -> list[str]:
+        src, rs, cs, transform = operand
+        at = f"{src}[(size_t)r * {rs}u + (size_t)c * {cs}u]"
+        lines = [f"const auto xf = {transform};"] if transform else []
+        value = f"xf({at}, r, c)" if transform else at
+        capture = "[=]" if transform else "[&]"
+        return [
+            f"const auto {label} = [&] {{",
+            *[f"    {x}" for x in lines],
+            f"    return {capture}(unsigned r, unsigned c) -> float "
+            f"{{ return r < {rows} && c < {cols} ? {value} : 0.0f; }};",
+            "}();",
+        ]
+
+    def render(self, ctx: CodegenContext) -> str:
+        c, t = self.config, self.config.tile
+        acc = f"acc{self.accumulator_suffix}"
+        k = c.K_dim_var
+        if self.persistent:
+            kb, ke = f"mt_kb * {t.tile_K}u", f"(mt_ke * {t.tile_K}u < {k} ? mt_ke * {t.tile_K}u : {k})"
+        else:
+            kb, ke = "0u", k
+        lines = [
+            f"if (mt_mfma_retry<{t.WM}, {t.WN}>({acc})) {{",
+            *["    " + x for x in self._operand("mt_fa", self.a, c.M_dim_var, k)],
+            *["    " + x for x in self._operand("mt_fb", self.b, k, c.N_dim_var)],
+            f"    mt_mfma_exact<{t.WM}, {t.WN}>(mt_fa, mt_fb, tile_m0 + wave_m0, tile_n0 + wave_n0, {kb}, {ke}, lane, {acc});",
+            "}",
+        ]
+        return "\n".join(lines)
+
+    @property
+    def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
+        return ()
 
 
 def _prod(shape) -> int:
@@ -442,14 +505,13 @@ class MatmulMainloopFragment:
     K_dim_var: str
     persistent: bool = False
     # > 0: the next chunk's register-path loads are issued in ``spread``
-    # parts at the first ``spread`` groups of 4 k-steps of the current
+    # parts at the first ``spread`` groups of 8 k's of the current
     # chunk's MFMAs (a hook of the first compute fragment) instead of all
     # before them; direct-to-LDS loads stay before the MFMAs unless
     # ``spread_dma``.
     spread: int = 0
     spread_dma: bool = False
-    # carry each chunk's last group of 4 k-steps over the barrier into the
-    # next chunk (``mt_mfma_tile_held``); not with spread loads
+    # a long mainloop's chunks (``mt_mfma_tile_held``); not with spread loads
     held: bool = False
     name: str = "matmul_mainloop"
     kind: str = "compute"
@@ -634,19 +696,18 @@ class MatmulMainloopFragment:
 @dataclass(frozen=True)
 class MatmulRowWavesFragment:
     """A whole matmul 128 columns wide on row-owning waves (``mt_rw_*``):
-    256 x 128 tiles on 1024 lanes, 16 waves of 16 rows x 128 columns of
-    16x16x4 MFMAs.  A wave reads its own A rows from global memory into
-    registers, a 64-wide k-chunk ahead, and applies the prologue there
-    (``prologue``: None; ``("transform", lambda)`` over (raw, row, col); or
-    ``("gather", gather, apply, plain_apply, plain_predicate)`` with operands
-    fixed per row, read once per lane); B goes straight into two LDS stages
-    (``B_tile[2][64][128]``) by direct-to-LDS loads.  With a plain form of
-    the prologue, every lane tests its row's divisors once
-    (``__syncthreads_and``) and the workgroup runs the k loop with the plain
-    form when all pass.  Needs M % 256 == 0, N == 128, K % 128 == 0 (the
-    loop takes two chunks a trip).  The epilogue stores 128 bits per row;
-    ``value_expr`` is a format string over ``{a0}`` with ``row`` and ``col``
-    in scope."""
+    256 x 128 tiles on 1024 lanes, 16 waves of 32 rows x 64 columns of split
+    MFMAs.  A wave reads its rows of A from global memory into registers, a
+    64-wide k-chunk ahead, and applies the prologue there (``prologue``: None;
+    ``("transform", lambda)`` over (raw, row, col); or ``("gather", gather,
+    apply, plain_apply, plain_predicate)`` with operands fixed per row, read
+    once per lane); B is split by the workgroup into two LDS stages
+    (``B_tile[2][64][128]``: parts 1 and 2, ``B_low[2][32][128]``: part 3).
+    With a plain form of the prologue, every lane tests its row's divisors
+    once (``__syncthreads_and``) and the workgroup runs the k loop with the
+    plain form when all pass.  Needs M % 256 == 0, N == 128, K % 128 == 0 (the
+    loop takes two chunks a trip).  ``value_expr`` is a format string over
+    ``{a0}`` with ``row`` and ``col`` in scope."""
 
     a_name: str
     b_name: str
@@ -664,21 +725,21 @@ class MatmulRowWavesFragment:
     THREADS = 1024
 
     def _loop(self, pa: str) -> list[str]:
-        a, b, brs = self.a_name, self.b_name, self.b_row_stride
+        b, brs = self.b_name, self.b_row_stride
+
+        def chunk(stage: int, ahead: int, more: str) -> list[str]:
+            return [
+                f"    if ({more}) ld_B.fetch({b}, {brs}u, (kt + {ahead}u) * 64u, threadIdx.x);",
+                f"    mt_rw_chunk(mt_a, mt_arow, (kt + {ahead}u) * 64u, {more}, &B_tile[{stage}][0][0], "
+                f"&B_low[{stage}][0][0], mt_n0, {pa}, lane, acc);",
+                f"    if ({more}) ld_B.commit(&B_tile[{stage ^ 1}][0][0], &B_low[{stage ^ 1}][0][0], threadIdx.x);",
+                "    __syncthreads();",
+            ]
+
         return [
             "for (unsigned kt = 0; kt < n_chunks; kt += 2u) {",
-            "    mt_rw_load(mt_a1, mt_arow, (kt + 1u) * 64u);",
-            f"    ld_B.fetch({b}, {brs}, (kt + 1u) * 64u, 0u, &B_tile[1][0][0]);",
-            f"    mt_rw_chunk(mt_a0, &B_tile[0][0][0], {pa}, lane, acc);",
-            "    __builtin_amdgcn_s_waitcnt(0);",
-            "    __syncthreads();",
-            "    if (kt + 2u < n_chunks) {",
-            "        mt_rw_load(mt_a0, mt_arow, (kt + 2u) * 64u);",
-            f"        ld_B.fetch({b}, {brs}, (kt + 2u) * 64u, 0u, &B_tile[0][0][0]);",
-            "    }",
-            f"    mt_rw_chunk(mt_a1, &B_tile[1][0][0], {pa}, lane, acc);",
-            "    __builtin_amdgcn_s_waitcnt(0);",
-            "    __syncthreads();",
+            *chunk(0, 1, "true"),
+            *chunk(1, 2, "kt + 2u < n_chunks"),
             "}",
         ]
 
@@ -688,34 +749,40 @@ class MatmulRowWavesFragment:
         lines = [
             "const unsigned lane = mt_lane();",
             "const unsigned wave = mt_wave();",
-            "const unsigned tile_m0 = blockIdx.y * 256u;",
-            "const unsigned mt_row = tile_m0 + wave * 16u + (lane & 15u);",
-            "mt_f32x4 acc[8];",
-            "#pragma unroll",
-            "for (int j = 0; j < 8; ++j) acc[j] = mt_f32x4{0.f, 0.f, 0.f, 0.f};",
-            f"const mt_tile_dma<64, 128, 1024, false> ld_B({self.b_row_stride}, threadIdx.x);",
-            f"const float* __restrict__ mt_arow = {a} + (size_t)mt_row * {self.a_row_stride}u + 16u * (lane >> 4);",
-            "mt_f32x4 mt_a0[4], mt_a1[4];",
+            "const unsigned mt_m0 = blockIdx.y * 256u + (wave >> 1) * 32u;",
+            "const unsigned mt_n0 = (wave & 1u) * 64u;",
+            "const unsigned mt_row = mt_m0 + (lane & 31u);",
+            "mt_f32x16 acc[1][2];",
+            "mt_zero(acc[0][0]);",
+            "mt_zero(acc[0][1]);",
+            "mt_rw_stage ld_B;",
+            f"const float* __restrict__ mt_arow = {a} + (size_t)mt_row * {self.a_row_stride}u + 8u * (lane >> 5);",
+            "mt_f32x4 mt_a[4][2];",
         ]
         plain = False
+        raw = f"{a}[(size_t)r * {self.a_row_stride}u + k]"
         if pro is None:
             lines.append("const auto mt_pa = [](float raw) -> float { return raw; };")
+            value_at = raw
         elif pro[0] == "transform":
             lines += [f"const auto xt = {pro[1]};",
                       "const auto mt_pa = [=](float raw) -> float { return xt(raw, mt_row, 0u); };"]
+            value_at = f"xt({raw}, r, 0u)"
         else:
             _, gather, apply, plain_apply, plain_pred = pro
             lines += [f"const auto xg = {gather};", f"const auto xa = {apply};",
                       "const auto mt_e = xg(mt_row, 0u);  // the row's operands",
                       "const auto mt_pa = [=](float raw) -> float { return xa(raw, mt_e); };"]
+            value_at = f"xa({raw}, xg(r, 0u))"
             if plain_apply is not None:
                 plain = True
                 lines += [f"const auto xq = {plain_apply};", f"const auto xp = {plain_pred};",
                           "const auto mt_pq = [=](float raw) -> float { return xq(raw, mt_e); };"]
         lines += [
-            "mt_rw_load(mt_a0, mt_arow, 0u);",
-            f"ld_B.fetch({b}, {self.b_row_stride}, 0u, 0u, &B_tile[0][0][0]);",
-            "__builtin_amdgcn_s_waitcnt(0);",
+            f"ld_B.fetch({b}, {self.b_row_stride}u, 0u, threadIdx.x);",
+            "#pragma unroll",
+            "for (int s = 0; s < 4; ++s) mt_rw_load(mt_a[s], mt_arow, 0u, s);",
+            "ld_B.commit(&B_tile[0][0][0], &B_low[0][0][0], threadIdx.x);",
             "__syncthreads();",
             "const unsigned n_chunks = K / 64u;",
         ]
@@ -725,22 +792,20 @@ class MatmulRowWavesFragment:
                       *[f"    {x}" for x in self._loop("mt_pa")], "}"]
         else:
             lines += self._loop("mt_pa")
-        value = self.value_expr.format(a0="acc[4 * h + j][i]") if self.value_expr else "acc[4 * h + j][i]"
+        value = self.value_expr.format(a0="acc[0][j][v]") if self.value_expr else "acc[0][j][v]"
         lines += [
+            "if (mt_mfma_retry<1, 2>(acc)) {",
+            f"    const auto mt_fa = [=](unsigned r, unsigned k) -> float {{ return {value_at}; }};",
+            f"    const auto mt_fb = [&](unsigned k, unsigned n) -> float {{ return {b}[(size_t)k * {self.b_row_stride}u + n]; }};",
+            "    mt_mfma_exact<1, 2>(mt_fa, mt_fb, mt_m0, mt_n0, 0u, K, lane, acc);",
+            "}",
             "#pragma unroll",
-            "for (int i = 0; i < 4; ++i) {",
-            "    const unsigned row = tile_m0 + wave * 16u + 4u * (lane >> 4) + (unsigned)i;",
+            "for (int v = 0; v < 16; ++v) {",
+            "    const unsigned row = mt_m0 + mt_acc_row(v, lane);",
             "#pragma unroll",
-            "    for (int h = 0; h < 2; ++h) {",
-            "        const unsigned col0 = 64u * (unsigned)h + 4u * (lane & 15u);",
-            "        mt_f32x4 mt_o;",
-            "#pragma unroll",
-            "        for (int j = 0; j < 4; ++j) {",
-            "            const unsigned col = col0 + (unsigned)j;",
-            "            (void)col;",
-            f"            mt_o[j] = {value};",
-            "        }",
-            f"        *reinterpret_cast<mt_f32x4*>(&{c}[(size_t)row * N + col0]) = mt_o;",
+            "    for (int j = 0; j < 2; ++j) {",
+            "        const unsigned col = mt_n0 + 32u * (unsigned)j + (lane & 31u);",
+            f"        {c}[(size_t)row * N + col] = {value};",
             "    }",
             "}",
         ]
@@ -748,7 +813,10 @@ class MatmulRowWavesFragment:
 
     @property
     def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
-        return (TgmemAccess("B_tile", "read", 2 * 64 * 128, (2, 64, 128)),)
+        return (
+            TgmemAccess("B_tile", "read", 2 * 64 * 128, (2, 64, 128)),
+            TgmemAccess("B_low", "read", 2 * 32 * 128, (2, 32, 128)),
+        )
 
 
 # K-resident row waves: the previous chunk's right half is stored one row

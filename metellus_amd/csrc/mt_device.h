@@ -26,12 +26,15 @@
 //   * mt_tile_dma / mt_swz    direct-to-LDS tile loads (global_load_lds_dwordx4,
 //                             no registers, no LDS stores) into dense tiles
 //                             whose 16-byte slots are XOR-swizzled per row
-//   * mt_mfma_tile            fp32 MFMA (v_mfma_f32_32x32x2f32) over one LDS
-//                             k-chunk for a wave's WM x WN grid of 32x32 blocks
-//   * mt_mfma_tile_held       the same with the chunk's last group of 4 k-steps
-//                             carried over the barrier (mt_mfma_group)
+//   * mt_mfma_tile            one LDS k-chunk for a wave's WM x WN grid of 32x32
+//                             blocks: fp32 operands split into three bf16 parts
+//                             in registers (mt_split), six bf16 MFMAs per step
+//   * mt_mfma_retry / mt_mfma_exact
+//                             the fp32 MFMAs a wave falls back to when the
+//                             split cannot represent its operands
+//   * mt_mfma_tile_f32        the same chunk on fp32 MFMAs (hand-composed kernels)
 //   * mt_rw_*                 row-owning waves for matmuls 128 columns wide
-//                             (16x16x4 MFMAs, A in registers, B in LDS)
+//                             (split MFMAs, A in registers, B's parts in LDS)
 //   * mt_acc_row              row of accumulator register v in a 32x32 block
 //   * mt_stream_k / mt_sk_*   stream-K schedule of a persistent matmul and the
 //                             workspace flags that hand split tiles' partial
@@ -45,6 +48,7 @@
 
 typedef float mt_f32x4 __attribute__((ext_vector_type(4)));
 typedef float mt_f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned mt_u32x4 __attribute__((ext_vector_type(4)));
 
 struct mt_dims {
     unsigned int v[16];
@@ -793,15 +797,9 @@ struct mt_tile_dma {
 // same order, so results are identical across layouts.
 // ---------------------------------------------------------------------------
 
-// hook(q) runs at the start of each group of 4 k-steps, q = 0 .. TK/8 - 1:
-// the mainloop issues its next chunk's loads there, spread over the MFMAs.
-struct mt_no_hook {
-    MT_INLINE void operator()(int) const {}
-};
-
-template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false, typename H = mt_no_hook>
-MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restrict__ Bs,
-                            mt_f32x16 (&acc)[WM][WN], unsigned lane, H hook = H{}) {
+template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false>
+MT_INLINE void mt_mfma_tile_f32(const float* __restrict__ As, const float* __restrict__ Bs,
+                                mt_f32x16 (&acc)[WM][WN], unsigned lane) {
     static_assert(TK % 8 == 0, "TK must be a multiple of 8");
     static_assert(LDA % 4 == 0, "LDA must keep 16-byte alignment");
     static_assert(!ASWZ || LDA == TK, "a swizzled A tile is dense");
@@ -822,7 +820,6 @@ MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restric
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int s0 = 0; s0 < HALF; s0 += 4) {
-        hook(s0 / 4);
         const unsigned slot = (lh * HALF + (unsigned)s0) / 4u;  // swizzled tiles: logical 16-byte slot
         mt_f32x4 a[WM];
 #pragma unroll
@@ -851,27 +848,126 @@ MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restric
 }
 
 // ---------------------------------------------------------------------------
-// The same MFMAs with the chunk's last group of 4 k-steps carried over the
-// barrier.  A group's operands (4 k-steps of WM A and WN B fragments) are
-// read from LDS into a mt_mfma_group first; mt_mfma_tile_held reads group
-// g + 1 while group g's MFMAs run, and leaves the last group's operands in
-// `held`: the next chunk (or mt_mfma_group_run after the k loop) runs them
-// first, after the barrier, so the matrix core has work while the waves
-// leave the barrier and read the next chunk.  Per accumulator the products
-// are added in the same k order as mt_mfma_tile, so the results are
-// identical.  The barrier's release fence waits for the LDS reads into
-// `held` (lgkmcnt(0)) before another wave may overwrite the buffer.
+// fp32 products on the bf16 matrix cores.  A float is the sum of three bf16
+// numbers: x1 = x rounded to bf16, x2 = x - x1 rounded to bf16, x3 = the rest.
+// 24 = 8 + 8 + 8 significant bits, so the sum is exact, and each remainder is
+// an exact fp32 subtraction.  Of the nine partial products of x y the six of
+// at least 2^-16 |x y| are accumulated, smallest first,
+//     x3 y1 + x2 y2 + x1 y3 + x2 y1 + x1 y2 + x1 y1,
+// by v_mfma_f32_32x32x16_bf16 into the fp32 accumulator; x2 y3, x3 y2 and
+// x3 y3 are below the last bit of the fp32 product.  Rounding x1 (instead of
+// cutting it off) gives x2 a sign of its own: the MFMA drops what lies far
+// below the accumulator's last bit, and with x2 y2 always of the product's
+// sign that added up (all-positive operands, K = 4096: 3.4e-6 instead of 5.9e-7).
+//
+// Why: the fp32 MFMA does 64 multiply-adds per cycle and SIMD, the bf16 one
+// 1024, so six of them have 2.7 times its rate.  Measured on MI355X, 4096^3:
+// 1018 us (135 TFLOP/s) with fp32 MFMAs, 741 us (185 TFLOP/s) this way; the
+// matrix cores are then busy 63 % of the cycles and the clock has fallen from
+// 2.05 to 1.68 GHz (a plain bf16 GEMM of 8192^3 reaches 1.22 PFLOP/s on the
+// same box, six times 203 TFLOP/s: power, not the split, is the next limit).
+// Error against 64 bits, relative 2-norm, fp32 MFMA -> split, N(0, 1) operands:
+// K = 64: 1.44e-7 -> 1.09e-7; 512: 4.1e-7 -> 3.4e-7; 1024: 5.8e-7 -> 4.9e-7;
+// 4096: 1.15e-6 -> 1.00e-6; 11008: 1.88e-6 -> 1.69e-6; all positive, 64:
+// 1.17e-7 -> 0.86e-7; 1024: 4.7e-7 -> 3.3e-7; 4096: 9.4e-7 -> 5.9e-7; 11008:
+// 1.52e-6 -> 0.96e-6 (fewer roundings of the accumulator: six per 16 k's, not
+// eight).
+//
+// The splits are made in registers from fp32 LDS tiles, so every loader and
+// prologue stays as it is.  A wave splits the WM + WN fragments it multiplies,
+// 5.5 VALU operations per element against 6 WM WN MFMAs of 32 cycles: square
+// wave tiles split the least per MFMA.  Each lane half supplies 8 consecutive
+// k's of an MFMA's 16 (the chunk's two halves, as in mt_mfma_tile_f32).
+//
+// What a split cannot do: an infinite x, or one that rounds to an infinite x1
+// (from 0x1.ffp+127), leaves a NaN or an infinity of the wrong sign as its
+// remainder, which makes every sum it enters a NaN; and below 2^-110 the lower
+// parts fall under bf16's smallest number.  mt_mfma_retry finds such tiles by
+// their results.
 // ---------------------------------------------------------------------------
 
-template <int WM, int WN>
-struct mt_mfma_group {
-    mt_f32x4 a[WM];
-    mt_f32x4 b[WN];
+typedef __bf16 mt_bf16x8 __attribute__((ext_vector_type(8)));
+
+// Eight floats as three vectors of eight bf16.
+struct mt_split8 {
+    mt_u32x4 p1, p2, p3;
 };
 
-template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ, bool BNM>
-MT_INLINE void mt_mfma_group_load(const float* __restrict__ As, const float* __restrict__ Bs, unsigned lane,
-                                  int s0, mt_mfma_group<WM, WN>& g) {
+MT_INLINE unsigned mt_cvt_pk_bf16(float lo, float hi) {  // round to nearest even
+    unsigned r;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
+    return r;
+}
+MT_INLINE unsigned mt_pack_hi16(float lo, float hi) {  // upper halves of two floats
+    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x07060302u);
+}
+MT_INLINE float mt_keep_hi16(unsigned x) { return __builtin_bit_cast(float, x & 0xffff0000u); }
+
+MT_INLINE mt_split8 mt_split(mt_f32x4 u, mt_f32x4 v) {
+    mt_split8 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float x0 = q < 2 ? u[2 * q] : v[2 * q - 4], x1 = q < 2 ? u[2 * q + 1] : v[2 * q - 3];
+        const unsigned h = mt_cvt_pk_bf16(x0, x1);
+        o.p1[q] = h;
+        const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - mt_keep_hi16(h);
+        const unsigned m = mt_cvt_pk_bf16(r0, r1);
+        o.p2[q] = m;
+        o.p3[q] = mt_pack_hi16(r0 - __builtin_bit_cast(float, m << 16), r1 - mt_keep_hi16(m));
+    }
+    return o;
+}
+
+MT_INLINE mt_f32x16 mt_mfma_bf16(mt_u32x4 a, mt_u32x4 b, mt_f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mt_bf16x8, a), __builtin_bit_cast(mt_bf16x8, b),
+                                                   c, 0, 0, 0);
+}
+
+// The six partial products of one 32x32 block and 16 k's, smallest first.
+MT_INLINE mt_f32x16 mt_mfma_parts(const mt_split8& a, const mt_split8& b, mt_f32x16 c) {
+    c = mt_mfma_bf16(a.p3, b.p1, c);
+    c = mt_mfma_bf16(a.p2, b.p2, c);
+    c = mt_mfma_bf16(a.p1, b.p3, c);
+    c = mt_mfma_bf16(a.p2, b.p1, c);
+    c = mt_mfma_bf16(a.p1, b.p2, c);
+    return mt_mfma_bf16(a.p1, b.p1, c);
+}
+
+// One row block of a step of 16 k's: a0, a1 the lane's 8 consecutive k's of A,
+// b[j] column block j's parts.  Product by product over the column blocks, so
+// an MFMA does not wait for the one before it (C4 X @ W1: 1840 us; block by
+// block 1924 us).
+template <int WN>
+MT_INLINE void mt_mfma_split(mt_f32x4 a0, mt_f32x4 a1, const mt_split8 (&b)[WN], mt_f32x16 (&acc)[WN]) {
+    const mt_split8 a = mt_split(a0, a1);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p3, b[j].p1, acc[j]);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p2, b[j].p2, acc[j]);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p1, b[j].p3, acc[j]);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p2, b[j].p1, acc[j]);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p1, b[j].p2, acc[j]);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p1, b[j].p1, acc[j]);
+}
+
+// hook(q) runs before the LDS reads of each group of 8 k's, q = 0 .. TK/8 - 1:
+// the mainloop issues its next chunk's loads there, spread over the MFMAs.
+struct mt_no_hook {
+    MT_INLINE void operator()(int) const {}
+};
+
+// The chunk in the layouts of mt_mfma_tile_f32.
+template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false, typename H = mt_no_hook>
+MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restrict__ Bs,
+                            mt_f32x16 (&acc)[WM][WN], unsigned lane, H hook = H{}) {
+    static_assert(TK % 16 == 0, "TK must be a multiple of 16");
+    static_assert(LDA % 4 == 0, "LDA must keep 16-byte alignment");
+    static_assert(!ASWZ || LDA == TK, "a swizzled A tile is dense");
+    static_assert(!BNM || LDB == TK, "an n-major B tile is dense");
     constexpr int HALF = TK / 2;
     const unsigned li = lane & 31u;
     const unsigned lh = lane >> 5;
@@ -879,127 +975,173 @@ MT_INLINE void mt_mfma_group_load(const float* __restrict__ As, const float* __r
     if constexpr (ASWZ || BNM) m = mt_swz<TK / 4>(li);
     const float* a_base = ASWZ ? As + li * TK : As + li * LDA + lh * HALF;
     const float* b_base = BNM ? Bs + li * TK : Bs + (lh * HALF) * LDB + li;
-    const unsigned slot = (lh * HALF + (unsigned)s0) / 4u;
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
-        g.a[i] = ASWZ ? mt_ld4(a_base + i * 32 * TK + 4u * (slot ^ m)) : mt_ld4(a_base + i * 32 * LDA + s0);
+    for (int s0 = 0; s0 < HALF; s0 += 8) {
+        // swizzled tiles: logical 16-byte slots of the lane's two quads
+        const unsigned slot0 = (lh * HALF + (unsigned)s0) / 4u, slot1 = slot0 + 1u;
+        mt_split8 b[WN];
+        hook(s0 / 4);
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-        if constexpr (BNM) {
-            g.b[j] = mt_ld4(b_base + j * 32 * TK + 4u * (slot ^ m));
-        } else {
+        for (int j = 0; j < WN; ++j) {
+            if constexpr (BNM) {
+                const float* row = b_base + j * 32 * TK;
+                b[j] = mt_split(mt_ld4(row + 4u * (slot0 ^ m)), mt_ld4(row + 4u * (slot1 ^ m)));
+            } else {
+                mt_f32x4 q[2];
 #pragma unroll
-            for (int ss = 0; ss < 4; ++ss) g.b[j][ss] = b_base[(s0 + ss) * LDB + j * 32];
+                for (int ss = 0; ss < 8; ++ss) q[ss / 4][ss % 4] = b_base[(s0 + ss) * LDB + j * 32];
+                b[j] = mt_split(q[0], q[1]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+            if (i == WM / 2) hook(s0 / 4 + 1);
+            const float* row = a_base + i * 32 * LDA;
+            const mt_f32x4 a0 = ASWZ ? mt_ld4(row + 4u * (slot0 ^ m)) : mt_ld4(row + s0);
+            const mt_f32x4 a1 = ASWZ ? mt_ld4(row + 4u * (slot1 ^ m)) : mt_ld4(row + s0 + 4);
+            mt_mfma_split<WN>(a0, a1, b, acc[i]);
         }
     }
+    __builtin_amdgcn_s_setprio(0);
 }
+
+// A long mainloop's chunk (MatmulMainloopFragment.held).  What one chunk leaves
+// to the next is empty: fp32 MFMAs gained 1 % from a group of operands carried
+// over the barrier, but the split's parts take the registers it was held in
+// (4096^3 with the group carried: 739 us on 8 waves and 1494 us, spilled, on 16;
+// without: 731 and 750 us).
+template <int WM, int WN>
+struct mt_mfma_group {};
 
 template <int WM, int WN>
-MT_INLINE void mt_mfma_group_run(const mt_mfma_group<WM, WN>& g, mt_f32x16 (&acc)[WM][WN]) {
-#pragma unroll
-    for (int ss = 0; ss < 4; ++ss)
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(g.a[i][ss], g.b[j][ss], acc[i][j], 0, 0, 0);
-}
+MT_INLINE void mt_mfma_group_run(const mt_mfma_group<WM, WN>&, mt_f32x16 (&)[WM][WN]) {}
 
-// Runs `held` (the previous chunk's last group) first when has_held, then
-// groups 0 .. G-2 of this chunk, and leaves group G-1's operands in `held`.
 template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false>
 MT_INLINE void mt_mfma_tile_held(const float* __restrict__ As, const float* __restrict__ Bs,
-                                 mt_f32x16 (&acc)[WM][WN], unsigned lane, mt_mfma_group<WM, WN>& held,
-                                 bool has_held) {
-    constexpr int G = TK / 8;
-    static_assert(TK % 8 == 0 && G >= 2, "a held group needs at least two groups of 4 k-steps per chunk");
-    static_assert(LDA % 4 == 0, "LDA must keep 16-byte alignment");
-    static_assert(!ASWZ || LDA == TK, "a swizzled A tile is dense");
-    static_assert(!BNM || LDB == TK, "an n-major B tile is dense");
-    __builtin_amdgcn_s_setprio(1);
-    mt_mfma_group<WM, WN> f[G - 1];
-    mt_mfma_group_load<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, lane, 0, f[0]);
-    if (has_held) mt_mfma_group_run<WM, WN>(held, acc);
+                                 mt_f32x16 (&acc)[WM][WN], unsigned lane, mt_mfma_group<WM, WN>&, bool) {
+    mt_mfma_tile<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, acc, lane);
+}
+
+// Whether the wave's accumulators may differ from the fp32 products' sums for
+// want of range: a NaN (every sum an infinite or NaN operand enters is one
+// here, where fp32 may give an infinity) or a nonzero result below 2^-96, which
+// takes operands small enough to have lost their lower parts.  Wave uniform.
+template <int WM, int WN>
+MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN]) {
+    bool odd = false;
 #pragma unroll
-    for (int g = 0; g < G - 1; ++g) {
-        if (g + 1 < G - 1)
-            mt_mfma_group_load<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, lane, 4 * (g + 1), f[g + 1]);
-        else
-            mt_mfma_group_load<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, lane, 4 * (g + 1), held);
-        mt_mfma_group_run<WM, WN>(f[g], acc);
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float x = acc[i][j][v];
+                odd |= !(__builtin_fabsf(x) >= 0x1.0p-96f) && x != 0.0f;
+            }
+    return __ballot(odd) != 0ull;
+}
+
+// The wave's blocks at (m0, n0) over k in [kb, ke) again, with fp32 MFMAs on
+// operands read from global memory: fa(row, k) and fb(k, col) give an operand
+// with its prologue applied, 0 outside the matrix.  Each wave decides and works
+// alone: no LDS, no barrier.  8 k's of loads are in flight at a time.
+template <int WM, int WN, typename FA, typename FB>
+MT_INLINE void mt_mfma_exact(FA fa, FB fb, unsigned m0, unsigned n0, unsigned kb, unsigned ke, unsigned lane,
+                             mt_f32x16 (&acc)[WM][WN]) {
+    const unsigned li = lane & 31u, lh = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) acc[i][j] = mt_f32x16{};
+    for (unsigned k = kb; k < ke; k += 8u) {
+        float a[4][WM], b[4][WN];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const unsigned kk = k + 2u * (unsigned)s + lh;
+#pragma unroll
+            for (int i = 0; i < WM; ++i) a[s][i] = kk < ke ? fa(m0 + 32u * (unsigned)i + li, kk) : 0.0f;
+#pragma unroll
+            for (int j = 0; j < WN; ++j) b[s][j] = kk < ke ? fb(kk, n0 + 32u * (unsigned)j + li) : 0.0f;
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s][i], b[s][j], acc[i][j], 0, 0, 0);
     }
-    __builtin_amdgcn_s_setprio(0);
 }
 
 // ---------------------------------------------------------------------------
-// Row-owning waves for matmuls 128 columns wide.  Each of a workgroup's 16
-// waves owns 16 rows x all 128 columns of a 256 x 128 tile, computed with
-// v_mfma_f32_16x16x4f32 (D[16x16] += A[16x4] * B[4x16]; lane l supplies
-// A[l%16][l/16] and B[l/16][l%16] and holds D[4 (l/16) + i][l%16], i < 4).
-// A wave's A rows are its own: they go from global memory straight into the
-// registers the MFMAs take (a prologue applied there), and only B is staged
-// in LDS, as 64-wide k-chunks in two stages (64 KiB).
-//   k: lane group g = l/16 takes a chunk's columns 16 g .. 16 g + 15, one per
-//      step, so its A values are 16 consecutive floats (four 128-bit loads);
-//   n: column block j < 4 puts lane column c = l%16 at output column 4 c + j,
-//      block j >= 4 at 64 + 4 c + (j - 4), so a step's 8 B values are two
-//      128-bit LDS reads (256 contiguous bytes per 16 lanes, no bank
-//      conflicts) and each output row is stored 128 bits at a time.
+// Row-owning waves for matmuls 128 columns wide, on the split products above.
+// A workgroup of 16 waves makes a 256 x 128 tile; waves 2w and 2w + 1 own rows
+// 32 w .. 32 w + 31, one column half each (two 32x32 blocks).  A goes from
+// global memory straight into the registers of the wave that splits it (a
+// prologue applied there).  B is split once per workgroup, not once per wave:
+// each lane loads 8 k's of one column, splits them and writes the three parts
+// to LDS as 16-byte units, which the MFMAs read as they are.
+//   k: step s of a 64-wide chunk takes k's 16 s .. 16 s + 15, lane half h the 8
+//      from 16 s + 8 h (k group 2 s + h);
+//   LDS stage: unit (group g, column n) of part 1 at 128 g + n of `hi`, part 2
+//      1024 units on, part 3 at 128 g + n of `lo`: lanes read and write
+//      consecutive units, so no bank conflicts.
+// Why: with 16 rows to a wave (fp32 MFMAs) every wave read all of B; LDS reads
+// were a quarter of the MFMA time and would be all of it at the split's rate.
+// Two waves sharing rows read half of B each and load A twice, the second time
+// from the caches.
 // ---------------------------------------------------------------------------
 
-struct mt_rw_group {
-    mt_f32x4 b[2][2];  // [step][column half]
+// This lane's share of a B chunk: column tid % 128, k group tid / 128.
+struct mt_rw_stage {
+    float v[8];
+
+    MT_INLINE void fetch(const float* __restrict__ src, unsigned ldb, unsigned k0, unsigned tid) {
+        const float* p = src + (size_t)(k0 + 8u * (tid >> 7)) * ldb + (tid & 127u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[(size_t)e * ldb];
+    }
+    MT_INLINE void commit(float* hi, float* lo, unsigned tid) const {
+        const mt_split8 x = mt_split(mt_f32x4{v[0], v[1], v[2], v[3]}, mt_f32x4{v[4], v[5], v[6], v[7]});
+        reinterpret_cast<mt_u32x4*>(hi)[tid] = x.p1;
+        reinterpret_cast<mt_u32x4*>(hi)[1024u + tid] = x.p2;
+        reinterpret_cast<mt_u32x4*>(lo)[tid] = x.p3;
+    }
 };
 
-MT_INLINE void mt_rw_group_load(mt_rw_group& g, const float* __restrict__ Bs, unsigned krow0, unsigned c) {
-#pragma unroll
-    for (int ss = 0; ss < 2; ++ss) {
-        g.b[ss][0] = mt_ld4(Bs + (krow0 + (unsigned)ss) * 128u + 4u * c);
-        g.b[ss][1] = mt_ld4(Bs + (krow0 + (unsigned)ss) * 128u + 64u + 4u * c);
-    }
+// This lane's A values of step s of the chunk at k0: arow points at its row's
+// column 8 (lane / 32).
+MT_INLINE void mt_rw_load(mt_f32x4 (&a)[2], const float* __restrict__ arow, unsigned k0, int s) {
+    a[0] = mt_ld4(arow + k0 + 16u * (unsigned)s);
+    a[1] = mt_ld4(arow + k0 + 16u * (unsigned)s + 4u);
 }
 
+// One 64-wide chunk: a holds its raw A values (pa applies the prologue) and,
+// step by step, receives those of the chunk at k_next (`more`): a step's loads
+// have the rest of this chunk and the steps before theirs in the next to land.
 template <typename P>
-MT_INLINE void mt_rw_group_run(const mt_rw_group& g, float a0, float a1, P pa, mt_f32x4 (&acc)[8]) {
-#pragma unroll
-    for (int ss = 0; ss < 2; ++ss) {
-        const float a = pa(ss == 0 ? a0 : a1);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, g.b[ss][0][j], acc[j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            acc[4 + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, g.b[ss][1][j], acc[4 + j], 0, 0, 0);
-    }
-}
-
-// One 64-wide chunk from the B stage at Bs (rows of 128 floats) and this
-// lane's 16 A values `a` (raw; pa applies the prologue): 8 groups of 2
-// steps, each group's B values read while the previous group's MFMAs run
-// (the order pinned with sched_barrier: left alone, the compiler reads each
-// value just before its MFMA and waits for it there).
-template <typename P>
-MT_INLINE void mt_rw_chunk(const mt_f32x4 (&a)[4], const float* __restrict__ Bs, P pa, unsigned lane,
-                           mt_f32x4 (&acc)[8]) {
-    const unsigned c = lane & 15u;
-    const unsigned k0 = 16u * (lane >> 4);
+MT_INLINE void mt_rw_chunk(mt_f32x4 (&a)[4][2], const float* __restrict__ arow, unsigned k_next, bool more,
+                           const float* __restrict__ hi, const float* __restrict__ lo, unsigned n0, P pa, unsigned lane,
+                           mt_f32x16 (&acc)[1][2]) {
+    const mt_u32x4* __restrict__ h4 = reinterpret_cast<const mt_u32x4*>(hi) + n0 + (lane & 31u);
+    const mt_u32x4* __restrict__ l4 = reinterpret_cast<const mt_u32x4*>(lo) + n0 + (lane & 31u);
     __builtin_amdgcn_s_setprio(1);
-    mt_rw_group f[8];
-    mt_rw_group_load(f[0], Bs, k0, c);
 #pragma unroll
-    for (int g = 0; g < 8; ++g) {
-        if (g + 1 < 8) mt_rw_group_load(f[g + 1], Bs, k0 + 2u * (unsigned)(g + 1), c);
-        __builtin_amdgcn_sched_barrier(0);
-        mt_rw_group_run(f[g], a[g / 2][2 * (g % 2)], a[g / 2][2 * (g % 2) + 1], pa, acc);
-        __builtin_amdgcn_sched_barrier(0);
+    for (int s = 0; s < 4; ++s) {
+        const unsigned g = 128u * (2u * (unsigned)s + (lane >> 5));
+        mt_f32x4 x[2];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e / 4][e % 4] = pa(a[s][e / 4][e % 4]);
+        if (more) mt_rw_load(a[s], arow, k_next, s);
+        const mt_split8 xa = mt_split(x[0], x[1]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const mt_split8 b = {h4[g + 32u * j], h4[1024u + g + 32u * j], l4[g + 32u * j]};
+            acc[0][j] = mt_mfma_parts(xa, b, acc[0][j]);
+        }
     }
     __builtin_amdgcn_s_setprio(0);
-}
-
-// This lane's A values of the chunk at k0: arow points at its row's column
-// 16 (lane / 16).
-MT_INLINE void mt_rw_load(mt_f32x4 (&a)[4], const float* __restrict__ arow, unsigned k0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = mt_ld4(arow + k0 + 4u * (unsigned)q);
 }
 
 // ---------------------------------------------------------------------------
@@ -1146,7 +1288,6 @@ MT_INLINE void mt_kr_chunk(const mt_f32x4 (&a)[K / 16], const float* __restrict_
 // workgroup (32-bit data, stride 0), so a store takes one per-lane byte
 // offset and one wave-uniform one instead of a 64-bit address per lane; the
 // hardware drops a store beyond the range instead of writing it.
-typedef unsigned mt_u32x4 __attribute__((ext_vector_type(4)));
 
 MT_INLINE mt_u32x4 mt_raw_buffer(const void* p, unsigned bytes) {
     const unsigned long long a = mt_uniform_addr(static_cast<const float*>(p));

@@ -7,7 +7,8 @@ first use), dims ``(M, K, N)``, grid ``(N tiles, M tiles, 1)``, operand
 strides read from the ``Tensor`` metadata (transposed views load
 transposed; K^T is read along K with 128-bit loads, no transpose kernel).
 
-gfx950 kernel: fp32 MFMA mainloop over double-buffered LDS, every epilogue
+gfx950 kernel: MFMA mainloop over double-buffered LDS (fp32 operands
+split into bf16 parts in registers, see ``mt_mfma_split``), every epilogue
 applied to the accumulator registers (both ``MATMUL_EPILOGUE_REGISTER`` and
 ``MATMUL_EPILOGUE_TG``; the label records the reference's decision), then a
 direct store.  LDS holds only the A and B chunks.  When the output tiles
@@ -39,6 +40,7 @@ from metellus_amd.compute.matmul.matmul import (
     MatmulComputeFragment,
     MatmulConfig,
     MatmulEpilogueStoreFragment,
+    MatmulExactRetryFragment,
     MatmulKResidentFragment,
     MatmulMainloopFragment,
     MatmulRowReduceFinishFragment,
@@ -239,13 +241,8 @@ LOAD_SPREAD = 4
 LOAD_SPREAD_DMA = False  # spread direct-to-LDS loads too (measurements only)
 
 
-# Each chunk's last group of 4 k-steps carried over the barrier into the next
-# chunk (MatmulMainloopFragment.held) for mainloops of at least HELD_MIN_CHUNKS
-# chunks whose loads are not spread.  Measured on MI355X as shader-clock
-# cycles summed over the XCDs (GRBM_GUI_ACTIVE), bit-identical outputs:
-# 4096^3 -1.0 %, C4 X @ W1 -0.6 %, C5 P @ V -0.5 to -0.8 %; C5 Q @ K^T
-# (4 chunks) +3.0 % and C4 (h1*s*h2) @ W3 (spread loads, 236 VGPRs)
-# +8.6 %, which keep the plain mainloop.
+# Mainloops of at least HELD_MIN_CHUNKS chunks whose loads are not spread take
+# ``mt_mfma_tile_held`` (MatmulMainloopFragment.held).
 HELD_GROUPS = True
 HELD_MIN_CHUNKS = 16
 
@@ -255,14 +252,9 @@ def held_groups(K: int, tile: TileConfig, spread: int) -> bool:
 
 
 # Matmuls 128 columns wide (C5 P @ V) on row-owning waves
-# (MatmulRowWavesFragment): every wave owns 16 rows x 128 columns, so its A
-# rows go from global memory straight into its registers and only B is
-# staged in LDS, which leaves room for 64-wide k-chunks -- half the barriers
-# of the LDS-tiled kernel, whose 256 x 128 tiles give each wave only 32
-# MFMAs per 32-wide chunk.  Measured on MI355X, C5 P @ V (32 heads batched),
-# same run: 249.8 -> 253.1 us against 257.6 -> 261.5 us for the LDS-tiled
-# kernel (0.863-0.874 of the fp32 MFMA peak against 0.835-0.848); outputs
-# agree to rounding (another MFMA shape: 16x16x4 instead of 32x32x2).
+# (MatmulRowWavesFragment): a wave's A rows go from global memory straight
+# into its registers and only B is staged in LDS, split there once for all
+# waves, in 64-wide k-chunks.
 ROW_WAVES = True
 ROW_WAVES_MIN_K = 1024
 
@@ -378,6 +370,18 @@ def b_tile_for(tile: TileConfig, src_b: Tensor, K: int, N: int) -> TileConfig:
     return dataclasses.replace(tile, b_pad=3)
 
 
+def exact_retry(config: MatmulConfig, src_a: Tensor, src_b: Tensor, pro_a: ChainCode | None,
+                pro_b: ChainCode | None, suffix: str = "", persistent: bool = False) -> MatmulExactRetryFragment:
+    """The fp32 fallback of a split mainloop over these operands."""
+
+    def operand(src: Tensor, pro: ChainCode | None):
+        return (param_name(src.buffer_key), src.row_stride, src.col_stride,
+                pro.lambda_transform() if pro is not None else None)
+
+    return MatmulExactRetryFragment(config, a=operand(src_a, pro_a), b=operand(src_b, pro_b),
+                                    accumulator_suffix=suffix, persistent=persistent)
+
+
 def rr_local(M: int, N: int, tile: TileConfig, batch: int = 1) -> bool:
     """The row-reduction epilogue completes rows inside one workgroup (row
     blocks walked whole, ``PersistentTiles.row_blocks``) when a tile spans
@@ -448,6 +452,10 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         # 16-wave tiles only without bounds checks (their masks cost registers)
         tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b, K, N)
         aligned = is_aligned_shape(M, K, N, tile)
+    if decision.reduction is not None and (tile.tile_N, tile.sg_M, tile.sg_N) == (256, 4, 4):
+        # each wave reduces its rows over its own columns: 2x8 waves leave
+        # half as many rows to every wave's lane exchanges
+        tile = dataclasses.replace(tile, sg_M=2, sg_N=8)
 
     tile = dma_layouts(tile, (src_a,), (src_b,), (pro_a,), (pro_b,), aligned)
     if full_gather and tile.b_layout == "pad":
@@ -487,7 +495,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
     spread = load_spread(pro_a, pro_b)
     mainloop = MatmulMainloopFragment(
         tile_K=tile.tile_K,
-        fragments=(a_load, b_load, BarrierFragment("inputs_ready"), MatmulComputeFragment(config),
+        fragments=(a_load, b_load, BarrierFragment("inputs_ready"), MatmulComputeFragment(config, split=True),
                    BarrierFragment("compute_done")),
         K_dim_var="K",
         persistent=persistent is not None,
@@ -511,6 +519,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         ThreadIndexFragment(tile),
         MatmulSetupFragment(config),
         mainloop,
+        exact_retry(config, src_a, src_b, pro_a, pro_b, persistent=persistent is not None),
         *((StreamKFixupFragment(config),) if stream_k else ()),
         store,
         *((PersistentLoopEndFragment(),) if persistent else ()),
@@ -574,7 +583,10 @@ def _assemble_row_waves(decision: DecisionView, function_name: str | None, src_a
         dims=("M", "K", "N"),
         tg_x=MatmulRowWavesFragment.THREADS,
         tg_y=1,
-        threadgroup_decls=(lds_decl("B_tile", (2, MatmulRowWavesFragment.TILE_K, MatmulRowWavesFragment.TILE_N)),),
+        threadgroup_decls=(
+            lds_decl("B_tile", (2, MatmulRowWavesFragment.TILE_K, MatmulRowWavesFragment.TILE_N)),
+            lds_decl("B_low", (2, MatmulRowWavesFragment.TILE_K // 2, MatmulRowWavesFragment.TILE_N)),
+        ),
         helpers=tuple(helpers),
     )
     return KernelGroup(

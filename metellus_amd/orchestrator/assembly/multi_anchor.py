@@ -43,7 +43,7 @@ from metellus_amd.orchestrator.assembly.decision import DecisionView
 from metellus_amd.orchestrator.assembly.expressions import ChainCode
 from metellus_amd.orchestrator.assembly.extras import Extras, input_param, output_param, param_name
 from metellus_amd.orchestrator.assembly import matmul as _mm
-from metellus_amd.orchestrator.assembly.matmul import b_tile_for, dma_layouts, operand_load
+from metellus_amd.orchestrator.assembly.matmul import b_tile_for, dma_layouts, exact_retry, operand_load
 from metellus_amd.orchestrator.ir import Tensor
 from metellus_amd.orchestrator.kernel_group import KernelGroup
 from metellus_amd.runtime.program import Kernel
@@ -139,8 +139,8 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
                     b_load(0),
                     b_load(1),
                     BarrierFragment("inputs_ready"),
-                    MatmulComputeFragment(configs[0], accumulator_suffix=suffixes[0]),
-                    MatmulComputeFragment(configs[1], accumulator_suffix=suffixes[1]),
+                    MatmulComputeFragment(configs[0], accumulator_suffix=suffixes[0], split=True),
+                    MatmulComputeFragment(configs[1], accumulator_suffix=suffixes[1], split=True),
                     BarrierFragment("compute_done"),
                 ),
                 K_dim_var="K",
@@ -161,7 +161,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
                         a_load,
                         b_load(i),
                         BarrierFragment(f"inputs{i}_ready"),
-                        MatmulComputeFragment(configs[i], accumulator_suffix=suffixes[i]),
+                        MatmulComputeFragment(configs[i], accumulator_suffix=suffixes[i], split=True),
                         BarrierFragment(f"compute{i}_done"),
                     ),
                     K_dim_var=kvars[i],
@@ -177,6 +177,11 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
         MatmulSetupFragment(configs[0], accumulator_suffix=suffixes[0]),
         MatmulSetupFragment(configs[1], accumulator_suffix=suffixes[1], emit_thread_coords=False),
         *mainloops,
+        *(
+            exact_retry(configs[i], src_a[0 if shared else i], src_b[i], tf_a[0 if shared else i], tf_b[i],
+                        suffix=suffixes[i], persistent=persistent is not None)
+            for i in range(2)
+        ),
         *((StreamKFixupFragment(configs[0], suffixes=suffixes),) if stream_k else ()),
         store,
         *((PersistentLoopEndFragment(),) if persistent else ()),
