@@ -252,6 +252,30 @@ class ChainCode:
         """Call with every external fetched by a scalar load at (row, col)."""
         return self.call(seed_values, [e.scalar_fetch(row, col) for e in self.externals])
 
+    def quad_lambda(self, raw: str, row: str = "r", col: str = "k") -> str | None:
+        """``[=](unsigned row, unsigned col) -> mt_f32x4``: the chain over the
+        four elements from (row, col) on, ``raw`` their 128-bit load; an
+        operand that varies along the columns is one such load too (any
+        element address), so None unless those have a unit column stride."""
+        loads, values = [], []
+        for k, e in enumerate(self.externals):
+            t = e.tensor
+            if e.broadcast in (BroadcastSpec.SCALAR, BroadcastSpec.COL):
+                loads.append(f"const float e{k} = {e.scalar_fetch(row, col)};")
+                values.append([f"e{k}"] * 4)
+                continue
+            if (t.col_stride if len(t.shape) == 2 else t.row_stride) != 1 or (
+                len(t.shape) == 1 and e.broadcast is BroadcastSpec.NONE
+            ):
+                return None
+            loads.append(f"const mt_f32x4 e{k} = mt_ld4u({param_name(t.buffer_key)} + {e.offset(row, col)});")
+            values.append([f"e{k}[{i}]" for i in range(4)])
+        out = ", ".join(self.call([f"x[{i}]"], [v[i] for v in values]) for i in range(4))
+        return (
+            f"[=](unsigned {row}, unsigned {col}) -> mt_f32x4 "
+            f"{{ const mt_f32x4 x = {raw}; {' '.join(loads)} return mt_f32x4{{{out}}}; }}"
+        )
+
     def gather_lambda(self, row: str = "global_row", col: str = "global_col") -> str:
         """``[=](unsigned row, unsigned col) -> mt_vals<E>``: this element's
         external operands, loaded with the tile (gather / apply loaders)."""

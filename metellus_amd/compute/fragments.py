@@ -71,6 +71,13 @@ class CodegenContext:
     # The kernel indexes its workspace by blockIdx.z, so its batched variant
     # shares one workspace (workspace_bytes covers the batch it was built for).
     workspace_batched: bool = False
+    # The kernel's fragments can do without the workspace (ctx.workspace_bytes
+    # 0): its batched variant does.
+    workspace_optional: bool = False
+    # A workgroup may wait for another one's partial sums (stream-K) and reports
+    # a wait that gave up in the workspace's error word; other users of the
+    # workspace never wait.
+    workspace_waits: bool = False
 
     @property
     def num_threads(self) -> int:

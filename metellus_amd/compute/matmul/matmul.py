@@ -819,6 +819,135 @@ class MatmulRowWavesFragment:
         )
 
 
+@dataclass(frozen=True)
+class MatmulSkinnyFragment:
+    """A whole matmul on ``mt_sn_*``: workgroups of ``waves`` waves make tiles
+    of ``16 * row_blocks`` x 64, their waves splitting the k's in groups of 16;
+    ``splits`` workgroups share a tile (grid x = column tiles x splits, y = row
+    tiles) and add their sums through the workspace, in split order, in the one
+    that arrives last.  ``b``: (parameter, row stride, col stride);
+    ``a_element``: an A element with its prologue, as an expression over (r, k);
+    ``a_quad``: a lambda of (r, k) giving the four from k on, where they can be
+    loaded 128 bits at a time.  ``nt``: B is read once and larger than what the
+    caches keep, so it streams past them.  ``value_expr`` is a format string over
+    ``{a0}`` with ``row`` and ``col`` in scope.
+
+    A batched variant of a kernel built for one program has no workspace of
+    its size: it walks the whole K in the first of a tile's workgroups."""
+
+    b: tuple[str, int, int]
+    c_name: str
+    row_blocks: int
+    waves: int
+    splits: int
+    a_element: str
+    a_quad: str | None = None
+    a_setup: tuple[str, ...] = ()
+    value_expr: str | None = None
+    nt: bool = False
+    name: str = "matmul_skinny"
+    kind: str = "compute"
+
+    TILE_N = 64
+
+    @property
+    def tile_M(self) -> int:
+        return 16 * self.row_blocks
+
+    def render(self, ctx: CodegenContext) -> str:
+        b, brs, bcs = self.b
+        along_k = "true" if brs == 1 and bcs != 1 else "false"
+        quads = "true" if self.a_quad is not None else "false"
+        mb, w, s = self.row_blocks, self.waves, self.splits
+        nt = "true" if self.nt else "false"
+        floats = 1024 * mb
+        lanes = 64 * w
+        whole = s > 1 and not ctx.workspace_bytes
+        value = self.value_expr.format(a0="mt_v") if self.value_expr else "mt_v"
+        lines = [
+            "const unsigned lane = mt_lane();",
+            "const unsigned wave = mt_wave();",
+            f"const unsigned mt_split_i = blockIdx.x % {s}u;",
+            f"const unsigned mt_n0 = (blockIdx.x / {s}u) * 64u;",
+            f"const unsigned mt_m0 = blockIdx.y * {16 * mb}u;",
+            *(["if (mt_split_i != 0u) return;"] if whole else []),
+            *self.a_setup,
+            f"const auto mt_fa = [=](unsigned r, unsigned k) -> float {{ return {self.a_element}; }};",
+            f"const auto mt_fv = {self.a_quad or '[](unsigned, unsigned) -> mt_f32x4 { return mt_f32x4{}; }'};",
+            f"mt_f32x4 acc[{mb}][4];",
+            "#pragma unroll",
+            f"for (int m = 0; m < {mb}; ++m)",
+            "#pragma unroll",
+            "    for (int j = 0; j < 4; ++j) acc[m][j] = mt_f32x4{0.f, 0.f, 0.f, 0.f};",
+            "const unsigned mt_groups = (K + 15u) / 16u;",
+            "const unsigned mt_unit = wave;" if whole or s == 1 else f"const unsigned mt_unit = mt_split_i * {w}u + wave;",
+            f"const unsigned mt_units = {w if whole else w * s}u;",
+            f"mt_sn_mainloop<{mb}, {quads}, {along_k}, {nt}>(mt_fv, mt_fa, {b}, "
+            f"{bcs if along_k == 'true' else brs}u, "
+            "(unsigned)((unsigned long long)mt_groups * mt_unit / mt_units), "
+            "(unsigned)((unsigned long long)mt_groups * (mt_unit + 1u) / mt_units), K, mt_m0, M, mt_n0, N, lane, acc);",
+            "#pragma unroll",
+            f"for (int m = 0; m < {mb}; ++m)",
+            "#pragma unroll",
+            "    for (int j = 0; j < 4; ++j)",
+            "#pragma unroll",
+            "        for (int i = 0; i < 4; ++i) sn_sum[wave][64u * (16u * m + 4u * j + i) + lane] = acc[m][j][i];",
+            "__syncthreads();",
+            f"float mt_sum[{floats // lanes}];",
+            "#pragma unroll",
+            f"for (int q = 0; q < {floats // lanes}; ++q) {{",
+            f"    const unsigned at = mt_sn_slot<{along_k}>((unsigned)q * {lanes}u + threadIdx.x);",
+            "    float t = sn_sum[0][at];",
+            "#pragma unroll",
+            f"    for (int v = 1; v < {w}; ++v) t += sn_sum[v][at];",
+            "    mt_sum[q] = t;",
+            "}",
+        ]
+        if s > 1 and not whole:
+            lines += [
+                f"const unsigned mt_tile = blockIdx.y * (gridDim.x / {s}u) + blockIdx.x / {s}u;",
+                f"float* mt_part = mt_ws + MT_WS_HEAD + (size_t)mt_tile * {s * floats}u;",
+                "#pragma unroll",
+                f"for (int q = 0; q < {floats // lanes}; ++q)",
+                f"    mt_sn_put(mt_part + mt_split_i * {floats}u + (unsigned)q * {lanes}u + threadIdx.x, mt_sum[q]);",
+                "if (!mt_sn_arrive(reinterpret_cast<unsigned*>(mt_ws) + mt_tile, "
+                f"{s}u, reinterpret_cast<unsigned*>(&sn_sum[0][0]))) return;",
+                "#pragma unroll",
+                f"for (int q = 0; q < {floats // lanes}; ++q) {{",
+                f"    const float* p = mt_part + (unsigned)q * {lanes}u + threadIdx.x;",
+                "    float t = mt_sn_get(p);",
+                "#pragma unroll",
+                f"    for (int v = 1; v < {s}; ++v) t += mt_sn_get(p + v * {floats}u);",
+                "    mt_sum[q] = t;",
+                "}",
+            ]
+        lines += [
+            "#pragma unroll",
+            f"for (int q = 0; q < {floats // lanes}; ++q) {{",
+            f"    const unsigned e = (unsigned)q * {lanes}u + threadIdx.x;",
+            "    const unsigned row = mt_m0 + (e >> 6), col = mt_n0 + (e & 63u);",
+            "    if (row < M && col < N) {",
+            "        const float mt_v = mt_sum[q];",
+            f"        {self.c_name}[(size_t)row * N + col] = {value};",
+            "    }",
+            "}",
+        ]
+        return "{\n" + textwrap.indent("\n".join(lines), "    ") + "\n}"
+
+    @property
+    def lds_shape(self) -> tuple[int, int]:
+        return (self.waves, 1024 * self.row_blocks)
+
+    @property
+    def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
+        return (TgmemAccess("sn_sum", "readwrite", _prod(self.lds_shape), self.lds_shape),)
+
+
+def skinny_workspace_bytes(tiles: int, row_blocks: int, splits: int) -> int:
+    """Counters, then every split's sums of every tile."""
+    return 4 * (STREAM_K_HEAD_WORDS + tiles * splits * 1024 * row_blocks) if splits > 1 else 0
+
+
 # K-resident row waves: the previous chunk's right half is stored one row
 # after every KR_STORE_STRIDE-th MFMA group of this chunk's left half (1:
 # after each of the first four groups); this chunk's left half one row after

@@ -35,6 +35,9 @@
 //   * mt_mfma_tile_f32        the same chunk on fp32 MFMAs (hand-composed kernels)
 //   * mt_rw_*                 row-owning waves for matmuls 128 columns wide
 //                             (split MFMAs, A in registers, B's parts in LDS)
+//   * mt_sn_*                 skinny matmuls (few rows): operands straight from
+//                             global memory into fp32 MFMAs, k split over waves
+//                             and workgroups
 //   * mt_acc_row              row of accumulator register v in a 32x32 block
 //   * mt_stream_k / mt_sk_*   stream-K schedule of a persistent matmul and the
 //                             workspace flags that hand split tiles' partial
@@ -65,6 +68,13 @@ struct mt_dims {
 #endif
 
 MT_INLINE mt_f32x4 mt_ld4(const float* p) { return *reinterpret_cast<const mt_f32x4*>(p); }
+// 128-bit load from any element address: the hardware asks for 4-byte
+// alignment only (every extra cache line touched costs a cycle or so).
+typedef float mt_f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+MT_INLINE mt_f32x4 mt_ld4u(const float* p) { return *reinterpret_cast<const mt_f32x4u*>(p); }
+MT_INLINE mt_f32x4 mt_ld4u_nt(const float* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const mt_f32x4u*>(p));
+}
 MT_INLINE void mt_st4(float* p, mt_f32x4 v) { *reinterpret_cast<mt_f32x4*>(p) = v; }
 // Streaming variants: nontemporal hint (data used once; do not keep in cache).
 MT_INLINE mt_f32x4 mt_ld4_nt(const float* p) {
@@ -1142,6 +1152,144 @@ MT_INLINE void mt_rw_chunk(mt_f32x4 (&a)[4][2], const float* __restrict__ arow, 
         }
     }
     __builtin_amdgcn_s_setprio(0);
+}
+
+// ---------------------------------------------------------------------------
+// Skinny matmuls: few output tiles, so what counts is how fast B streams in
+// (decoding: a few rows against whole weights) or how short the chain of
+// dependent loads is (small matrices).  A workgroup makes a 16 MB x 64 tile;
+// its waves split the tile's k's, and workgroups may split them further.  Both
+// operands go from global memory straight into the registers of
+// v_mfma_f32_16x16x4f32 (D[16x16] += A[16x4] * B[4x16]; lane l supplies
+// A[l%16][l/16], B[l/16][l%16] and holds D[4 (l/16) + i][l%16]): nothing is
+// shared between waves, so there is no LDS stage and no barrier in the k loop,
+// and each wave keeps its own loads in flight.
+//   k: a group of 16 k's is 4 steps; lane quarter g = l/16 takes k's
+//      4 g .. 4 g + 3 of it, one per step, so an A row is one 128-bit load;
+//   n: B read along n (row-major): the load of step s holds row k + 4 g + s,
+//      columns 4 c .. 4 c + 3, c = l%16 -- column block j is columns 4 c + j,
+//      and 16 lanes read 256 contiguous bytes; B read along k (a transposed
+//      view): load j holds column 16 j + c, the quarter's 4 k's.
+// The waves' sums meet in LDS and are added in wave order; workgroups that
+// split a tile add theirs through the workspace in split order (the last to
+// arrive does, mt_sn_arrive), so results do not depend on timing.
+// ---------------------------------------------------------------------------
+
+// One group's B values at k (k < ke; rows from ke on are 0): b[s][j] (along n)
+// or b[j][s] (along k) for step s, column block j.
+template <bool ALONG_K, bool NT>
+MT_INLINE void mt_sn_load_b(mt_f32x4 (&b)[4], const float* __restrict__ src, unsigned pitch, unsigned k, unsigned ke,
+                            unsigned n0, unsigned N, unsigned lane) {
+    const unsigned c = lane & 15u, kg = k + 4u * (lane >> 4);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        const unsigned major = ALONG_K ? n0 + 16u * (unsigned)x + c : kg + (unsigned)x;
+        const unsigned minor = ALONG_K ? kg : n0 + 4u * c;
+        const unsigned major_end = ALONG_K ? N : ke, minor_end = ALONG_K ? ke : N;
+        mt_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (major < major_end) {
+            const float* p = src + (size_t)major * pitch + minor;
+            if (minor + 4u <= minor_end) {
+                v = NT ? mt_ld4u_nt(p) : mt_ld4u(p);
+            } else {
+                if (minor < minor_end) v.x = p[0];
+                if (minor + 1u < minor_end) v.y = p[1];
+                if (minor + 2u < minor_end) v.z = p[2];
+            }
+        }
+        b[x] = v;
+    }
+}
+
+// One group's A values: row block m, this lane's 4 k's, its prologue applied:
+// fv(row, k) gives four k's at once (QUADS), fa(row, k) one.
+template <int MB, bool QUADS, typename FV, typename FA>
+MT_INLINE void mt_sn_load_a(mt_f32x4 (&a)[MB], FV fv, FA fa, unsigned k, unsigned ke, unsigned m0, unsigned M,
+                            unsigned lane) {
+    const unsigned kg = k + 4u * (lane >> 4);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        const unsigned row = m0 + 16u * (unsigned)m + (lane & 15u);
+        mt_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (row < M) {
+            if (QUADS && kg + 4u <= ke) {
+                v = fv(row, kg);
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if (kg + (unsigned)s < ke) v[s] = fa(row, kg + (unsigned)s);
+            }
+        }
+        a[m] = v;
+    }
+}
+
+// The wave's groups [g0, g1) of 16 k's each (K in all), UNROLL of them loaded
+// before any is multiplied.  Two keep the registers low enough for the other
+// waves to hide the loads (8 rows, 4096 x 11008: 39.8 us with 2, 42.7 with 4,
+// 47.8 with 8).
+template <int MB, bool QUADS_A, bool B_ALONG_K, bool NT_B, typename FV, typename FA>
+MT_INLINE void mt_sn_mainloop(FV fv, FA fa, const float* __restrict__ B, unsigned ldb, unsigned g0, unsigned g1,
+                              unsigned K, unsigned m0, unsigned M, unsigned n0, unsigned N, unsigned lane,
+                              mt_f32x4 (&acc)[MB][4]) {
+    constexpr int UNROLL = 2;
+    for (unsigned g = g0; g < g1; g += UNROLL) {
+        mt_f32x4 a[UNROLL][MB], b[UNROLL][4];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            if (g + (unsigned)u >= g1) {  // wave uniform
+#pragma unroll
+                for (int m = 0; m < MB; ++m) a[u][m] = mt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int x = 0; x < 4; ++x) b[u][x] = mt_f32x4{0.f, 0.f, 0.f, 0.f};
+                continue;
+            }
+            mt_sn_load_b<B_ALONG_K, NT_B>(b[u], B, ldb, 16u * (g + (unsigned)u), K, n0, N, lane);
+            mt_sn_load_a<MB, QUADS_A>(a[u], fv, fa, 16u * (g + (unsigned)u), K, m0, M, lane);
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][m][s], B_ALONG_K ? b[u][j][s] : b[u][s][j],
+                                                                        acc[m][j], 0, 0, 0);
+    }
+}
+
+// Partial sums handed between workgroups of one launch: device-scope stores
+// and loads (through the XCD's L2, which is not coherent with the others')
+// instead of the fences of mt_rr_publish -- an agent-scope release writes back
+// the whole L2 and an acquire invalidates it, per workgroup.
+MT_INLINE void mt_sn_put(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+MT_INLINE float mt_sn_get(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Count this workgroup in, its mt_sn_put stores complete; true in the last of
+// `parts` workgroups, which resets the counter for the next launch.
+MT_INLINE bool mt_sn_arrive(unsigned* counter, unsigned parts, unsigned* flag_lds) {
+    __builtin_amdgcn_s_waitcnt(0);  // every lane's stores have reached memory
+    __syncthreads();
+    if (threadIdx.x == 0u) {
+        const unsigned old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = old + 1u == parts;
+        if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *flag_lds = last ? 1u : 0u;
+    }
+    __syncthreads();
+    return *flag_lds != 0u;
+}
+
+// Element e = 64 row + col of a wave's tile in its LDS slab: register
+// (m, j, i) of lane l at 64 (16 m + 4 j + i) + l.
+template <bool B_ALONG_K>
+MT_INLINE unsigned mt_sn_slot(unsigned e) {
+    const unsigned row = e >> 6, col = e & 63u;
+    const unsigned j = B_ALONG_K ? col >> 4 : col & 3u, c = B_ALONG_K ? col & 15u : col >> 2;
+    return 64u * (16u * (row >> 4) + 4u * j + (row & 3u)) + 16u * ((row >> 2) & 3u) + c;
 }
 
 // ---------------------------------------------------------------------------

@@ -48,6 +48,7 @@ from metellus_amd.compute.matmul.matmul import (
     MatmulRowReduceStoreFragment,
     MatmulRowWavesFragment,
     MatmulSetupFragment,
+    MatmulSkinnyFragment,
     MatmulTileMappingFragment,
     PersistentLoopEndFragment,
     PersistentTiles,
@@ -56,6 +57,7 @@ from metellus_amd.compute.matmul.matmul import (
     rr_lds_shape,
     rr_row_blocks,
     rr_workspace_bytes,
+    skinny_workspace_bytes,
     stream_k_workspace_bytes,
 )
 from metellus_amd.memory.memory import TgLoadFragment, dma_offsets_fit
@@ -330,6 +332,48 @@ def k_resident_chunks(M: int, N: int, batch: int = 1) -> int:
     return total // groups
 
 
+# Skinny matmuls (MatmulSkinnyFragment): up to SKINNY_MAX_M rows.  Measured on
+# MI355X against the LDS-tiled kernel, whose one or two waves per compute unit
+# leave the memory idle: 8 x 4096 @ 4096 x 11008 127 -> 40 us (4.5 TB/s), 8 x
+# 11008 @ 11008 x 4096 with a two-operand prologue 763 -> 52 us, 32 rows 89 ->
+# 60 us, 64 x 4096 @ 4096 x 4096 91 -> 34 us, 13 x 1000 @ 1000 x 3001 46 -> 10 us.
+SKINNY = True
+SKINNY_MAX_M = 64
+SKINNY_MIN_B = 8192  # elements of B: up to here the call is a tile or two, all launch
+SKINNY_MAX_SPLITS = 16
+# B of more bytes than this is not kept by the 256 MiB Infinity Cache from one
+# pass to the next, so it is loaded past the caches (180 MB: 42.3 -> 39.8 us; a
+# 67 MB one, which stays, 33.9 -> 36.5 us).  Reads along k use half of a cache
+# line at a time and keep the caches (16.7 against 22.2 us).
+SKINNY_STREAM_BYTES = 1 << 27
+
+
+def skinny(M: int, K: int, N: int, src_b: Tensor, pro_b: ChainCode | None, reduction) -> bool:
+    """Whether a matmul takes the skinny kernel: few rows, a B read along one
+    of its axes with no prologue, no reduction epilogue."""
+    if not SKINNY or reduction is not None or pro_b is not None:
+        return False
+    if src_b.col_stride != 1 and src_b.row_stride != 1:
+        return False
+    return M <= SKINNY_MAX_M and K * N > SKINNY_MIN_B
+
+
+def skinny_shape(M: int, K: int, N: int, batch: int = 1) -> tuple[int, int, int]:
+    """(row blocks, waves, splits) of the skinny kernel.  Splits: the time goes
+    with how many workgroups a compute unit gets in turn, each a split's share
+    of the k's; a split more costs about a hundredth of an unsplit tile (its sums
+    through memory), and a wave keeps at least one group of 16 k's.  Batched
+    programs have their tiles, and no workspace each: no splits."""
+    row_blocks = 1 if M <= 16 else 2 if M <= 32 else 4
+    waves = 4 if row_blocks == 4 else 8  # 64 KiB of sums in LDS at most
+    tiles = ceil_div(M, 16 * row_blocks) * ceil_div(N, MatmulSkinnyFragment.TILE_N)
+    most = min(SKINNY_MAX_SPLITS, K // (16 * waves))
+    if batch != 1 or tiles >= STREAM_K_MAX_WORKGROUPS or most < 2:
+        return row_blocks, waves, 1
+    splits = min(range(1, most + 1), key=lambda s: ceil_div(tiles * s, NUM_CUS) / s + 0.012 * s)
+    return row_blocks, waves, splits
+
+
 # One-tile-per-workgroup matmuls whose row tiles split evenly over the 8
 # XCDs take the XCD-grouped tile order (MatmulTileMappingFragment.xcd_rows).
 XCD_TILE_ORDER = False
@@ -444,6 +488,10 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         return _assemble_k_resident(decision, function_name, src_a, src_b, pro_a, value_expr, slots, out_key,
                                     extras, helpers, M, K, N, batch)
 
+    if skinny(M, K, N, src_b, pro_b, decision.reduction):
+        return _assemble_skinny(decision, function_name, src_a, src_b, pro_a, value_expr, slots, out_key, extras,
+                                helpers, M, K, N, batch)
+
     full_gather = gathers_full_operands(pro_a) or gathers_full_operands(pro_b)
     wide = WIDE_TILES and (not full_gather or WIDE_GATHER_TILES)
     tile = b_tile_for(select_tile_config(M, K, N, batch=batch, wide=wide), src_b, K, N)
@@ -543,6 +591,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         helpers=tuple(helpers),
         workspace_bytes=workspace,
         workspace_batched=red is not None,
+        workspace_waits=stream_k,
     )
     return KernelGroup(
         kernel=Kernel(fragments=fragments, ctx=ctx),
@@ -595,6 +644,55 @@ def _assemble_row_waves(decision: DecisionView, function_name: str | None, src_a
         dims=(M, K, N),
         grid=(1, M // MatmulRowWavesFragment.TILE_M, 1),
         threads=(MatmulRowWavesFragment.THREADS, 1, 1),
+        ops=decision.ops,
+        strategy=decision.strategy,
+    )
+
+
+def _assemble_skinny(decision: DecisionView, function_name: str | None, src_a: Tensor, src_b: Tensor,
+                     pro_a: ChainCode | None, value_expr: str | None, slots: dict[str, int], out_key: str,
+                     extras: Extras, helpers: list[str], M: int, K: int, N: int, batch: int) -> KernelGroup:
+    """The matmul as one MatmulSkinnyFragment (``skinny`` holds)."""
+    row_blocks, waves, splits = skinny_shape(M, K, N, batch)
+    a_name = param_name(src_a.buffer_key)
+    element = f"{a_name}[(size_t)r * {src_a.row_stride}u + (size_t)k * {src_a.col_stride}u]"
+    raw = f"mt_ld4u({a_name} + (size_t)r * {src_a.row_stride}u + k)"
+    setup, quad = (), None
+    if src_a.col_stride == 1:
+        quad = pro_a.quad_lambda(raw) if pro_a is not None else f"[=](unsigned r, unsigned k) -> mt_f32x4 {{ return {raw}; }}"
+    if pro_a is not None:
+        setup = (f"const auto xt = {pro_a.lambda_transform()};",)
+        element = f"xt({element}, r, k)"
+    frag = MatmulSkinnyFragment(
+        b=(param_name(src_b.buffer_key), src_b.row_stride, src_b.col_stride),
+        c_name=param_name(out_key),
+        row_blocks=row_blocks,
+        waves=waves,
+        splits=splits,
+        a_element=element,
+        a_quad=quad,
+        a_setup=setup,
+        value_expr=value_expr,
+        nt=src_b.col_stride == 1 and 4 * K * N >= SKINNY_STREAM_BYTES,
+    )
+    grid = (ceil_div(N, frag.TILE_N) * splits, ceil_div(M, frag.tile_M), 1)
+    ctx = CodegenContext(
+        function_name=function_name or f"matmul_{decision.anchor.out.name}_fused",
+        buffers=(*(input_param(k) for k in slots), output_param(out_key), *extras.buffers),
+        dims=("M", "K", "N"),
+        tg_x=64 * waves,
+        tg_y=1,
+        threadgroup_decls=(lds_decl("sn_sum", frag.lds_shape),),
+        helpers=tuple(helpers),
+        workspace_bytes=skinny_workspace_bytes(grid[0] // splits * grid[1], row_blocks, splits),
+        workspace_optional=True,
+    )
+    return KernelGroup(
+        kernel=Kernel(fragments=(frag,), ctx=ctx),
+        bindings=(*slots, out_key, *extras.bindings),
+        dims=(M, K, N),
+        grid=grid,
+        threads=(64 * waves, 1, 1),
         ops=decision.ops,
         strategy=decision.strategy,
     )

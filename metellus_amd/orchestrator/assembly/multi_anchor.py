@@ -208,6 +208,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
         threadgroup_decls=tuple(decls),
         helpers=tuple(helpers),
         workspace_bytes=stream_k_workspace_bytes(tile.tile_M, tile.tile_N, n_persistent, anchors=2) if stream_k else 0,
+        workspace_waits=stream_k,
     )
     return KernelGroup(
         kernel=Kernel(fragments=fragments, ctx=ctx),

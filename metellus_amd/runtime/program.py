@@ -157,13 +157,15 @@ class Kernel:
         (launch with grid z = batch size)."""
         if self.ctx.batched:
             return self
-        if self.ctx.workspace_bytes and not self.ctx.workspace_batched:
+        solo = self.ctx.workspace_optional and not self.ctx.workspace_batched
+        if self.ctx.workspace_bytes and not (self.ctx.workspace_batched or solo):
             raise ValueError(f"{self.function_name}: a kernel with a workspace (stream-K) is not batched")
         cached = getattr(self, "_batched", None)
         if cached is None:
             import dataclasses
 
-            ctx = dataclasses.replace(self.ctx, batched=True, function_name=self.ctx.function_name + "_batched")
+            ctx = dataclasses.replace(self.ctx, batched=True, function_name=self.ctx.function_name + "_batched",
+                                      **({"workspace_bytes": 0} if solo else {}))
             cached = Kernel(self.fragments, ctx, self.compile_options)
             self._batched = cached
         return cached
@@ -215,7 +217,7 @@ class Runtime:
             env = {}
         for step in self.fragments:
             step.execute(env)
-        if any(isinstance(s, Dispatch) and s.kernel.workspace_bytes for s in self.fragments):
+        if any(isinstance(s, Dispatch) and s.kernel.ctx.workspace_waits for s in self.fragments):
             from metellus_amd.runtime import hip_backend
 
             hip_backend.check_workspace()  # raises if a stream-K wait gave up
