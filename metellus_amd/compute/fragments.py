@@ -148,10 +148,13 @@ def lds_decl(name: str, shape: tuple[int, ...]) -> str:
 
 @functools.lru_cache(maxsize=1)
 def device_header() -> str:
-    """The hand-written gfx950 device library prepended to every kernel."""
+    """The hand-written gfx950 device library prepended to every kernel, without
+    its comment lines and blank lines: the text is joined, encoded and looked up
+    in the code-object cache on every compile of a kernel."""
     path = os.path.join(os.path.dirname(os.path.dirname(__file__)), "csrc", "mt_device.h")
     with open(path, encoding="utf-8") as f:
-        return f.read()
+        lines = (line.rstrip() for line in f)
+        return "".join(f"{line}\n" for line in lines if line and not line.lstrip().startswith("//"))
 
 
 _PARAM_RE = re.compile(r"^\s*(const\s+)?float\s*\*\s*__restrict__\s+(\w+)\s*$")

@@ -20,6 +20,7 @@ workgroups (``persistent_workgroups``) with a stream-K last round
 
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 
 NUM_CUS = 256  # MI355X compute units (8 XCDs x 32)
@@ -198,6 +199,112 @@ def tile_score(t: TileConfig, M: int, N: int, anchors: int = 1, batch: int = 1) 
     return t.tile_M * t.tile_N * min(wps, 4.0) * useful * fill, wps
 
 
+@dataclass(frozen=True)
+class FillTile:
+    """A tile for problems whose best-scored tile leaves compute units idle, with
+    what one 32-wide k-chunk of it costs on MI355X in microseconds: ``alone`` with
+    at most one workgroup on every other compute unit, where it waits for its own
+    loads and barriers; ``base + each * n`` with n workgroups on every unit, but
+    not below ``shared * n``, the unit's rate.  ``registers``: factor when an operand goes through registers (no direct-to-LDS
+    loads).  Fitted to 10 shapes from 256^3 to 2048 x 4096 x 1024, every tile in 1
+    to 16 parts; the pick is within 10 % of the best of all measured ones."""
+
+    tile: TileConfig
+    alone: float
+    base: float
+    each: float
+    registers: float = 1.05
+    shared: float = 0.0
+
+
+FILL_TILES = (
+    FillTile(TileConfig(256, 256, 32, 4, 4), 4.0, 0.0, 5.2, 1.4),
+    FillTile(TileConfig(256, 128, 32, 4, 4), 2.5, 0.2, 3.4, 1.1),
+    FillTile(TileConfig(128, 256, 32, 4, 4), 2.5, 0.2, 3.4, 1.1),
+    FillTile(TileConfig(128, 128, 32, 2, 2), 1.5, 0.25, 1.55, 1.1),
+    FillTile(TileConfig(128, 64, 32, 2, 2), 1.0, 0.3, 0.85),
+    FillTile(TileConfig(64, 128, 32, 2, 2), 1.0, 0.25, 0.83),
+    FillTile(TileConfig(64, 64, 32, 2, 2), 0.65, 0.3, 0.43, 1.25, shared=0.5),
+    FillTile(TileConfig(32, 64, 32, 1, 2), 0.5, 0.45, 0.165, shared=0.29),
+    FillTile(TileConfig(32, 32, 32, 1, 1), 0.5, 0.42, 0.07, shared=0.175),
+)
+FILL_MAX_PARTS = 16
+# Products of fewer k's keep one sum in one order: as the product of a pair or
+# with a row reduction their kernels give the same bits.
+FILL_PARTS_MIN_K = 1024
+FILL_WORKSPACE = 64 << 20  # bytes of partial sums a split may need (both anchors' of a pair)
+
+
+def fill_time(tiles: int, chunks: int, parts: int, f: FillTile, registers: bool) -> float:
+    """Microseconds of ``tiles`` tiles in ``parts`` parts each: the chunks the
+    busiest compute unit walks, and for a split the partial sums (5 TB/s out, and
+    the last workgroup reads its tile's at about 80 GB/s; 2 us to meet)."""
+    groups = tiles * parts
+    n = ceil_div(groups, NUM_CUS)
+    chunk = f.alone if 2 * groups <= NUM_CUS else max(f.base + f.each * n, f.shared * n)
+    time = ceil_div(chunks, parts) * chunk * (f.registers if registers else 1.0)
+    if parts == 1:
+        return time
+    tile_bytes = 4 * f.tile.tile_M * f.tile.tile_N
+    return time + 2.0 + groups * tile_bytes / 5e6 + parts * tile_bytes / 80e3
+
+
+def _fill_candidates(M: int, N: int, min_waves: int, anchors: int) -> list[FillTile]:
+    fit = [f for f in FILL_TILES if f.tile.tile_M <= _pow2_at_least(M) and f.tile.tile_N <= _pow2_at_least(N)
+           and (anchors == 1 or 16 * f.tile.WM * f.tile.WN * anchors <= 128)]
+    return [f for f in fit if f.tile.sg_M * f.tile.sg_N >= min_waves] or fit
+
+
+@functools.lru_cache(maxsize=1024)
+def filled_parts(M: int, K: int, N: int, batch: int = 1) -> int:
+    """Workgroups per tile of the least ``fill_time`` (one for batched programs and
+    fewer than FILL_PARTS_MIN_K k's).  It depends on the sizes alone: however a
+    product of these sizes is fused, its terms are added in the same order."""
+    chunks = ceil_div(K, 32)
+    best = (float("inf"), 1)
+    for f in _fill_candidates(M, N, 1, 1):
+        t = f.tile
+        tiles = ceil_div(M, t.tile_M) * ceil_div(N, t.tile_N)
+        for parts in range(1, FILL_MAX_PARTS + 1):
+            if parts > 1 and (
+                batch != 1 or K < FILL_PARTS_MIN_K or 2 * parts > chunks or tiles >= STREAM_K_MAX_WORKGROUPS
+                or 2 * tiles * parts * t.tile_M * t.tile_N * 4 > FILL_WORKSPACE
+            ):
+                break
+            best = min(best, (fill_time(batch * tiles, chunks, parts, f, False), parts))
+    return best[1]
+
+
+@functools.lru_cache(maxsize=1024)  # fusion assembles a vertex several times
+def select_filled(M: int, K: int, N: int, batch: int = 1, splittable: bool = True, registers: bool = False,
+                  min_waves: int = 1, anchors: int = 1) -> tuple[TileConfig, int]:
+    """(tile, parts): ``filled_parts`` workgroups per tile, and the tile of least
+    ``fill_time`` for them; tiles of at least ``min_waves`` waves, if M and N reach
+    such a tile's size."""
+    parts = filled_parts(M, K, N, batch) if splittable else 1
+    chunks = ceil_div(K, 32)
+
+    def time(f: FillTile) -> float:
+        t = f.tile
+        tiles = ceil_div(M, t.tile_M) * ceil_div(N, t.tile_N)
+        if parts > 1 and (tiles >= STREAM_K_MAX_WORKGROUPS
+                          or anchors * tiles * parts * t.tile_M * t.tile_N * 4 > FILL_WORKSPACE):
+            return float("inf")
+        return fill_time(batch * tiles, chunks, parts, f, registers)
+
+    return min(_fill_candidates(M, N, min_waves, anchors), key=time).tile, parts
+
+
+def fills(M: int, N: int, t: TileConfig, batch: int = 1) -> bool:
+    """Whether tile ``t`` occupies at least three quarters of the compute units in
+    every round of workgroups (a persistent loop, whose last round is shared out,
+    always does)."""
+    if persistent_workgroups(M, N, t, batch) is not None:
+        return True
+    tiles = batch * ceil_div(M, t.tile_M) * ceil_div(N, t.tile_N)
+    return 4 * tiles >= 3 * NUM_CUS * ceil_div(tiles, NUM_CUS)
+
+
 PERSISTENT = True  # tuning switch for the persistent tile loop
 PERSISTENT_CAPACITY: int | None = None  # override of resident workgroups (tests)
 # Split the last partial round of a persistent loop by k-chunks (stream-K)
@@ -252,8 +359,11 @@ def select_tile_config(
     Measured on MI355X: 256x256 for 4096^3 and the C4/C5 Q.K^T GEMMs
     (16 waves when wide, else 8); 256x128 as 16 waves (wide) or 128x128 as
     8 waves for the C5 P.V GEMM (N = 128, batched heads)."""
-    if FORCE_TILE is not None:
-        return FORCE_TILE
+    return FORCE_TILE or _best_scored(M, N, anchors, batch, wide)
+
+
+@functools.lru_cache(maxsize=1024)
+def _best_scored(M: int, N: int, anchors: int, batch: int, wide: bool) -> TileConfig:
     pool = SINGLE_ANCHOR_TILES if anchors == 1 else DUAL_ANCHOR_TILES
     if wide and anchors == 1:
         pool = WIDE_TILES + pool

@@ -100,6 +100,11 @@ class MatmulTileMappingFragment:
 
     persistent: PersistentTiles | None = None
     xcd_rows: int = 0
+    # (workgroups per tile, tile_K): each takes its share of the tile's k-chunks
+    # (one loop item for the persistent mainloop) and ``MatmulSplitSumFragment``
+    # adds their sums; workgroups of a tile are neighbours along x.  Without the
+    # workspace (a batched variant) the first one walks the whole K.
+    split: tuple[int, int] | None = None
     name: str = "tile_mapping"
     kind: str = "setup"
 
@@ -108,8 +113,27 @@ class MatmulTileMappingFragment:
         """LDS lifetime analysis: fragments up to the loop end run repeatedly."""
         return self.persistent is not None
 
+    def _render_split(self, ctx: CodegenContext) -> str:
+        parts, tile_K = self.split
+        alone = not ctx.workspace_bytes
+        return "\n".join(
+            [
+                f"const unsigned mt_part_i = blockIdx.x % {parts}u;",
+                *(["if (mt_part_i != 0u) return;"] if alone else []),
+                f"const uint3 tg = make_uint3(blockIdx.x / {parts}u, blockIdx.y, blockIdx.z);",
+                f"const unsigned mt_chunks = (K + {tile_K - 1}u) / {tile_K}u;",
+                f"const unsigned mt_kb = {'0u' if alone else f'mt_chunks * mt_part_i / {parts}u'};",
+                f"const unsigned mt_ke = {'mt_chunks' if alone else f'mt_chunks * (mt_part_i + 1u) / {parts}u'};",
+                "unsigned mt_stage = 0u;",
+                "const bool mt_first_tile = true, mt_has_next = false;",
+                "const unsigned mt_next_m0 = 0u, mt_next_n0 = 0u, mt_next_kb = 0u;",
+            ]
+        )
+
     def render(self, ctx: CodegenContext) -> str:
         p = self.persistent
+        if self.split is not None:
+            return self._render_split(ctx)
         if p is None and self.xcd_rows:
             return "\n".join([
                 "// XCD-grouped tile order: this XCD's workgroups share their A row tiles",
@@ -269,6 +293,75 @@ class StreamKFixupFragment:
     @property
     def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
         return ()
+
+
+@dataclass(frozen=True)
+class MatmulSplitSumFragment:
+    """After the mainloop of a tile split over ``parts`` workgroups: each stores
+    its accumulators to the workspace (registers 4q .. 4q + 3 of block b of lane t as
+    the float4 at (4 b + q) NT + t of its part, so a wave's stores are contiguous), and the one
+    that arrives last adds all parts in order and goes on to the epilogue.
+    Nobody waits for anybody."""
+
+    config: MatmulConfig
+    parts: int
+    suffixes: tuple[str, ...] = ("",)
+    name: str = "matmul_split_sum"
+    kind: str = "compute"
+
+    def render(self, ctx: CodegenContext) -> str:
+        if not ctx.workspace_bytes:
+            return ""
+        t, n = self.config.tile, self.parts
+        nt, blocks = t.num_threads, t.WM * t.WN
+        floats = t.tile_M * t.tile_N * len(self.suffixes)
+
+        def loop(k: int) -> list[str]:
+            return [
+                "#pragma unroll",
+                f"    for (int i = 0; i < {t.WM}; ++i)",
+                "#pragma unroll",
+                f"        for (int j = 0; j < {t.WN}; ++j)",
+                "#pragma unroll",
+                "            for (int q = 0; q < 4; ++q) {",
+                f"                const unsigned at = 16u * ((4u * (unsigned)({k * blocks} + i * {t.WN} + j) + (unsigned)q) "
+                f"* {nt}u + threadIdx.x);",
+            ]
+
+        lines = [
+            "{",
+            f"    const unsigned mt_tile = tg.y * (gridDim.x / {n}u) + tg.x;",
+            f"    const mt_sn_part mt_sums(mt_ws + MT_WS_HEAD + (size_t)mt_tile * {n * floats}u, {4 * n * floats}u);",
+        ]
+        for k, sfx in enumerate(self.suffixes):
+            quad = ", ".join(f"acc{sfx}[i][j][4 * q + {e}]" for e in range(4))
+            lines += [*loop(k), f"                mt_sums.put(mt_part_i * {4 * floats}u + at, mt_f32x4{{{quad}}});", "            }"]
+        lines += [
+            f"    if (!mt_sn_arrive(reinterpret_cast<unsigned*>(mt_ws) + mt_tile, {n}u, "
+            f"reinterpret_cast<unsigned*>(&{self.config.a_tile_name}[0][0][0]))) return;",
+        ]
+        for k, sfx in enumerate(self.suffixes):
+            lines += [
+                *loop(k),
+                f"                mt_f32x4 x[{n}];",
+                "#pragma unroll",
+                f"                for (int p = 0; p < {n}; ++p) x[p] = mt_sums.get((unsigned)p * {4 * floats}u + at);",
+                "#pragma unroll",
+                f"                for (int p = 1; p < {n}; ++p) x[0] += x[p];",
+                "#pragma unroll",
+                f"                for (int e = 0; e < 4; ++e) acc{sfx}[i][j][4 * q + e] = x[0][e];",
+                "            }",
+            ]
+        return "\n".join([*lines, "}"])
+
+    @property
+    def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
+        return ()
+
+
+def split_workspace_bytes(tiles: int, tile_M: int, tile_N: int, parts: int, anchors: int = 1) -> int:
+    """Counters, then every part's sums of every tile (every accumulator set)."""
+    return 4 * (STREAM_K_HEAD_WORDS + tiles * parts * tile_M * tile_N * anchors) if parts > 1 else 0
 
 
 @dataclass(frozen=True)

@@ -221,16 +221,13 @@ struct mt_tile_colvec {
         }
     }
 
-    // Any row stride, limits and base alignment (the strides and limits are
-    // run-time values): a slot is loaded with one 128-bit load when its row
-    // start is 16-byte aligned and all 4 columns are in bounds, otherwise
+    // Any row stride, limits and base alignment: a slot is one 128-bit load
+    // (at any element address) when its 4 columns are in bounds, otherwise
     // element by element (out-of-bounds elements are 0, and f is applied to
     // in-bounds elements only).  Same register layout as fetch().
     template <typename F>
     MT_INLINE void fetch_safe(const float* __restrict__ src, unsigned rs, unsigned row0, unsigned col0,
                               unsigned rlim, unsigned clim, unsigned tid, F f, int q = 0, int Q = 1) {
-        const bool aligned =
-            ((rs & 3u) == 0u) && ((reinterpret_cast<unsigned long long>(src) & 15ull) == 0ull) && ((col0 & 3u) == 0u);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             if (!mt_in_part(i, PER, q, Q)) continue;
@@ -240,8 +237,8 @@ struct mt_tile_colvec {
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && gr < rlim && gc < clim) {
                 const float* p = src + (size_t)gr * rs + gc;
-                if (aligned && gc + 3u < clim) {
-                    x = mt_ld4(p);
+                if (gc + 3u < clim) {
+                    x = mt_ld4u(p);
                     x.x = f(x.x, gr, gc);
                     x.y = f(x.y, gr, gc + 1u);
                     x.z = f(x.z, gr, gc + 2u);
@@ -329,6 +326,35 @@ struct mt_tile_rowvec {
                 x.y = f(x.y, gr + 1u, gc);
                 x.z = f(x.z, gr + 2u, gc);
                 x.w = f(x.w, gr + 3u, gc);
+            }
+            v[i] = x;
+        }
+    }
+
+    // Any column stride, limits and base alignment (see mt_tile_colvec).
+    template <typename F>
+    MT_INLINE void fetch_safe(const float* __restrict__ src, unsigned cs, unsigned row0, unsigned col0,
+                              unsigned rlim, unsigned clim, unsigned tid, F f, int q = 0, int Q = 1) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if (!mt_in_part(i, PER, q, Q)) continue;
+            const unsigned idx = tid + i * NT;
+            const unsigned c = idx / RV, r = (idx % RV) * 4u;
+            const unsigned gr = row0 + r, gc = col0 + c;
+            mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
+            if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && gr < rlim && gc < clim) {
+                const float* p = src + gr + (size_t)gc * cs;
+                if (gr + 3u < rlim) {
+                    x = mt_ld4u(p);
+                    x.x = f(x.x, gr, gc);
+                    x.y = f(x.y, gr + 1u, gc);
+                    x.z = f(x.z, gr + 2u, gc);
+                    x.w = f(x.w, gr + 3u, gc);
+                } else {
+                    x.x = f(p[0], gr, gc);
+                    if (gr + 1u < rlim) x.y = f(p[1], gr + 1u, gc);
+                    if (gr + 2u < rlim) x.z = f(p[2], gr + 2u, gc);
+                }
             }
             v[i] = x;
         }
@@ -1268,7 +1294,21 @@ MT_INLINE void mt_sn_put(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_
 MT_INLINE float mt_sn_get(const float* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Count this workgroup in, its mt_sn_put stores complete; true in the last of
+// The same 128 bits at a time, at byte offset `at` of a part of `bytes` bytes
+// (16: the device-scope policy of buffer instructions).
+struct mt_sn_part {
+    __amdgpu_buffer_rsrc_t r;
+    MT_INLINE mt_sn_part(float* base, unsigned bytes) {
+        r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
+    }
+    MT_INLINE void put(unsigned at, mt_f32x4 v) const {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(mt_u32x4, v), r, at, 0, 16);
+    }
+    MT_INLINE mt_f32x4 get(unsigned at) const {
+        return __builtin_bit_cast(mt_f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 16));
+    }
+};
+// Count this workgroup in, its device-scope stores complete; true in the last of
 // `parts` workgroups, which resets the counter for the next launch.
 MT_INLINE bool mt_sn_arrive(unsigned* counter, unsigned parts, unsigned* flag_lds) {
     __builtin_amdgcn_s_waitcnt(0);  // every lane's stores have reached memory

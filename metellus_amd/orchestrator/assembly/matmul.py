@@ -24,15 +24,20 @@ from __future__ import annotations
 import dataclasses
 
 from metellus_amd.compute.fragments import BarrierFragment, CodegenContext, lds_decl
+from metellus_amd.compute.matmul import config as _config
 from metellus_amd.compute.matmul.config import (
+    FILL_PARTS_MIN_K,
     NUM_CUS,
     STREAM_K_MAX_WORKGROUPS,
     TileConfig,
     ceil_div,
+    filled_parts,
+    fills,
     grid_for,
     is_aligned_shape,
     persistent_workgroups,
     resident_workgroups,
+    select_filled,
     select_tile_config,
     uses_stream_k,
 )
@@ -49,6 +54,7 @@ from metellus_amd.compute.matmul.matmul import (
     MatmulRowWavesFragment,
     MatmulSetupFragment,
     MatmulSkinnyFragment,
+    MatmulSplitSumFragment,
     MatmulTileMappingFragment,
     PersistentLoopEndFragment,
     PersistentTiles,
@@ -58,6 +64,7 @@ from metellus_amd.compute.matmul.matmul import (
     rr_row_blocks,
     rr_workspace_bytes,
     skinny_workspace_bytes,
+    split_workspace_bytes,
     stream_k_workspace_bytes,
 )
 from metellus_amd.memory.memory import TgLoadFragment, dma_offsets_fit
@@ -119,6 +126,13 @@ def operand_load(
     else:
         mode = "scalar"
     gather = gathers(prologue)
+    if mode == "scalar" and prologue is None:
+        # odd sizes or strides: 128-bit loads at any element address, bounds
+        # per slot (a prologue keeps the element loader, which defers it)
+        if cs == 1 and pitch % 4 == 0:
+            mode = "colvec_safe"
+        elif rs == 1:
+            mode = "rowvec_safe"
     lam = prologue.lambda_transform() if prologue is not None and not gather else None
     # one gather per 128-bit slot when the operands do not change along it
     along = {"colvec": "col", "rowvec": "row"}.get(mode)
@@ -339,6 +353,7 @@ def k_resident_chunks(M: int, N: int, batch: int = 1) -> int:
 # 60 us, 64 x 4096 @ 4096 x 4096 91 -> 34 us, 13 x 1000 @ 1000 x 3001 46 -> 10 us.
 SKINNY = True
 SKINNY_MAX_M = 64
+SKINNY_ANY_K_M = 32  # more rows only for products of at least FILL_PARTS_MIN_K k's
 SKINNY_MIN_B = 8192  # elements of B: up to here the call is a tile or two, all launch
 SKINNY_MAX_SPLITS = 16
 # B of more bytes than this is not kept by the 256 MiB Infinity Cache from one
@@ -355,6 +370,8 @@ def skinny(M: int, K: int, N: int, src_b: Tensor, pro_b: ChainCode | None, reduc
         return False
     if src_b.col_stride != 1 and src_b.row_stride != 1:
         return False
+    if M > SKINNY_ANY_K_M and K < FILL_PARTS_MIN_K:
+        return False  # one sum in one order, as in every kernel of such a product
     return M <= SKINNY_MAX_M and K * N > SKINNY_MIN_B
 
 
@@ -388,6 +405,22 @@ def xcd_rows(grid: tuple[int, int, int]) -> int:
     return gy // 8
 
 
+# Single matmuls whose best-scored tile leaves compute units idle take
+# ``select_filled``'s tile and split.  Measured on MI355X, before -> after: 256^3
+# 23.5 -> 8.2 us, 512^3 43 -> 13 us, 1024^3 84 -> 24 us, 2048 x 4096 x 1024 with
+# W^T 320 -> 116 us, 1024 x 2048 x 4096 with X^T 217 -> 133 us, 128 x 4096 x 4096
+# 194 -> 42 us, 300 x 777 x 1000 47 -> 28 us.
+FILL = True
+FILL_MIN_K = 128  # fewer k-chunks are over before a smaller tile pays
+
+
+def fill(M: int, K: int, N: int, batch: int = 1) -> bool:
+    """Whether a product of these sizes (and ``batch`` like it) has too few tiles,
+    or a nearly empty last round of them, by its best-scored tile."""
+    return FILL and _config.FORCE_TILE is None and K >= FILL_MIN_K and not fills(
+        M, N, select_tile_config(M, K, N, batch=batch, wide=WIDE_TILES), batch)
+
+
 def load_spread(*prologues: ChainCode | None) -> int:
     """Spread parts for a mainloop whose A / B prologues are ``prologues``."""
     return LOAD_SPREAD if any(gathers_full_operands(p) for p in prologues) else 0
@@ -401,15 +434,16 @@ def gathers_full_operands(prologue: ChainCode | None) -> bool:
     return gathers(prologue) and not prologue.broadcast_operands_only
 
 
-def b_tile_for(tile: TileConfig, src_b: Tensor, K: int, N: int) -> TileConfig:
+def b_tile_for(tile: TileConfig, src_b: Tensor, K: int, N: int, prologue: bool = False) -> TileConfig:
     """Row pitch of the B tile in LDS.  A B operand read 128-bit along
     columns is committed with 128-bit stores and keeps a pitch that is a
     multiple of 4 floats.  Any other B (a transposed view such as K^T, or
     odd strides) is committed by 32-bit stores walking down columns, where a
     pitch of tile_N + 4 puts rows 0, 4, 8, ... of a column on colliding
     banks; an odd pitch (tile_N + 3) spreads them (measured on MI355X for
-    the attention S = Q @ K^T kernel: 372.8 -> 360.5 us)."""
-    if src_b.col_stride == 1 and src_b.row_stride % 4 == 0 and N % 4 == 0:
+    the attention S = Q @ K^T kernel: 372.8 -> 360.5 us).  ``prologue``: B has
+    one, so odd sizes go element by element."""
+    if src_b.col_stride == 1 and (not prologue or (src_b.row_stride % 4 == 0 and N % 4 == 0)):
         return tile
     return dataclasses.replace(tile, b_pad=3)
 
@@ -494,16 +528,31 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
 
     full_gather = gathers_full_operands(pro_a) or gathers_full_operands(pro_b)
     wide = WIDE_TILES and (not full_gather or WIDE_GATHER_TILES)
-    tile = b_tile_for(select_tile_config(M, K, N, batch=batch, wide=wide), src_b, K, N)
+    tile = b_tile_for(select_tile_config(M, K, N, batch=batch, wide=wide), src_b, K, N, pro_b is not None)
     aligned = is_aligned_shape(M, K, N, tile)
     if tile.num_threads > 512 and not aligned:
         # 16-wave tiles only without bounds checks (their masks cost registers)
-        tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b, K, N)
+        tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b, K, N, pro_b is not None)
         aligned = is_aligned_shape(M, K, N, tile)
     if decision.reduction is not None and (tile.tile_N, tile.sg_M, tile.sg_N) == (256, 4, 4):
         # each wave reduces its rows over its own columns: 2x8 waves leave
         # half as many rows to every wave's lane exchanges
         tile = dataclasses.replace(tile, sg_M=2, sg_N=8)
+
+    parts, filled = 1, decision.reduction is None and fill(M, K, N, batch)
+    if filled:
+        # Divisors tested once per tile (mt_plain) keep their tiles whole: a
+        # split's loop would test them at every commit.  A prologue's operands
+        # are loaded once per tile: not by one or two waves.
+        direct = dma_layouts(tile, (src_a,), (src_b,), (pro_a,), (pro_b,), True)
+        prologues = [p for p in (pro_a, pro_b) if p is not None]
+        tile, parts = select_filled(
+            M, K, N, batch, splittable=not any(p.plain_divisors() for p in prologues),
+            registers=not aligned or direct.a_layout == "pad" or direct.b_layout == "pad",
+            min_waves=4 if prologues else 1,
+        )
+        tile = b_tile_for(tile, src_b, K, N, pro_b is not None)
+        aligned = is_aligned_shape(M, K, N, tile)
 
     tile = dma_layouts(tile, (src_a,), (src_b,), (pro_a,), (pro_b,), aligned)
     if full_gather and tile.b_layout == "pad":
@@ -531,7 +580,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
                           M=M, K=K, N=N, aligned=aligned, prologue=pro_a)
     b_load = operand_load(name="load_B_tile", src=src_b, dst="B_tile", tile=tile, side="b",
                           M=M, K=K, N=N, aligned=aligned, prologue=pro_b)
-    n_persistent = persistent_workgroups(M, N, tile, batch)
+    n_persistent = None if filled else persistent_workgroups(M, N, tile, batch)
     red = decision.reduction
     # the row-reduction epilogue needs each tile whole in one workgroup
     stream_k = red is None and uses_stream_k(M, K, N, tile, n_persistent, batch)
@@ -546,7 +595,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         fragments=(a_load, b_load, BarrierFragment("inputs_ready"), MatmulComputeFragment(config, split=True),
                    BarrierFragment("compute_done")),
         K_dim_var="K",
-        persistent=persistent is not None,
+        persistent=persistent is not None or parts > 1,
         spread=spread,
         spread_dma=LOAD_SPREAD_DMA,
         held=held_groups(K, tile, spread),
@@ -563,11 +612,13 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
                                              value_expr=value_expr, check=not aligned, local=local_rr)
     fragments = (
         *((MatmulRowReduceSetupFragment(local=local_rr),) if red is not None else ()),
-        MatmulTileMappingFragment(persistent, xcd_rows=xcd_rows(grid_for(M, N, tile)) if persistent is None else 0),
+        MatmulTileMappingFragment(persistent, xcd_rows=xcd_rows(grid_for(M, N, tile)) if persistent is None else 0,
+                                  split=(parts, tile.tile_K) if parts > 1 else None),
         ThreadIndexFragment(tile),
         MatmulSetupFragment(config),
         mainloop,
-        exact_retry(config, src_a, src_b, pro_a, pro_b, persistent=persistent is not None),
+        exact_retry(config, src_a, src_b, pro_a, pro_b, persistent=persistent is not None or parts > 1),
+        *((MatmulSplitSumFragment(config, parts),) if parts > 1 else ()),
         *((StreamKFixupFragment(config),) if stream_k else ()),
         store,
         *((PersistentLoopEndFragment(),) if persistent else ()),
@@ -580,6 +631,8 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         decls += (lds_decl("row_red", rr_lds_shape(tile)),)
     else:
         workspace = stream_k_workspace_bytes(tile.tile_M, tile.tile_N, n_persistent) if stream_k else 0
+        grid_x, grid_y, _ = grid_for(M, N, tile)
+        workspace = workspace or split_workspace_bytes(grid_x * grid_y, tile.tile_M, tile.tile_N, parts)
     ctx = CodegenContext(
         function_name=function_name or f"matmul_{anchor.out.name}_fused",
         buffers=(*(input_param(k) for k in slots), output_param(out_key), *extras.buffers,
@@ -591,13 +644,14 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         helpers=tuple(helpers),
         workspace_bytes=workspace,
         workspace_batched=red is not None,
+        workspace_optional=parts > 1,
         workspace_waits=stream_k,
     )
     return KernelGroup(
         kernel=Kernel(fragments=fragments, ctx=ctx),
         bindings=(*slots, out_key, *extras.bindings, *red_keys),
         dims=(M, K, N),
-        grid=(n_persistent, 1, 1) if n_persistent else grid_for(M, N, tile),
+        grid=(n_persistent, 1, 1) if n_persistent else (ceil_div(N, tile.tile_N) * parts, ceil_div(M, tile.tile_M), 1),
         threads=(tile.tg_x, 1, 1),
         ops=decision.ops,
         strategy=decision.strategy,

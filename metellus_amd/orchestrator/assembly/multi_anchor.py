@@ -23,6 +23,7 @@ from metellus_amd.compute.matmul.config import (
     grid_for,
     is_aligned_shape,
     persistent_workgroups,
+    select_filled,
     select_tile_config,
     uses_stream_k,
 )
@@ -32,11 +33,13 @@ from metellus_amd.compute.matmul.matmul import (
     MatmulEpilogueStoreFragment,
     MatmulMainloopFragment,
     MatmulSetupFragment,
+    MatmulSplitSumFragment,
     MatmulTileMappingFragment,
     PersistentLoopEndFragment,
     PersistentTiles,
     StreamKFixupFragment,
     ThreadIndexFragment,
+    split_workspace_bytes,
     stream_k_workspace_bytes,
 )
 from metellus_amd.orchestrator.assembly.decision import DecisionView
@@ -65,7 +68,11 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
     assert all(isinstance(t, Tensor) for t in (*src_a, *src_b))
     out_key = merge.out.buffer_key
     tile = select_tile_config(M, max(K0, K1), N, anchors=2, batch=batch)
-    padded = [b_tile_for(tile, src_b[i], (K0, K1)[i], N) for i in range(2)]
+    parts, filled = 1, shared and _mm.fill(M, K0, N, batch)
+    if filled:
+        prologues = any((*pro_a, *pro_b))
+        tile, parts = select_filled(M, K0, N, batch, min_waves=4 if prologues else 1, anchors=2)
+    padded = [b_tile_for(tile, src_b[i], (K0, K1)[i], N, bool(pro_b[i])) for i in range(2)]
     if all(p.b_pad != tile.b_pad for p in padded):
         tile = padded[0]  # both B tiles committed by 32-bit stores
     aligned = is_aligned_shape(M, K0, N, tile) and is_aligned_shape(M, K1, N, tile)
@@ -124,7 +131,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
         return operand_load(name=f"load_B{i}_tile", src=src_b[i], dst=f"B{i}_tile", tile=tile, side="b",
                             M=M, K=ks[i], N=N, aligned=aligned, k_limit=kvars[i], prologue=tf_b[i])
 
-    n_persistent = persistent_workgroups(M, N, tile, batch, anchors=2) if shared else None
+    n_persistent = persistent_workgroups(M, N, tile, batch, anchors=2) if shared and not filled else None
     stream_k = uses_stream_k(M, K0, N, tile, n_persistent, batch)
     persistent = PersistentTiles(tile.tile_M, tile.tile_N, stream_k=stream_k, tile_K=tile.tile_K) \
         if n_persistent else None
@@ -144,7 +151,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
                     BarrierFragment("compute_done"),
                 ),
                 K_dim_var="K",
-                persistent=persistent is not None,
+                persistent=persistent is not None or parts > 1,
                 spread=_mm.load_spread(*tf_b),
                 spread_dma=_mm.LOAD_SPREAD_DMA,
             )
@@ -172,16 +179,17 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
 
     store = MatmulEpilogueStoreFragment(configs[0], value_expr=value_expr, suffixes=suffixes, check=not aligned)
     fragments = (
-        MatmulTileMappingFragment(persistent),
+        MatmulTileMappingFragment(persistent, split=(parts, tile.tile_K) if parts > 1 else None),
         ThreadIndexFragment(tile),
         MatmulSetupFragment(configs[0], accumulator_suffix=suffixes[0]),
         MatmulSetupFragment(configs[1], accumulator_suffix=suffixes[1], emit_thread_coords=False),
         *mainloops,
         *(
             exact_retry(configs[i], src_a[0 if shared else i], src_b[i], tf_a[0 if shared else i], tf_b[i],
-                        suffix=suffixes[i], persistent=persistent is not None)
+                        suffix=suffixes[i], persistent=persistent is not None or parts > 1)
             for i in range(2)
         ),
+        *((MatmulSplitSumFragment(configs[0], parts, suffixes=suffixes),) if parts > 1 else ()),
         *((StreamKFixupFragment(configs[0], suffixes=suffixes),) if stream_k else ()),
         store,
         *((PersistentLoopEndFragment(),) if persistent else ()),
@@ -196,6 +204,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
         dim_names, dim_values = ("M", "K", "N"), (M, K0, N)
     else:
         dim_names, dim_values = ("M", "K0", "K1", "N"), (M, K0, K1, N)
+    grid_x, grid_y, _ = grid_for(M, N, tile)
     ctx = CodegenContext(
         # the reference's name; a merge chain (an extension) is named apart
         function_name=function_name or (
@@ -207,14 +216,16 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
         tg_y=1,
         threadgroup_decls=tuple(decls),
         helpers=tuple(helpers),
-        workspace_bytes=stream_k_workspace_bytes(tile.tile_M, tile.tile_N, n_persistent, anchors=2) if stream_k else 0,
+        workspace_bytes=stream_k_workspace_bytes(tile.tile_M, tile.tile_N, n_persistent, anchors=2) if stream_k
+        else split_workspace_bytes(grid_x * grid_y, tile.tile_M, tile.tile_N, parts, anchors=2),
+        workspace_optional=parts > 1,
         workspace_waits=stream_k,
     )
     return KernelGroup(
         kernel=Kernel(fragments=fragments, ctx=ctx),
         bindings=(*keys, out_key, *extras.bindings),
         dims=dim_values,
-        grid=(n_persistent, 1, 1) if n_persistent else grid_for(M, N, tile),
+        grid=(n_persistent, 1, 1) if n_persistent else (grid_x * parts, grid_y, 1),
         threads=(tile.tg_x, 1, 1),
         ops=decision.ops,
         strategy=decision.strategy,

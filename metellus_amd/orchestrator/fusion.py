@@ -382,6 +382,17 @@ MATMUL_REDUCTION_EPILOGUES = False
 _ROW_REDUCTIONS = ("sum", "max", "min", "product")
 
 
+def _summed_in_parts(op: MatmulOp) -> bool:
+    """A product whose own kernel adds its terms in several parts: with the
+    reduction it would be one sum, rounding differently from the partition
+    without the extension (and slower: its parts are what fill the GPU)."""
+    from metellus_amd.orchestrator.assembly import matmul as mm
+
+    M, K = op.a.shape
+    N = op.b.shape[1]
+    return mm.skinny(M, K, N, op.b, None, None) or (mm.fill(M, K, N) and mm.filled_parts(M, K, N) > 1)
+
+
 def try_matmul_reduction_fuse(graph: Graph, blacklist: Blacklist) -> Graph | None:
     """(Extension, ``MATMUL_REDUCTION_EPILOGUES``.)  A vertex holding one
     reduction whose input is the last output of a vertex holding one matmul
@@ -397,7 +408,7 @@ def try_matmul_reduction_fuse(graph: Graph, blacklist: Blacklist) -> Graph | Non
             continue
         if not all(isinstance(op, ElementwiseOp) and _is_lane_agnostic(op) for op in a.ops[1:]):
             continue
-        if (a.op_ids | r.op_ids) in blacklist:
+        if (a.op_ids | r.op_ids) in blacklist or _summed_in_parts(a.ops[0]):
             continue
         return graph.replace(absorbed=(a, r), ops=_by_position(graph, (*a.ops, *r.ops)))
     return None

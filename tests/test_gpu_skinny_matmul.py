@@ -14,7 +14,7 @@ from metellus_amd.orchestrator.assembly import matmul as mm
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 129, 64), (1, 4096, 65), (3, 128, 128), (16, 1000, 331), (17, 77, 1001), (33, 515, 258), (64, 2048, 67),
+SHAPES = [(1, 129, 64), (1, 4096, 65), (3, 128, 128), (16, 1000, 331), (17, 77, 1001), (33, 1027, 258), (64, 2048, 67),
           (8, 4096, 1024)]
 
 
@@ -75,7 +75,7 @@ def test_shapes_and_views(shape, a_view, b_view):
 @pytest.mark.parametrize("prologue", ["none", "row", "col", "scalar"])
 @pytest.mark.parametrize("a_view", [False, True])
 def test_prologues(prologue, a_view):
-    for shape in ((8, 1000, 331), (40, 515, 131)):
+    for shape in ((8, 1000, 331), (40, 1031, 131)):
         print(f"skinny prologue {prologue} {shape} a_view={a_view}", flush=True)
         ops, out, ref, bound = _program(shape, a_view=a_view, prologue=prologue)
         assert "mt_sn_mainloop<" in compile_program(ops)[-1].kernel.source.split('extern "C"')[-1]
