@@ -225,7 +225,7 @@ FILL_TILES = (
     FillTile(TileConfig(128, 64, 32, 2, 2), 1.0, 0.3, 0.85),
     FillTile(TileConfig(64, 128, 32, 2, 2), 1.0, 0.25, 0.83),
     FillTile(TileConfig(64, 64, 32, 2, 2), 0.65, 0.3, 0.43, 1.25, shared=0.5),
-    FillTile(TileConfig(32, 64, 32, 1, 2), 0.5, 0.45, 0.165, shared=0.29),
+    FillTile(TileConfig(32, 64, 32, 1, 2), 0.5, 0.45, 0.165, shared=0.32),
     FillTile(TileConfig(32, 32, 32, 1, 1), 0.5, 0.42, 0.07, shared=0.175),
 )
 FILL_MAX_PARTS = 16

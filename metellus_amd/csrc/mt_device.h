@@ -192,7 +192,25 @@ __host__ __device__ __forceinline__ constexpr bool mt_in_part(int i, int n, int 
     return Q <= 1 || (i * Q) / n == q;
 }
 
-// Vectorised along columns: cs == 1, rs % 4 == 0, COLS % 4 == 0, clim % 4 == 0.
+// Four consecutive elements from p, of which the first `left` (at least one)
+// are inside the matrix: one 128-bit load at any element address, or element by
+// element at its edge (0 outside).
+MT_INLINE mt_f32x4 mt_ld_slot(const float* p, unsigned left) {
+    if (left >= 4u) return mt_ld4u(p);
+    mt_f32x4 x = {p[0], 0.f, 0.f, 0.f};
+    if (left > 1u) x.y = p[1];
+    if (left > 2u) x.z = p[2];
+    return x;
+}
+// The slot's elements outside the matrix are 0 again after a transform.
+MT_INLINE void mt_clear_slot(mt_f32x4& x, unsigned left) {
+    if (left < 2u) x.y = 0.f;
+    if (left < 3u) x.z = 0.f;
+    if (left < 4u) x.w = 0.f;
+}
+
+// Vectorised along columns: cs == 1, COLS % 4 == 0, any row stride and (CHECK)
+// limits.
 template <int ROWS, int COLS, int NT>
 struct mt_tile_colvec {
     static constexpr int CV = COLS / 4;
@@ -211,11 +229,12 @@ struct mt_tile_colvec {
             const unsigned gr = row0 + r, gc = col0 + c;
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rlim && gc < clim))) {
-                x = mt_ld4(src + (size_t)gr * rs + gc);
+                const unsigned left = CHECK ? clim - gc : 4u;
+                x = mt_ld_slot(src + (size_t)gr * rs + gc, left);
                 x.x = f(x.x, gr, gc);
-                x.y = f(x.y, gr, gc + 1u);
-                x.z = f(x.z, gr, gc + 2u);
-                x.w = f(x.w, gr, gc + 3u);
+                if (left > 1u) x.y = f(x.y, gr, gc + 1u);
+                if (left > 2u) x.z = f(x.z, gr, gc + 2u);
+                if (left > 3u) x.w = f(x.w, gr, gc + 3u);
             }
             v[i] = x;
         }
@@ -292,17 +311,19 @@ struct mt_tile_colvec {
             const unsigned r = idx / CV, c = (idx % CV) * 4u;
             const unsigned gr = r0 + r, gc = c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rl && gc < cl))) {
+                const unsigned left = CHECK ? cl - gc : 4u;
                 v[i].x = f(v[i].x, gr, gc);
-                v[i].y = f(v[i].y, gr, gc + 1u);
-                v[i].z = f(v[i].z, gr, gc + 2u);
-                v[i].w = f(v[i].w, gr, gc + 3u);
+                if (left > 1u) v[i].y = f(v[i].y, gr, gc + 1u);
+                if (left > 2u) v[i].z = f(v[i].z, gr, gc + 2u);
+                if (left > 3u) v[i].w = f(v[i].w, gr, gc + 3u);
             }
         }
         commit<LD>(lds, tid);
     }
 };
 
-// Vectorised along rows: rs == 1, cs % 4 == 0, ROWS % 4 == 0, rlim % 4 == 0.
+// Vectorised along rows: rs == 1, ROWS % 4 == 0, any column stride and (CHECK)
+// limits.
 template <int ROWS, int COLS, int NT>
 struct mt_tile_rowvec {
     static constexpr int RV = ROWS / 4;
@@ -321,40 +342,12 @@ struct mt_tile_rowvec {
             const unsigned gr = row0 + r, gc = col0 + c;
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rlim && gc < clim))) {
-                x = mt_ld4(src + gr + (size_t)gc * cs);
+                const unsigned left = CHECK ? rlim - gr : 4u;
+                x = mt_ld_slot(src + gr + (size_t)gc * cs, left);
                 x.x = f(x.x, gr, gc);
-                x.y = f(x.y, gr + 1u, gc);
-                x.z = f(x.z, gr + 2u, gc);
-                x.w = f(x.w, gr + 3u, gc);
-            }
-            v[i] = x;
-        }
-    }
-
-    // Any column stride, limits and base alignment (see mt_tile_colvec).
-    template <typename F>
-    MT_INLINE void fetch_safe(const float* __restrict__ src, unsigned cs, unsigned row0, unsigned col0,
-                              unsigned rlim, unsigned clim, unsigned tid, F f, int q = 0, int Q = 1) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            if (!mt_in_part(i, PER, q, Q)) continue;
-            const unsigned idx = tid + i * NT;
-            const unsigned c = idx / RV, r = (idx % RV) * 4u;
-            const unsigned gr = row0 + r, gc = col0 + c;
-            mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
-            if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && gr < rlim && gc < clim) {
-                const float* p = src + gr + (size_t)gc * cs;
-                if (gr + 3u < rlim) {
-                    x = mt_ld4u(p);
-                    x.x = f(x.x, gr, gc);
-                    x.y = f(x.y, gr + 1u, gc);
-                    x.z = f(x.z, gr + 2u, gc);
-                    x.w = f(x.w, gr + 3u, gc);
-                } else {
-                    x.x = f(p[0], gr, gc);
-                    if (gr + 1u < rlim) x.y = f(p[1], gr + 1u, gc);
-                    if (gr + 2u < rlim) x.z = f(p[2], gr + 2u, gc);
-                }
+                if (left > 1u) x.y = f(x.y, gr + 1u, gc);
+                if (left > 2u) x.z = f(x.z, gr + 2u, gc);
+                if (left > 3u) x.w = f(x.w, gr + 3u, gc);
             }
             v[i] = x;
         }
@@ -392,10 +385,11 @@ struct mt_tile_rowvec {
             const unsigned c = idx / RV, r = (idx % RV) * 4u;
             const unsigned gr = r0 + r, gc = c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rl && gc < cl))) {
+                const unsigned left = CHECK ? rl - gr : 4u;
                 v[i].x = f(v[i].x, gr, gc);
-                v[i].y = f(v[i].y, gr + 1u, gc);
-                v[i].z = f(v[i].z, gr + 2u, gc);
-                v[i].w = f(v[i].w, gr + 3u, gc);
+                if (left > 1u) v[i].y = f(v[i].y, gr + 1u, gc);
+                if (left > 2u) v[i].z = f(v[i].z, gr + 2u, gc);
+                if (left > 3u) v[i].w = f(v[i].w, gr + 3u, gc);
             }
         }
         commit<LD>(lds, tid);
@@ -502,9 +496,11 @@ struct mt_tile_colvec_g : mt_tile_colvec<ROWS, COLS, NT> {
             const unsigned gr = row0 + r, gc = col0 + c;
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rlim && gc < clim))) {
-                x = mt_ld4(src + (size_t)gr * rs + gc);
+                const unsigned left = CHECK ? clim - gc : 4u;
+                x = mt_ld_slot(src + (size_t)gr * rs + gc, left);
 #pragma unroll
-                for (int j = 0; j < NG; ++j) ex[i][j] = g(gr, gc + (unsigned)j);
+                for (int j = 0; j < NG; ++j)
+                    if (j == 0 || (unsigned)j < left) ex[i][j] = g(gr, gc + (unsigned)j);
             }
             this->v[i] = x;
         }
@@ -534,7 +530,8 @@ struct mt_tile_colvec_g : mt_tile_colvec<ROWS, COLS, NT> {
             const unsigned gr = this->r0 + r, gc = this->c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < this->rl && gc < this->cl))) {
 #pragma unroll
-                for (int j = 0; j < NG; ++j) ok = ok && p(ex[i][j]);
+                for (int j = 0; j < NG; ++j)
+                    if (j == 0 || !CHECK || (unsigned)j < this->cl - gc) ok = ok && p(ex[i][j]);
             }
         }
         return __builtin_amdgcn_ballot_w64(!ok) == 0ull;
@@ -564,6 +561,7 @@ struct mt_tile_colvec_g : mt_tile_colvec<ROWS, COLS, NT> {
                 this->v[i].y = a(this->v[i].y, ex[i][1 % NG]);
                 this->v[i].z = a(this->v[i].z, ex[i][2 % NG]);
                 this->v[i].w = a(this->v[i].w, ex[i][3 % NG]);
+                if (CHECK) mt_clear_slot(this->v[i], this->cl - gc);
             }
         }
         Base::template commit<LD>(lds, tid);
@@ -591,9 +589,11 @@ struct mt_tile_rowvec_g : mt_tile_rowvec<ROWS, COLS, NT> {
             const unsigned gr = row0 + r, gc = col0 + c;
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rlim && gc < clim))) {
-                x = mt_ld4(src + gr + (size_t)gc * cs);
+                const unsigned left = CHECK ? rlim - gr : 4u;
+                x = mt_ld_slot(src + gr + (size_t)gc * cs, left);
 #pragma unroll
-                for (int j = 0; j < NG; ++j) ex[i][j] = g(gr + (unsigned)j, gc);
+                for (int j = 0; j < NG; ++j)
+                    if (j == 0 || (unsigned)j < left) ex[i][j] = g(gr + (unsigned)j, gc);
             }
             this->v[i] = x;
         }
@@ -619,7 +619,8 @@ struct mt_tile_rowvec_g : mt_tile_rowvec<ROWS, COLS, NT> {
             const unsigned gr = this->r0 + r, gc = this->c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < this->rl && gc < this->cl))) {
 #pragma unroll
-                for (int j = 0; j < NG; ++j) ok = ok && p(ex[i][j]);
+                for (int j = 0; j < NG; ++j)
+                    if (j == 0 || !CHECK || (unsigned)j < this->rl - gr) ok = ok && p(ex[i][j]);
             }
         }
         return __builtin_amdgcn_ballot_w64(!ok) == 0ull;
@@ -649,6 +650,7 @@ struct mt_tile_rowvec_g : mt_tile_rowvec<ROWS, COLS, NT> {
                 this->v[i].y = a(this->v[i].y, ex[i][1 % NG]);
                 this->v[i].z = a(this->v[i].z, ex[i][2 % NG]);
                 this->v[i].w = a(this->v[i].w, ex[i][3 % NG]);
+                if (CHECK) mt_clear_slot(this->v[i], this->rl - gr);
             }
         }
         Base::template commit<LD>(lds, tid);

@@ -61,9 +61,6 @@ def _is_int(s: str) -> bool:
     return True
 
 
-_SAFE_MODES = ("colvec_safe", "rowvec_safe")  # bounds checked in every fetch, transforms applied there
-
-
 def dma_offsets_fit(rows: int, cols: int, row_stride) -> bool:
     """A direct-to-LDS loader keeps each lane's byte offset from the tile
     origin in 32 bits (``mt_tile_dma``): the row stride must be a literal and
@@ -91,9 +88,7 @@ class TgLoadFragment:
     # gfx950 layout controls
     dst_pitch: int | None = None
     stages: int = 1
-    # "colvec" | "rowvec" | "scalar" | "dma", or "colvec_safe" | "rowvec_safe": the
-    # vector loaders at any stride and limit (default: from strides)
-    mode: str | None = None
+    mode: str | None = None  # "colvec" | "rowvec" | "scalar" | "dma" (default: from strides)
     transform_lambda: str | None = None
     # Apply the transform when the registers are written to LDS rather than
     # when the loads return, so a pipelined mainloop does not wait for the
@@ -200,9 +195,9 @@ class TgLoadFragment:
             return (f"const mt_tile_dma<{rows}, {cols}, {self.num_threads}, {swz}> "
                     f"{self.loader}({self.src_row_stride}, threadIdx.x);")
         tmpl = {"colvec": "mt_tile_colvec", "colvec_safe": "mt_tile_colvec", "rowvec": "mt_tile_rowvec",
-                "rowvec_safe": "mt_tile_rowvec", "scalar": "mt_tile_scalar"}[mode]
+                "scalar": "mt_tile_scalar"}[mode]
         if self.gathering:
-            if mode in _SAFE_MODES or self.apply_lambda is None or self.n_gathered < 1:
+            if mode == "colvec_safe" or self.apply_lambda is None or self.n_gathered < 1:
                 raise ValueError(f"{self.name}: gather/apply needs a proven load mode and an apply lambda")
             if self.gather_per_slot and mode not in ("colvec", "rowvec"):
                 raise ValueError(f"{self.name}: per-slot gathers need a vectorised load mode")
@@ -256,18 +251,18 @@ class TgLoadFragment:
         clim = self.col_limit if self.col_limit is not None else "0xffffffffu"
         check = "true" if self.check else "false"
         mode = self.resolved_mode()
-        deferred = self.defer_transform and self._has_transform() and mode not in _SAFE_MODES
+        deferred = self.defer_transform and self._has_transform() and mode != "colvec_safe"
         if self.gathering:
             head = f"{self.loader}.template fetch_gather<{check}>({self.src_name}, "
             deferred = False
-        elif mode in _SAFE_MODES:
+        elif mode == "colvec_safe":
             head = f"{self.loader}.fetch_safe({self.src_name}, "
         else:
             verb = "fetch_raw" if deferred else "fetch"
             head = f"{self.loader}.template {verb}<{check}>({self.src_name}, "
         if mode in ("colvec", "colvec_safe"):
             strides = f"{self.src_row_stride}"
-        elif mode in ("rowvec", "rowvec_safe"):
+        elif mode == "rowvec":
             strides = f"{self.src_col_stride}"
         else:
             strides = f"{self.src_row_stride}, {self.src_col_stride}"
@@ -320,7 +315,7 @@ class TgLoadFragment:
                 f"{self.loader}.template commit_apply<{self.pitch}, {check}>"
                 f"({self.stage_ptr(stage)}, {tid}, xa_{d});"
             )
-        if self.defer_transform and self._has_transform() and self.resolved_mode() not in _SAFE_MODES:
+        if self.defer_transform and self._has_transform() and self.resolved_mode() != "colvec_safe":
             check = "true" if self.check else "false"
             return (
                 f"{self.loader}.template commit_xf<{self.pitch}, {check}>"

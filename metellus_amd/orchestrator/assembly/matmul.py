@@ -113,26 +113,18 @@ def operand_load(
         shape, pitch = (tile.tile_M, tile.tile_K), tile.lda
         row_start, col_start = "tile_m0", "k_chunk"
         row_lim, col_lim = "M", k_limit
-        rows_total, cols_total = M, K
     else:
         shape, pitch = (tile.tile_K, tile.tile_N), tile.ldb
         row_start, col_start = "k_chunk", "tile_n0"
         row_lim, col_lim = k_limit, "N"
-        rows_total, cols_total = K, N
-    if cs == 1 and rs % 4 == 0 and cols_total % 4 == 0 and pitch % 4 == 0:
+    # 128-bit loads at any element address, bounds per slot where sizes are odd
+    if cs == 1 and pitch % 4 == 0:
         mode = "colvec"
-    elif rs == 1 and cs % 4 == 0 and rows_total % 4 == 0:
+    elif rs == 1:
         mode = "rowvec"
     else:
         mode = "scalar"
     gather = gathers(prologue)
-    if mode == "scalar" and prologue is None:
-        # odd sizes or strides: 128-bit loads at any element address, bounds
-        # per slot (a prologue keeps the element loader, which defers it)
-        if cs == 1 and pitch % 4 == 0:
-            mode = "colvec_safe"
-        elif rs == 1:
-            mode = "rowvec_safe"
     lam = prologue.lambda_transform() if prologue is not None and not gather else None
     # one gather per 128-bit slot when the operands do not change along it
     along = {"colvec": "col", "rowvec": "row"}.get(mode)
@@ -434,16 +426,15 @@ def gathers_full_operands(prologue: ChainCode | None) -> bool:
     return gathers(prologue) and not prologue.broadcast_operands_only
 
 
-def b_tile_for(tile: TileConfig, src_b: Tensor, K: int, N: int, prologue: bool = False) -> TileConfig:
+def b_tile_for(tile: TileConfig, src_b: Tensor) -> TileConfig:
     """Row pitch of the B tile in LDS.  A B operand read 128-bit along
     columns is committed with 128-bit stores and keeps a pitch that is a
     multiple of 4 floats.  Any other B (a transposed view such as K^T, or
     odd strides) is committed by 32-bit stores walking down columns, where a
     pitch of tile_N + 4 puts rows 0, 4, 8, ... of a column on colliding
     banks; an odd pitch (tile_N + 3) spreads them (measured on MI355X for
-    the attention S = Q @ K^T kernel: 372.8 -> 360.5 us).  ``prologue``: B has
-    one, so odd sizes go element by element."""
-    if src_b.col_stride == 1 and (not prologue or (src_b.row_stride % 4 == 0 and N % 4 == 0)):
+    the attention S = Q @ K^T kernel: 372.8 -> 360.5 us)."""
+    if src_b.col_stride == 1:
         return tile
     return dataclasses.replace(tile, b_pad=3)
 
@@ -458,6 +449,14 @@ def exact_retry(config: MatmulConfig, src_a: Tensor, src_b: Tensor, pro_a: Chain
 
     return MatmulExactRetryFragment(config, a=operand(src_a, pro_a), b=operand(src_b, pro_b),
                                     accumulator_suffix=suffix, persistent=persistent)
+
+
+# A 256x256 tile with bounds stores its 256 KiB after a short k loop with no
+# other workgroup on the unit to work meanwhile; two 256x128 ones overlap.
+# Measured on MI355X: 17872 x 64 x 1117 47.6 -> 39.0 us, 4000 x 333 x 7001 232.8 ->
+# 198.9 us; 2049 x 1111 x 3333 and longer k's are as fast or faster on 256x256.
+SHORT_K = 512
+SHORT_K_TILE = TileConfig(256, 128, 32, 4, 2)
 
 
 def rr_local(M: int, N: int, tile: TileConfig, batch: int = 1) -> bool:
@@ -528,12 +527,14 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
 
     full_gather = gathers_full_operands(pro_a) or gathers_full_operands(pro_b)
     wide = WIDE_TILES and (not full_gather or WIDE_GATHER_TILES)
-    tile = b_tile_for(select_tile_config(M, K, N, batch=batch, wide=wide), src_b, K, N, pro_b is not None)
+    tile = b_tile_for(select_tile_config(M, K, N, batch=batch, wide=wide), src_b)
     aligned = is_aligned_shape(M, K, N, tile)
     if tile.num_threads > 512 and not aligned:
         # 16-wave tiles only without bounds checks (their masks cost registers)
-        tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b, K, N, pro_b is not None)
+        tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b)
         aligned = is_aligned_shape(M, K, N, tile)
+    if not aligned and K <= SHORT_K and (tile.tile_M, tile.tile_N) == (256, 256) and _config.FORCE_TILE is None:
+        tile = b_tile_for(SHORT_K_TILE, src_b)
     if decision.reduction is not None and (tile.tile_N, tile.sg_M, tile.sg_N) == (256, 4, 4):
         # each wave reduces its rows over its own columns: 2x8 waves leave
         # half as many rows to every wave's lane exchanges
@@ -551,7 +552,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
             registers=not aligned or direct.a_layout == "pad" or direct.b_layout == "pad",
             min_waves=4 if prologues else 1,
         )
-        tile = b_tile_for(tile, src_b, K, N, pro_b is not None)
+        tile = b_tile_for(tile, src_b)
         aligned = is_aligned_shape(M, K, N, tile)
 
     tile = dma_layouts(tile, (src_a,), (src_b,), (pro_a,), (pro_b,), aligned)

@@ -72,7 +72,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
     if filled:
         prologues = any((*pro_a, *pro_b))
         tile, parts = select_filled(M, K0, N, batch, min_waves=4 if prologues else 1, anchors=2)
-    padded = [b_tile_for(tile, src_b[i], (K0, K1)[i], N, bool(pro_b[i])) for i in range(2)]
+    padded = [b_tile_for(tile, src_b[i]) for i in range(2)]
     if all(p.b_pad != tile.b_pad for p in padded):
         tile = padded[0]  # both B tiles committed by 32-bit stores
     aligned = is_aligned_shape(M, K0, N, tile) and is_aligned_shape(M, K1, N, tile)

@@ -112,3 +112,35 @@ def test_pair_sharing_a(parts, monkeypatch):
     assert np.array_equal(z, h1 * h2) and np.array_equal(z, again)
     ref = (x.astype(np.float64) @ w1) * (x.astype(np.float64) @ w2)
     np.testing.assert_allclose(z, ref, rtol=1e-4, atol=1e-2)
+
+
+@pytest.mark.parametrize("a_view", [False, True])
+@pytest.mark.parametrize("kind", ["recip", "none", "row", "col"])
+def test_odd_prologues(kind, a_view):
+    """Bounds inside a 128-bit slot: nothing outside the matrix is loaded for a
+    prologue's operands or reaches the product (1 / 0 would)."""
+    rng = np.random.default_rng(19)
+    for M, K, N in ((201, 131, 77), (67, 258, 130), (130, 1030, 35)):
+        print(f"odd prologue {kind} {(M, K, N)} a_view={a_view}", flush=True)
+        a = (rng.random((M, K)) + 0.5).astype(np.float32)
+        b = rng.standard_normal((K, N)).astype(np.float32)
+        ops = Operations()
+        ops.from_numpy(np.ascontiguousarray(a.T) if a_view else a, "A")
+        ops.from_numpy(b, "B")
+        left, ref_a = "A", a.astype(np.float64)
+        if a_view:
+            ops.transpose("A", out="At")
+            left = "At"
+        if kind == "recip":
+            ops.elementwise("recip", out="P", operands=(left,))
+            ref_a = 1.0 / ref_a
+        else:
+            v = (rng.random({"none": (M, K), "row": (1, K), "col": (M, 1)}[kind]) + 0.5).astype(np.float32)
+            ops.from_numpy(v, "v")
+            ops.elementwise("div", out="P", operands=(left, "v"), y_broadcast=kind)
+            ref_a = ref_a / v
+        ops.matmul(a="P", b="B", out="C")
+        got = run(ops).env["C"]
+        ref = ref_a @ b.astype(np.float64)
+        # the quotients are within 2 ulp, the sum as above
+        assert np.all(np.abs(got - ref) <= (K + 12) * 2.0**-24 * (np.abs(ref_a) @ np.abs(b.astype(np.float64))))
