@@ -11,8 +11,11 @@ transposed views and other irregular strides.  Two forms:
 * ``transpose`` -- a column-major source (row stride 1, column stride
   ``ld``), i.e. a transposed view: tiles staged through LDS, read along the
   source's contiguous axis and written along the output's, both coalesced;
-  128-bit nontemporal loads and device-scope stores when the sizes and
-  ``ld`` are multiples of 4, one element per lane otherwise.  Measured on
+  128-bit nontemporal loads and device-scope stores: aligned when the sizes
+  and ``ld`` are multiples of 4, at any element address otherwise (4099x3001
+  35.6 -> 22.4 us, 14110x1024 40 -> 24.7 us against one element per lane;
+  ordinary loads and stores 24.0 and 29.6 us), one element per lane for small
+  odd ones.  Measured on
   MI355X, a transposed 4096x4096 view (64 MiB each way): 79.3 us with one
   lane per output element gathering through the strides, 35.1 us with
   scalar 64x64 tiles, 28.7 us with 128-bit 64x64 tiles and ordinary loads
@@ -46,6 +49,9 @@ TRANSPOSE_PAD = 1  # LDS row padding: column reads hit distinct banks
 # Streaming cache policy of the 128-bit form: nontemporal loads and
 # device-scope stores (written through L2), as the flat elementwise streams.
 TRANSPOSE_STREAMING = True
+# Odd sizes take the 128-bit form (unaligned, bounds per group) from this many
+# elements on; fewer are a few workgroups of one element per lane, all launch.
+TRANSPOSE_VECTOR_MIN = 1 << 16
 
 
 def transpose_lds_shape(ti: int = 0, tj: int = 0) -> tuple[int, int]:
@@ -108,36 +114,51 @@ class StridedCopyFragment:
             f"// source (i, j) at [i + j * {ld}]: tile i0..i0+{ti} x j0..j0+{tj}, staged as copy_tile[j][i]",
             f"const unsigned i0 = blockIdx.y * {ti}u, j0 = blockIdx.x * {tj}u;",
         ]
-        if rows % 4 == 0 and cols % 4 == 0 and ld % 4 == 0:
-            # 128-bit loads of 4 consecutive i and stores of 4 consecutive j
-            # (a 4-float group is wholly inside or outside the matrix); the
-            # transposed LDS reads (odd pitch) stay on distinct banks
-            qi, qj = ti // 4, tj // 4
-            if lanes % qi or lanes % qj or tj % (lanes // qi) or ti % (lanes // qj):
-                raise ValueError(f"transpose tile {ti}x{tj} does not split over {lanes} lanes")
+        aligned = rows % 4 == 0 and cols % 4 == 0 and ld % 4 == 0
+        if not aligned and rows * cols < TRANSPOSE_VECTOR_MIN:
+            return self._render_scalar_tiles(head, lanes)
+        # 128-bit loads of 4 consecutive i and stores of 4 consecutive j; the
+        # transposed LDS reads (odd pitch) stay on distinct banks
+        qi, qj = ti // 4, tj // 4
+        if lanes % qi or lanes % qj or tj % (lanes // qi) or ti % (lanes // qj):
+            raise ValueError(f"transpose tile {ti}x{tj} does not split over {lanes} lanes")
+        src = f"{self.input_name} + (size_t)(j0 + jj) * {ld}u + i0 + li"
+        dst = f"{self.output_name} + (size_t)(i0 + ii) * {cols}u + j0 + sj"
+        if aligned:
+            # a 4-float group is wholly inside or outside the matrix
             ld4, st4 = ("mt_ld4_nt", "mt_st4_wt") if self.streaming else ("mt_ld4", "mt_st4")
-            return "\n".join(
-                [
-                    *head,
-                    f"const unsigned li = 4u * (threadIdx.x % {qi}u), lj = threadIdx.x / {qi}u;",
-                    "#pragma unroll",
-                    f"for (unsigned jj = lj; jj < {tj}u; jj += {lanes // qi}u) {{",
-                    f"    const bool in = i0 + li < {rows}u && j0 + jj < {cols}u;",
-                    f"    const mt_f32x4 v = in ? {ld4}("
-                    f"{self.input_name} + (size_t)(j0 + jj) * {ld}u + i0 + li) : mt_f32x4{{0.f, 0.f, 0.f, 0.f}};",
-                    "    copy_tile[jj][li] = v.x; copy_tile[jj][li + 1u] = v.y;",
-                    "    copy_tile[jj][li + 2u] = v.z; copy_tile[jj][li + 3u] = v.w;",
-                    "}",
-                    "__syncthreads();",
-                    f"const unsigned sj = 4u * (threadIdx.x % {qj}u), si = threadIdx.x / {qj}u;",
-                    "#pragma unroll",
-                    f"for (unsigned ii = si; ii < {ti}u; ii += {lanes // qj}u) {{",
-                    f"    if (i0 + ii < {rows}u && j0 + sj < {cols}u)",
-                    f"        {st4}({self.output_name} + (size_t)(i0 + ii) * {cols}u + j0 + sj, mt_f32x4{{",
-                    "            copy_tile[sj][ii], copy_tile[sj + 1u][ii], copy_tile[sj + 2u][ii], copy_tile[sj + 3u][ii]});",
-                    "}",
-                ]
-            ) + f"\n// LDS rows padded to {ti + p} floats"
+            load, store = f"{ld4}({src})", f"{st4}({dst}, o)"
+        else:
+            # any element address, and bounds inside a group
+            stream = "true" if self.streaming else "false"
+            load = f"mt_ld_slot<{stream}>({src}, {rows}u - i0 - li)"
+            store = f"mt_st_slot<{stream}>({dst}, o, {cols}u - j0 - sj)"
+        return "\n".join(
+            [
+                *head,
+                f"const unsigned li = 4u * (threadIdx.x % {qi}u), lj = threadIdx.x / {qi}u;",
+                "#pragma unroll",
+                f"for (unsigned jj = lj; jj < {tj}u; jj += {lanes // qi}u) {{",
+                f"    const bool in = i0 + li < {rows}u && j0 + jj < {cols}u;",
+                f"    const mt_f32x4 v = in ? {load} : mt_f32x4{{0.f, 0.f, 0.f, 0.f}};",
+                "    copy_tile[jj][li] = v.x; copy_tile[jj][li + 1u] = v.y;",
+                "    copy_tile[jj][li + 2u] = v.z; copy_tile[jj][li + 3u] = v.w;",
+                "}",
+                "__syncthreads();",
+                f"const unsigned sj = 4u * (threadIdx.x % {qj}u), si = threadIdx.x / {qj}u;",
+                "#pragma unroll",
+                f"for (unsigned ii = si; ii < {ti}u; ii += {lanes // qj}u) {{",
+                f"    if (i0 + ii < {rows}u && j0 + sj < {cols}u) {{",
+                "        const mt_f32x4 o = {copy_tile[sj][ii], copy_tile[sj + 1u][ii], copy_tile[sj + 2u][ii], copy_tile[sj + 3u][ii]};",
+                f"        {store};",
+                "    }",
+                "}",
+            ]
+        ) + f"\n// LDS rows padded to {ti + p} floats"
+
+    def _render_scalar_tiles(self, head: list[str], lanes: int) -> str:
+        ti, tj, p = self.tile_i, self.tile_j, TRANSPOSE_PAD
+        rows, cols, ld = self.input_rows, self.input_cols, self.input_col_stride
         if lanes % ti or lanes % tj or tj % (lanes // ti) or ti % (lanes // tj):
             raise ValueError(f"transpose tile {ti}x{tj} does not split over {lanes} lanes")
         return "\n".join(

@@ -235,6 +235,108 @@ class LastAxisReductionComputeFragment:
         return "\n".join(L)
 
 
+STRIDED_ROWS = 32  # rows of a workgroup: 128 contiguous bytes per load and 32 lanes
+STRIDED_LANES = 512
+STRIDED_GROUPS = STRIDED_LANES // STRIDED_ROWS  # lanes that share a row
+STRIDED_LOADS = 16  # elements in flight per lane
+
+
+@dataclass(frozen=True)
+class StridedReductionFragment(LastAxisReductionComputeFragment):
+    """The same reduction of rows that are contiguous across each other (row
+    stride 1: the columns of a row-major matrix, e.g. a bias gradient), in the
+    same order.  One wave per row would load one element per cache line; here a
+    workgroup takes STRIDED_ROWS rows, 32 lanes load one element of each at a
+    time, and lane group G keeps the partial values of lanes t = J G .. J G + J - 1
+    of the wave-per-row order (J = T / 16).  They meet in LDS, where one lane per
+    row folds them along the butterfly's tree.  Measured on MI355X, 4096 rows of
+    2048: 47.3 us with a wave per row.  Includes the store (``out_name``,
+    ``epilogue``)."""
+
+    rows_dim: str = "M"
+    out_name: str = ""
+    epilogue: ValueTransform | None = None
+    kind: str = "compute"
+
+    @property
+    def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
+        shape = strided_scratch_shape(self.W)
+        return (TgmemAccess(self.scratch_name, "readwrite", shape[0] * shape[1], shape),)
+
+    def render(self, ctx: CodegenContext) -> str:
+        _check_op(self.op)
+        W, R = self.W, STRIDED_ROWS
+        T = 64 * W
+        J = T // STRIDED_GROUPS
+        U = max(1, STRIDED_LOADS // J)  # chunks of T elements in flight
+        ident = _identity(self.op)
+        tf = self.value_transform or (lambda raw: raw)
+        ep = self.epilogue or (lambda raw: raw)
+        sc = self.scratch_name
+        at = f"src[(size_t)idx * {_uint(self.col_stride)}]"
+        lines = [
+            f"const unsigned mt_r = threadIdx.x % {R}u, mt_g = threadIdx.x / {R}u;",
+            f"const unsigned row = blockIdx.x * {R}u + mt_r;",
+            f"const bool row_ok = row < {self.rows_dim};",
+            f"float mt_acc[{J}];",
+            "#pragma unroll",
+            f"for (int j = 0; j < {J}; ++j) mt_acc[j] = {ident};",
+            "if (row_ok) {",
+            f"    const float* __restrict__ src = {self.input_name} + row;",
+            f"    unsigned e = mt_g * {J}u;  // this lane's first element of the chunk",
+            f"    for (; e + {(U - 1) * T + J - 1}u < {self.reduce_dim}; e += {U * T}u) {{",
+            f"        float x[{U}][{J}];",
+            "#pragma unroll",
+            f"        for (int u = 0; u < {U}; ++u)",
+            "#pragma unroll",
+            f"            for (int j = 0; j < {J}; ++j) {{",
+            f"                const unsigned idx = e + (unsigned)(u * {T} + j);",
+            f"                x[u][j] = {at};",
+            "            }",
+            "#pragma unroll",
+            f"        for (int u = 0; u < {U}; ++u)",
+            "#pragma unroll",
+            f"            for (int j = 0; j < {J}; ++j) {{",
+            f"                const unsigned idx = e + (unsigned)(u * {T} + j);",
+            "                (void)idx;",
+            f"                mt_acc[j] = {_combine(self.op, 'mt_acc[j]', tf('x[u][j]'))};",
+            "            }",
+            "    }",
+            f"    for (; e < {self.reduce_dim}; e += {T}u)",
+            "#pragma unroll",
+            f"        for (int j = 0; j < {J}; ++j) {{",
+            "            const unsigned idx = e + (unsigned)j;",
+            f"            if (idx < {self.reduce_dim}) {{",
+            f"                const float xv = {at};",
+            f"                mt_acc[j] = {_combine(self.op, 'mt_acc[j]', tf('xv'))};",
+            "            }",
+            "        }",
+            "}",
+            "#pragma unroll",
+            f"for (int j = 0; j < {J}; ++j) {sc}[mt_g * {J}u + (unsigned)j][mt_r] = mt_acc[j];",
+            "__syncthreads();",
+            f"if (threadIdx.x < {R}u && row_ok) {{",
+            "    float r = 0.0f;",
+            f"    for (unsigned w = 0; w < {W}u; ++w) {{  // a wave's 64 lanes, then the waves left to right",
+            "        float mt_v[64];",
+            "#pragma unroll",
+            f"        for (int t = 0; t < 64; ++t) mt_v[t] = {sc}[64u * w + (unsigned)t][mt_r];",
+            "#pragma unroll",
+            "        for (int off = 32; off > 0; off >>= 1)",
+            "#pragma unroll",
+            f"            for (int t = 0; t < off; ++t) mt_v[t] = {_combine(self.op, 'mt_v[t]', 'mt_v[t + off]')};",
+            f"        r = w == 0u ? mt_v[0] : {_combine(self.op, 'r', 'mt_v[0]')};",
+            "    }",
+            f"    {self.out_name}[row] = {ep('r')};",
+            "}",
+        ]
+        return "\n".join(lines)
+
+
+def strided_scratch_shape(waves_per_row: int) -> tuple[int, int]:
+    return (64 * waves_per_row, STRIDED_ROWS)
+
+
 @dataclass(frozen=True)
 class StoreReductionResultFragment:
     """Lane 0 of the row's first wave stores ``r`` (optionally transformed)."""

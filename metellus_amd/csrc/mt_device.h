@@ -195,12 +195,27 @@ __host__ __device__ __forceinline__ constexpr bool mt_in_part(int i, int n, int 
 // Four consecutive elements from p, of which the first `left` (at least one)
 // are inside the matrix: one 128-bit load at any element address, or element by
 // element at its edge (0 outside).
+template <bool NT = false>
 MT_INLINE mt_f32x4 mt_ld_slot(const float* p, unsigned left) {
-    if (left >= 4u) return mt_ld4u(p);
+    if (left >= 4u) return NT ? mt_ld4u_nt(p) : mt_ld4u(p);
     mt_f32x4 x = {p[0], 0.f, 0.f, 0.f};
     if (left > 1u) x.y = p[1];
     if (left > 2u) x.z = p[2];
     return x;
+}
+// The first `left` of four consecutive elements to p (any element address).
+template <bool WT = false>
+MT_INLINE void mt_st_slot(float* p, mt_f32x4 v, unsigned left) {
+    if (left >= 4u) {
+        if (WT)
+            mt_st4_wt(p, v);
+        else
+            *reinterpret_cast<mt_f32x4u*>(p) = v;
+        return;
+    }
+    p[0] = v.x;
+    if (left > 1u) p[1] = v.y;
+    if (left > 2u) p[2] = v.z;
 }
 // The slot's elements outside the matrix are 0 again after a transform.
 MT_INLINE void mt_clear_slot(mt_f32x4& x, unsigned left) {

@@ -14,7 +14,9 @@ from metellus_amd.compute.reduction.reduction import (
     LastAxisReductionComputeFragment,
     LastAxisReductionSetupFragment,
     StoreReductionResultFragment,
+    StridedReductionFragment,
     scratch_floats,
+    strided_scratch_shape,
 )
 from metellus_amd.orchestrator.assembly.decision import DecisionView
 from metellus_amd.orchestrator.assembly.expressions import (
@@ -41,6 +43,52 @@ def reduction_waves_per_row(M: int, K: int) -> int:
     return W
 
 
+def strided_rows(src: Tensor) -> bool:
+    """Rows lying side by side in memory (the columns of a row-major matrix), at
+    least a workgroup of them and a wave's 64 elements each: 32 lanes then load
+    128 contiguous bytes where a wave per row loads 64 cache lines."""
+    M, K = src.shape
+    return src.row_stride == 1 and src.col_stride != 1 and M >= _red.STRIDED_ROWS and K >= 64
+
+
+def _assemble_strided(decision: DecisionView, function_name: str | None, src: Tensor, final_out: Tensor,
+                      extras: Extras, helpers: list[str], prologue, epilogue, M: int, K: int, W: int) -> KernelGroup:
+    anchor = decision.anchor
+    frag = StridedReductionFragment(
+        op=anchor.op,
+        input_name=param_name(src.buffer_key),
+        scratch_name="scratch",
+        reduce_dim="K",
+        row_stride=str(src.row_stride),
+        col_stride=str(src.col_stride),
+        name="reduction_compute",
+        tg_x=_red.STRIDED_LANES,
+        value_transform=prologue,
+        waves_per_row=W,
+        vectorized=False,
+        out_name=param_name(final_out.buffer_key),
+        epilogue=epilogue,
+    )
+    ctx = CodegenContext(
+        function_name=function_name or f"reduce_{anchor.out.name}_fused",
+        buffers=(input_param(src.buffer_key), output_param(final_out.buffer_key), *extras.buffers),
+        dims=("M", "K"),
+        tg_x=_red.STRIDED_LANES,
+        tg_y=1,
+        threadgroup_decls=(lds_decl("scratch", strided_scratch_shape(W)),),
+        helpers=tuple(helpers),
+    )
+    return KernelGroup(
+        kernel=Kernel(fragments=(frag,), ctx=ctx),
+        bindings=(src.buffer_key, final_out.buffer_key, *extras.bindings),
+        dims=(M, K),
+        grid=((M + _red.STRIDED_ROWS - 1) // _red.STRIDED_ROWS, 1, 1),
+        threads=(_red.STRIDED_LANES, 1, 1),
+        ops=decision.ops,
+        strategy=decision.strategy,
+    )
+
+
 def assemble_reduction(decision: DecisionView, function_name: str | None) -> KernelGroup:
     anchor = decision.anchor
     assert isinstance(anchor, ReductionOp)
@@ -62,6 +110,8 @@ def assemble_reduction(decision: DecisionView, function_name: str | None) -> Ker
         helpers.append(epilogue.helper)
 
     W = reduction_waves_per_row(M, K)
+    if strided_rows(src):
+        return _assemble_strided(decision, function_name, src, final_out, extras, helpers, prologue, epilogue, M, K, W)
     R = WG_LANES // (64 * W)
     vec = src.col_stride == 1 and K % 4 == 0 and src.row_stride % 4 == 0
     setup = LastAxisReductionSetupFragment(rows_dim="M", name="reduction_setup", waves_per_row=W, rows_per_group=R)
