@@ -130,6 +130,26 @@ int mt_compile_only(const char* source, const char* options, const char* target,
 int mt_launch(uint64_t kernel, const uint64_t* buffers, int nbuf, const uint32_t* dims, int ndims,
               int dims_slot, const uint32_t* grid, const uint32_t* block, int timed, float* ms);
 
+/* No counterpart in the reference, which crosses into its native module once
+ * per dispatch (reference: src/runtime/program.py:179-196).  Launch n kernels in
+ * order, untimed, in one call: each item is mt_launch's arguments, and
+ * workspace > 0 appends the mt_workspace buffer (grown to at least that many
+ * bytes) as the kernel's last parameter.  Stops at the first item that fails;
+ * the ones before it are queued. */
+typedef struct mt_launch_item {
+    uint64_t kernel;
+    const uint64_t* buffers;
+    const uint32_t* dims;
+    size_t workspace;
+    int nbuf;
+    int ndims;
+    int dims_slot;
+    uint32_t grid[3];
+    uint32_t block[3];
+} mt_launch_item;
+
+int mt_launch_many(const mt_launch_item* items, int n);
+
 /* Allocation-free variant of mt_launch.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory -- code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.

@@ -646,6 +646,73 @@ static int lookup(State& s, uint64_t handle, Buffer* out) {
     return 0;
 }
 
+// The argument checks and the launch shared by mt_launch and mt_launch_many;
+// ws: the workspace, appended as the last parameter (null: none).
+int launch_locked(State& s, uint64_t kernel, const uint64_t* buffers, int nbuf, const uint32_t* dims, int ndims,
+                  int dims_slot, const uint32_t* grid, const uint32_t* block, void* ws) {
+    if (ndims < 0 || ndims > kMaxDims) return fail("mt_launch: at most 16 dims");
+    if (nbuf < 0 || dims_slot < 0 || dims_slot > nbuf) return fail("mt_launch: bad dims slot");
+    if (kernel == 0 || kernel > s.kernels.size()) return fail("mt_launch: unknown kernel handle");
+    for (int i = 0; i < 3; ++i) {
+        if (grid[i] == 0 || block[i] == 0) return fail("mt_launch: zero grid or block extent");
+    }
+    if (static_cast<uint64_t>(block[0]) * block[1] * block[2] > 1024)
+        return fail("mt_launch: more than 1024 lanes per workgroup");
+    void* few[kMaxLaunchBuffers];
+    std::vector<void*> many;
+    void** ptrs = few;
+    if (nbuf > kMaxLaunchBuffers) {
+        many.resize(static_cast<size_t>(nbuf));
+        ptrs = many.data();
+    }
+    for (int i = 0; i < nbuf; ++i) {
+        Buffer b;
+        if (lookup(s, buffers[i], &b)) return 1;
+        ptrs[i] = b.ptr;
+    }
+    DimsArg d{};
+    for (int i = 0; i < ndims; ++i) d.v[i] = dims[i];
+    void* few_params[kMaxLaunchBuffers + 2];
+    std::vector<void*> many_params;
+    void** params = few_params;
+    if (nbuf > kMaxLaunchBuffers) {
+        many_params.resize(static_cast<size_t>(nbuf) + 2);
+        params = many_params.data();
+    }
+    int np = 0;
+    for (int i = 0; i <= nbuf; ++i) {
+        if (i == dims_slot) params[np++] = &d;
+        if (i < nbuf) params[np++] = &ptrs[i];
+    }
+    if (ws) params[np++] = &ws;
+    const Kernel& k = s.kernels[kernel - 1];
+    MT_HIP(hipModuleLaunchKernel(k.function, grid[0], grid[1], grid[2], block[0], block[1], block[2], 0, s.stream,
+                                 params, nullptr));
+    return 0;
+}
+
+// The workspace, at least nbytes of it (see mt_workspace).
+int workspace_locked(State& s, size_t nbytes, void** ptr) {
+    if (nbytes > s.ws_bytes) {
+        if (s.ws_handle) {
+            // Stream-ordered: kernels already queued on the old one finish first.
+            MT_HIP(hipFreeAsync(s.buffers[s.ws_handle].ptr, s.stream));
+            s.buffers.erase(s.ws_handle);
+            s.ws_handle = 0;
+            s.ws_bytes = 0;
+        }
+        void* p = nullptr;
+        MT_HIP(hipMallocAsync(&p, nbytes, s.stream));
+        ++s.device_allocs;
+        MT_HIP(hipMemsetAsync(p, 0, kWsHeadBytes, s.stream));  // flags and error word start at 0
+        s.ws_handle = s.next_buffer++;
+        s.buffers.emplace(s.ws_handle, Buffer{p, nbytes, nbytes});
+        s.ws_bytes = nbytes;
+    }
+    if (ptr) *ptr = s.buffers[s.ws_handle].ptr;
+    return 0;
+}
+
 int mt_size(uint64_t handle, size_t* nbytes) {
     State& s = state();
     std::lock_guard<std::mutex> lock(s.mu);
@@ -801,41 +868,32 @@ int mt_compile(const char* source, const char* function_name, const char* option
 int mt_launch(uint64_t kernel, const uint64_t* buffers, int nbuf, const uint32_t* dims, int ndims,
               int dims_slot, const uint32_t* grid, const uint32_t* block, int timed, float* ms) {
     if (!grid || !block) return fail("mt_launch: grid and block are required");
-    if (ndims < 0 || ndims > kMaxDims) return fail("mt_launch: at most 16 dims");
-    if (nbuf < 0 || dims_slot < 0 || dims_slot > nbuf) return fail("mt_launch: bad dims slot");
     State& s = state();
     std::lock_guard<std::mutex> lock(s.mu);
     if (init_locked(s)) return 1;
-    if (kernel == 0 || kernel > s.kernels.size()) return fail("mt_launch: unknown kernel handle");
-    for (int i = 0; i < 3; ++i) {
-        if (grid[i] == 0 || block[i] == 0) return fail("mt_launch: zero grid or block extent");
-    }
-    if (static_cast<uint64_t>(block[0]) * block[1] * block[2] > 1024)
-        return fail("mt_launch: more than 1024 lanes per workgroup");
-    std::vector<void*> ptrs(static_cast<size_t>(nbuf));
-    for (int i = 0; i < nbuf; ++i) {
-        Buffer b;
-        if (lookup(s, buffers[i], &b)) return 1;
-        ptrs[i] = b.ptr;
-    }
-    DimsArg d{};
-    for (int i = 0; i < ndims; ++i) d.v[i] = dims[i];
-    std::vector<void*> params;
-    params.reserve(static_cast<size_t>(nbuf) + 1);
-    for (int i = 0; i <= nbuf; ++i) {
-        if (i == dims_slot) params.push_back(&d);
-        if (i < nbuf) params.push_back(&ptrs[i]);
-    }
-    const Kernel& k = s.kernels[kernel - 1];
     if (timed) MT_HIP(hipEventRecord(s.ev_start, s.stream));
-    MT_HIP(hipModuleLaunchKernel(k.function, grid[0], grid[1], grid[2], block[0], block[1], block[2], 0,
-                                 s.stream, params.data(), nullptr));
+    if (launch_locked(s, kernel, buffers, nbuf, dims, ndims, dims_slot, grid, block, nullptr)) return 1;
     if (timed) {
         MT_HIP(hipEventRecord(s.ev_stop, s.stream));
         MT_HIP(hipEventSynchronize(s.ev_stop));
         float t = 0.f;
         MT_HIP(hipEventElapsedTime(&t, s.ev_start, s.ev_stop));
         if (ms) *ms = t;
+    }
+    return 0;
+}
+
+int mt_launch_many(const mt_launch_item* items, int n) {
+    if (n < 0 || (n > 0 && !items)) return fail("mt_launch_many: bad items");
+    State& s = state();
+    std::lock_guard<std::mutex> lock(s.mu);
+    if (init_locked(s)) return 1;
+    for (int i = 0; i < n; ++i) {
+        const mt_launch_item& it = items[i];
+        void* ws = nullptr;
+        if (it.workspace != 0 && workspace_locked(s, it.workspace, &ws)) return 1;
+        if (launch_locked(s, it.kernel, it.buffers, it.nbuf, it.dims, it.ndims, it.dims_slot, it.grid, it.block, ws))
+            return 1;
     }
     return 0;
 }
@@ -906,22 +964,7 @@ int mt_workspace(size_t nbytes, uint64_t* handle) {
     State& s = state();
     std::lock_guard<std::mutex> lock(s.mu);
     if (init_locked(s)) return 1;
-    if (nbytes > s.ws_bytes) {
-        if (s.ws_handle) {
-            // Stream-ordered: kernels already queued on the old one finish first.
-            MT_HIP(hipFreeAsync(s.buffers[s.ws_handle].ptr, s.stream));
-            s.buffers.erase(s.ws_handle);
-            s.ws_handle = 0;
-            s.ws_bytes = 0;
-        }
-        void* p = nullptr;
-        MT_HIP(hipMallocAsync(&p, nbytes, s.stream));
-        ++s.device_allocs;
-        MT_HIP(hipMemsetAsync(p, 0, kWsHeadBytes, s.stream));  // flags and error word start at 0
-        s.ws_handle = s.next_buffer++;
-        s.buffers.emplace(s.ws_handle, Buffer{p, nbytes, nbytes});
-        s.ws_bytes = nbytes;
-    }
+    if (workspace_locked(s, nbytes, nullptr)) return 1;
     *handle = s.ws_handle;
     return 0;
 }

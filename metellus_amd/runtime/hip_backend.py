@@ -48,6 +48,7 @@ EXPORTED_SYMBOLS = (
     "mt_compile",
     "mt_compile_only",
     "mt_launch",
+    "mt_launch_many",
     "mt_launch_noalloc",
     "mt_mark",
     "mt_mark_elapsed",
@@ -62,6 +63,22 @@ _lock = threading.Lock()
 
 _u64 = ctypes.c_uint64
 _u32p = ctypes.POINTER(ctypes.c_uint32)
+
+
+class LaunchItem(ctypes.Structure):
+    """``mt_launch_item``."""
+
+    _fields_ = [
+        ("kernel", _u64),
+        ("buffers", ctypes.POINTER(_u64)),
+        ("dims", _u32p),
+        ("workspace", ctypes.c_size_t),
+        ("nbuf", ctypes.c_int),
+        ("ndims", ctypes.c_int),
+        ("dims_slot", ctypes.c_int),
+        ("grid", ctypes.c_uint32 * 3),
+        ("block", ctypes.c_uint32 * 3),
+    ]
 
 
 def library_path() -> str:
@@ -118,6 +135,7 @@ def _load():
                  ctypes.c_int, ctypes.POINTER(ctypes.c_float)],
                 ctypes.c_int,
             ),
+            "mt_launch_many": ([ctypes.POINTER(LaunchItem), ctypes.c_int], ctypes.c_int),
             "mt_launch_noalloc": (
                 [_u64, ctypes.POINTER(_u64), ctypes.c_int, _u32p, ctypes.c_int, ctypes.c_int, _u32p, _u32p,
                  ctypes.c_size_t, _u32p],
@@ -361,6 +379,44 @@ def launch(
         )
     )
     return float(ms.value) if timed else None
+
+
+class LaunchSequence:
+    """Untimed launches issued back to back by one native call.  ``launches``:
+    (kernel, number of buffers, dims, dims_slot, grid, threads, workspace) each;
+    everything but the buffers is laid out once.  Threads may share one."""
+
+    def __init__(self, launches) -> None:
+        total = sum(nb for _, nb, *_ in launches)
+        self._handles = (_u64 * max(total, 1))()
+        self._items = (LaunchItem * max(len(launches), 1))()
+        self._count = len(launches)
+        self._keep = []
+        self._lock = threading.Lock()  # the handle array is filled per call
+        at = 0
+        for item, (kernel, nb, dims, slot, grid, threads, workspace) in zip(self._items, launches):
+            dims_l = [int(d) for d in dims]
+            for d in dims_l:
+                if not 0 <= d < 2**32:
+                    raise ValueError(f"dim value {d} does not fit in uint32")
+            dims_a = (ctypes.c_uint32 * max(len(dims_l), 1))(*dims_l)
+            self._keep.append(dims_a)
+            item.kernel, item.workspace = kernel, workspace
+            item.buffers = ctypes.cast(ctypes.byref(self._handles, at * 8), ctypes.POINTER(_u64))
+            item.dims = ctypes.cast(dims_a, _u32p)
+            item.nbuf, item.ndims, item.dims_slot = nb, len(dims_l), int(slot)
+            item.grid[:] = [int(g) for g in grid]
+            item.block[:] = [int(t) for t in threads]
+            at += nb
+        self._launch = _load().mt_launch_many
+
+    def launch(self, buffers) -> None:
+        """``buffers``: the launches' buffers (or handles), one after another."""
+        handles = [b.handle if hasattr(b, "handle") else _handle_of(b) for b in buffers]
+        with self._lock:
+            self._handles[: len(handles)] = handles
+            rc = self._launch(self._items, self._count)
+        _check(rc)
 
 
 def launch_noalloc(kernel: int, buffers, dims, dims_slot: int, grid, threads, scratch: int = 0,
