@@ -3,8 +3,8 @@
 Replaces the reference's Apple tile picker (reference:
 src/compute/matmul/config.py:40-51: 32x32x16 .. 128x64x32 tiles, four
 32-wide simdgroups).  Here a workgroup of ``sg_M x sg_N`` wave64s computes a
-``tile_M x tile_N`` output tile with fp32 MFMA (32x32 blocks); each wave owns
-a ``(tile_M/sg_M) x (tile_N/sg_N)`` sub-tile, i.e. ``WM x WN`` accumulator
+``tile_M x tile_N`` output tile with MFMAs (32x32 blocks); each wave owns a
+``(tile_M/sg_M) x (tile_N/sg_N)`` sub-tile, i.e. ``WM x WN`` accumulator
 blocks of 16 registers.  A and B k-chunks of ``tile_K`` are double-buffered
 in LDS: dense, XOR-swizzled tiles filled by direct-to-LDS loads, or rows
 padded by ``a_pad``/``b_pad`` floats when filled through registers (see

@@ -1047,7 +1047,7 @@ def skinny_workspace_bytes(tiles: int, row_blocks: int, splits: int) -> int:
 # each of the first four groups of its right half.  KR_STORE_POLICY is the
 # buffer stores' cache-policy operand (0: default; 16: sc1, device scope,
 # written through the L2).  Measured on C5 S (32 heads, medians of 25-30
-# launches, one box):
+# launches, one GPU):
 # stores after the chunk's MFMAs 263.4 us; one row per group of the other
 # half 255.1; spread over every other group of the left half 251.2; sc1
 # 246.7; the right half's stores in the first four groups 245.6 (0.889 of

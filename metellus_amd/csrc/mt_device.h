@@ -50,6 +50,7 @@
 // All indices are unsigned 32-bit except global offsets (size_t).
 
 typedef float mt_f32x4 __attribute__((ext_vector_type(4)));
+typedef float mt_f32x2 __attribute__((ext_vector_type(2)));
 typedef float mt_f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned mt_u32x4 __attribute__((ext_vector_type(4)));
 
@@ -344,7 +345,29 @@ struct mt_tile_rowvec {
     static constexpr int RV = ROWS / 4;
     static constexpr int TOTAL = RV * COLS;
     static constexpr int PER = (TOTAL + NT - 1) / NT;
+    // Tall tiles (an A operand) give each lane KB neighbouring columns of its
+    // four rows, which leave as one store per row; eight lanes read a 128-byte
+    // line and the next eight the next KB columns.  Single stores met in a bank
+    // eight at a time: 1024 x 2048 x 4096 with X^T 182 -> 152 us on MI355X.
+    static constexpr int KB = RV % 8 != 0 || ROWS <= COLS || TOTAL % NT != 0 ? 1
+                              : PER % 4 == 0 && COLS % 4 == 0                ? 4
+                              : PER % 2 == 0 && COLS % 2 == 0                ? 2
+                                                                             : 1;
     mt_f32x4 v[PER];
+
+    // The tile's column (in c) and first row of slot i.
+    static MT_INLINE unsigned slot(unsigned tid, int i, unsigned& c) {
+        if constexpr (KB == 1) {
+            const unsigned idx = tid + i * NT;
+            c = idx / RV;
+            return (idx % RV) * 4u;
+        } else {
+            constexpr unsigned KQ = COLS / KB;
+            const unsigned b = tid + (i / KB) * NT;
+            c = (b / 8u) % KQ * KB + (unsigned)(i % KB);
+            return (b / (8u * KQ) * 8u + b % 8u) * 4u;
+        }
+    }
 
     template <bool CHECK, typename F>
     MT_INLINE void fetch(const float* __restrict__ src, unsigned cs, unsigned row0, unsigned col0,
@@ -353,7 +376,8 @@ struct mt_tile_rowvec {
         for (int i = 0; i < PER; ++i) {
             if (!mt_in_part(i, PER, q, Q)) continue;
             const unsigned idx = tid + i * NT;
-            const unsigned c = idx / RV, r = (idx % RV) * 4u;
+            unsigned c;
+            const unsigned r = slot(tid, i, c);
             const unsigned gr = row0 + r, gc = col0 + c;
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rlim && gc < clim))) {
@@ -370,11 +394,29 @@ struct mt_tile_rowvec {
 
     template <int LD>
     MT_INLINE void commit(float* lds, unsigned tid) const {
+        if constexpr (KB > 1 && LD % KB == 0) {
+#pragma unroll
+            for (int i = 0; i < PER; i += KB) {
+                unsigned c;
+                float* at = lds + slot(tid, i, c) * LD;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (KB == 4) {
+                        *reinterpret_cast<mt_f32x4*>(at + j * LD + c) =
+                            mt_f32x4{v[i][j], v[i + 1][j], v[i + 2][j], v[i + 3][j]};
+                    } else {
+                        *reinterpret_cast<mt_f32x2*>(at + j * LD + c) = mt_f32x2{v[i][j], v[i + 1][j]};
+                    }
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const unsigned idx = tid + i * NT;
             if (TOTAL % NT == 0 || idx < (unsigned)TOTAL) {
-                const unsigned c = idx / RV, r = (idx % RV) * 4u;
+                unsigned c;
+            const unsigned r = slot(tid, i, c);
                 lds[(r + 0u) * LD + c] = v[i].x;
                 lds[(r + 1u) * LD + c] = v[i].y;
                 lds[(r + 2u) * LD + c] = v[i].z;
@@ -397,7 +439,8 @@ struct mt_tile_rowvec {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const unsigned idx = tid + i * NT;
-            const unsigned c = idx / RV, r = (idx % RV) * 4u;
+            unsigned c;
+            const unsigned r = slot(tid, i, c);
             const unsigned gr = r0 + r, gc = c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rl && gc < cl))) {
                 const unsigned left = CHECK ? rl - gr : 4u;
@@ -600,7 +643,8 @@ struct mt_tile_rowvec_g : mt_tile_rowvec<ROWS, COLS, NT> {
         for (int i = 0; i < PER; ++i) {
             if (!mt_in_part(i, PER, q, Q)) continue;
             const unsigned idx = tid + i * NT;
-            const unsigned c = idx / RV, r = (idx % RV) * 4u;
+            unsigned c;
+            const unsigned r = Base::slot(tid, i, c);
             const unsigned gr = row0 + r, gc = col0 + c;
             mt_f32x4 x = {0.f, 0.f, 0.f, 0.f};
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < rlim && gc < clim))) {
@@ -630,7 +674,8 @@ struct mt_tile_rowvec_g : mt_tile_rowvec<ROWS, COLS, NT> {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const unsigned idx = tid + i * NT;
-            const unsigned c = idx / RV, r = (idx % RV) * 4u;
+            unsigned c;
+            const unsigned r = Base::slot(tid, i, c);
             const unsigned gr = this->r0 + r, gc = this->c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < this->rl && gc < this->cl))) {
 #pragma unroll
@@ -658,7 +703,8 @@ struct mt_tile_rowvec_g : mt_tile_rowvec<ROWS, COLS, NT> {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const unsigned idx = tid + i * NT;
-            const unsigned c = idx / RV, r = (idx % RV) * 4u;
+            unsigned c;
+            const unsigned r = Base::slot(tid, i, c);
             const unsigned gr = this->r0 + r, gc = this->c0 + c;
             if ((TOTAL % NT == 0 || idx < (unsigned)TOTAL) && (!CHECK || (gr < this->rl && gc < this->cl))) {
                 this->v[i].x = a(this->v[i].x, ex[i][0]);
@@ -918,7 +964,7 @@ MT_INLINE void mt_mfma_tile_f32(const float* __restrict__ As, const float* __res
 // 1018 us (135 TFLOP/s) with fp32 MFMAs, 741 us (185 TFLOP/s) this way; the
 // matrix cores are then busy 63 % of the cycles and the clock has fallen from
 // 2.05 to 1.68 GHz (a plain bf16 GEMM of 8192^3 reaches 1.22 PFLOP/s on the
-// same box, six times 203 TFLOP/s: power, not the split, is the next limit).
+// same GPU, six times 203 TFLOP/s: power, not the split, is the next limit).
 // Error against 64 bits, relative 2-norm, fp32 MFMA -> split, N(0, 1) operands:
 // K = 64: 1.44e-7 -> 1.09e-7; 512: 4.1e-7 -> 3.4e-7; 1024: 5.8e-7 -> 4.9e-7;
 // 4096: 1.15e-6 -> 1.00e-6; 11008: 1.88e-6 -> 1.69e-6; all positive, 64:

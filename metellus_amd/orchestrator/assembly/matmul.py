@@ -400,7 +400,7 @@ def xcd_rows(grid: tuple[int, int, int]) -> int:
 # Single matmuls whose best-scored tile leaves compute units idle take
 # ``select_filled``'s tile and split.  Measured on MI355X, before -> after: 256^3
 # 23.5 -> 8.2 us, 512^3 43 -> 13 us, 1024^3 84 -> 24 us, 2048 x 4096 x 1024 with
-# W^T 320 -> 116 us, 1024 x 2048 x 4096 with X^T 217 -> 133 us, 128 x 4096 x 4096
+# W^T 320 -> 116 us, 1024 x 2048 x 4096 with X^T 312 -> 152 us, 128 x 4096 x 4096
 # 194 -> 42 us, 300 x 777 x 1000 47 -> 28 us.
 FILL = True
 FILL_MIN_K = 128  # fewer k-chunks are over before a smaller tile pays

@@ -144,3 +144,18 @@ def test_odd_prologues(kind, a_view):
         ref = ref_a @ b.astype(np.float64)
         # the quotients are within 2 ulp, the sum as above
         assert np.all(np.abs(got - ref) <= (K + 12) * 2.0**-24 * (np.abs(ref_a) @ np.abs(b.astype(np.float64))))
+
+
+@pytest.mark.parametrize("divisor", [False, True])
+@pytest.mark.parametrize("index", range(len(config.FILL_TILES)))
+def test_a_along_its_rows(index, divisor, monkeypatch):
+    """A transposed view of A: its loader stores 4, 2 or 1 columns of a row at a
+    time, by the tile and its lanes; whole and ragged rows and k's."""
+    tile = config.FILL_TILES[index].tile
+    monkeypatch.setattr(mm, "select_filled", lambda *a, **k: (tile, 1))
+    monkeypatch.setattr(mm, "fills", lambda *a, **k: False)
+    for shape in ((256, 256, 256), (300, 517, 259)):
+        print(f"filled A^T {shape} {tile.tile_M}x{tile.tile_N} divisor={divisor}", flush=True)
+        ops, ref, bound = _program(shape, a_view=True, divisor=divisor)
+        # the quotient rounds once more and its divisor's reciprocal twice
+        _check(ops, ref, bound + 4 * 2.0**-24 * bound / ((shape[1] + 8) * 2.0**-24))
