@@ -1123,9 +1123,11 @@ MT_INLINE void mt_mfma_tile_held(const float* __restrict__ As, const float* __re
 }
 
 // Whether the wave's accumulators may differ from the fp32 products' sums for
-// want of range: a NaN (every sum an infinite or NaN operand enters is one
-// here, where fp32 may give an infinity) or a nonzero result below 2^-96, which
-// takes operands small enough to have lost their lower parts.  Wave uniform.
+// want of range: a value that is not finite (every sum an infinite or NaN operand
+// enters is a NaN here, where fp32 may give an infinity; and a part of a product
+// may pass the largest float where the product does not, as x1 is rounded up) or a
+// nonzero result below 2^-96, which takes operands small enough to have lost their
+// lower parts.  Wave uniform.
 template <int WM, int WN>
 MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN]) {
     bool odd = false;
@@ -1135,8 +1137,8 @@ MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN]) {
         for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const float x = acc[i][j][v];
-                odd |= !(__builtin_fabsf(x) >= 0x1.0p-96f) && x != 0.0f;
+                const float x = __builtin_fabsf(acc[i][j][v]);
+                odd |= !(x >= 0x1.0p-96f && x <= 0x1.fffffep+127f) && x != 0.0f;
             }
     return __ballot(odd) != 0ull;
 }
