@@ -406,11 +406,13 @@ class ThreadIndexFragment:
 
 @dataclass(frozen=True)
 class MatmulSetupFragment:
-    """Zeroed accumulators ``acc{suffix}[WM][WN]``."""
+    """Zeroed accumulators ``acc{suffix}[WM][WN]``, and for a split mainloop what
+    its splits cut off (``mt_cut{suffix}``)."""
 
     config: MatmulConfig
     accumulator_suffix: str = ""
     emit_thread_coords: bool = True
+    split: bool = False
     name: str = "matmul_setup"
     kind: str = "setup"
 
@@ -419,6 +421,7 @@ class MatmulSetupFragment:
         a = f"acc{self.accumulator_suffix}"
         return "\n".join(
             [
+                *([f"mt_lost mt_cut{self.accumulator_suffix} = {{}};"] if self.split else ()),
                 f"mt_f32x16 {a}[{t.WM}][{t.WN}];",
                 "#pragma unroll",
                 f"for (int i = 0; i < {t.WM}; ++i)",
@@ -436,8 +439,8 @@ class MatmulSetupFragment:
 class MatmulComputeFragment:
     """MFMAs over the LDS k-chunk in buffer ``stage`` (set by the mainloop).
     ``split``: fp32 operands as three bf16 parts on the bf16 matrix cores
-    (``mt_mfma_tile``; a ``MatmulExactRetryFragment`` follows the mainloop);
-    without it, fp32 MFMAs (``mt_mfma_tile_f32``), which need nothing after
+    (``mt_mfma_tile``; the setup is split too and a ``MatmulExactRetryFragment``
+    follows the mainloop); without it, fp32 MFMAs (``mt_mfma_tile_f32``), which need nothing after
     them -- the default for kernels composed by hand."""
 
     config: MatmulConfig
@@ -472,6 +475,7 @@ class MatmulComputeFragment:
                 f"mt_mfma_tile_f32<{t.WM}, {t.WN}, {t.tile_K}, {t.lda}, {t.ldb}{flags}>"
                 f"({a_ptr}, {b_ptr}, acc{self.accumulator_suffix}, lane);"
             )
+        sfx = self.accumulator_suffix
         if hook is not None and not flags:
             flags = ", false, false"
         if held is not None:
@@ -479,12 +483,12 @@ class MatmulComputeFragment:
                 raise ValueError("a held group and a load hook do not combine")
             return (
                 f"mt_mfma_tile_held<{t.WM}, {t.WN}, {t.tile_K}, {t.lda}, {t.ldb}{flags}>"
-                f"({a_ptr}, {b_ptr}, acc{self.accumulator_suffix}, lane, {held[0]}, {held[1]});"
+                f"({a_ptr}, {b_ptr}, mt_cut{sfx}, acc{sfx}, lane, {held[0]}, {held[1]});"
             )
         hook_arg = f", {hook}" if hook is not None else ""
         return (
             f"mt_mfma_tile<{t.WM}, {t.WN}, {t.tile_K}, {t.lda}, {t.ldb}{flags}>"
-            f"({a_ptr}, {b_ptr}, acc{self.accumulator_suffix}, lane{hook_arg});"
+            f"({a_ptr}, {b_ptr}, mt_cut{sfx}, acc{sfx}, lane{hook_arg});"
         )
 
     def render_held_decl(self, var: str) -> str:
@@ -513,17 +517,19 @@ class MatmulComputeFragment:
 
 @dataclass(frozen=True)
 class MatmulExactRetryFragment:
-    """After a split mainloop: a wave whose accumulators hold a NaN or a
-    vanishingly small value (``mt_mfma_retry``) computes its blocks again with
-    fp32 MFMAs on operands read from global memory (``mt_mfma_exact``), over
-    the chunks this workgroup walked.  ``a`` / ``b`` are (parameter, row
-    stride, col stride, prologue lambda over (raw, row, col) or None)."""
+    """After a split mainloop: a wave whose accumulators the splits may have got
+    wrong (``mt_mfma_retry``) computes its blocks again with fp32 MFMAs on
+    operands read from global memory (``mt_mfma_exact``), over the chunks this
+    workgroup walked.  ``a`` / ``b`` are (parameter, row stride, col stride,
+    prologue lambda over (raw, row, col) or None); ``check``: the tile may reach
+    past the matrix."""
 
     config: MatmulConfig
     a: tuple[str, int, int, str | None]
     b: tuple[str, int, int, str | None]
     accumulator_suffix: str = ""
     persistent: bool = False
+    check: bool = False
     name: str = "matmul_exact_retry"
     kind: str = "compute"
 
@@ -542,6 +548,16 @@ class MatmulExactRetryFragment:
             "}();",
         ]
 
+    @staticmethod
+    def _largest(operand: tuple, rows: tuple[str, str], cols: tuple[str, str]) -> str:
+        """A lambda: the operand's largest magnitude in [rows) x [cols), or an
+        infinity where its floats do not lie in lines or have a prologue."""
+        src, rs, cs, transform = operand
+        if transform or (rs != 1 and cs != 1):
+            return "[] { return __builtin_inff(); }"
+        lines, elements, pitch = (rows, cols, rs) if cs == 1 else (cols, rows, cs)
+        return f"[&] {{ return mt_largest({src}, {pitch}u, {', '.join((*lines, *elements))}, lane); }}"
+
     def render(self, ctx: CodegenContext) -> str:
         c, t = self.config, self.config.tile
         acc = f"acc{self.accumulator_suffix}"
@@ -550,8 +566,16 @@ class MatmulExactRetryFragment:
             kb, ke = f"mt_kb * {t.tile_K}u", f"(mt_ke * {t.tile_K}u < {k} ? mt_ke * {t.tile_K}u : {k})"
         else:
             kb, ke = "0u", k
+        m0, n0 = "tile_m0 + wave_m0", "tile_n0 + wave_n0"
+        rows, cols = f"{t.wave_M}u", f"{t.wave_N}u"
+        if self.check:
+            rows, cols = (f"({at} < {end} ? {end} - ({at}) : 0u)" for at, end in ((m0, c.M_dim_var), (n0, c.N_dim_var)))
+            rows, cols = f"min({rows}, {t.wave_M}u)", f"min({cols}, {t.wave_N}u)"
+        top_a = self._largest(self.a, (m0, f"{m0} + {rows}"), (kb, ke))
+        top_b = self._largest(self.b, (kb, ke), (n0, f"{n0} + {cols}"))
         lines = [
-            f"if (mt_mfma_retry<{t.WM}, {t.WN}>({acc})) {{",
+            f"if (mt_mfma_retry<{t.WM}, {t.WN}>({acc}, mt_cut{self.accumulator_suffix}, {k}, {rows}, {cols}, lane, "
+            f"{top_a}, {top_b})) {{",
             *["    " + x for x in self._operand("mt_fa", self.a, c.M_dim_var, k)],
             *["    " + x for x in self._operand("mt_fb", self.b, k, c.N_dim_var)],
             f"    mt_mfma_exact<{t.WM}, {t.WN}>(mt_fa, mt_fb, tile_m0 + wave_m0, tile_n0 + wave_n0, {kb}, {ke}, lane, {acc});",
@@ -824,8 +848,8 @@ class MatmulRowWavesFragment:
             return [
                 f"    if ({more}) ld_B.fetch({b}, {brs}u, (kt + {ahead}u) * 64u, threadIdx.x);",
                 f"    mt_rw_chunk(mt_a, mt_arow, (kt + {ahead}u) * 64u, {more}, &B_tile[{stage}][0][0], "
-                f"&B_low[{stage}][0][0], mt_n0, {pa}, lane, acc);",
-                f"    if ({more}) ld_B.commit(&B_tile[{stage ^ 1}][0][0], &B_low[{stage ^ 1}][0][0], threadIdx.x);",
+                f"&B_low[{stage}][0][0], mt_n0, {pa}, lane, mt_cut, acc);",
+                f"    if ({more}) ld_B.commit(&B_tile[{stage ^ 1}][0][0], &B_low[{stage ^ 1}][0][0], threadIdx.x, mt_cut);",
                 "    __syncthreads();",
             ]
 
@@ -845,6 +869,7 @@ class MatmulRowWavesFragment:
             "const unsigned mt_m0 = blockIdx.y * 256u + (wave >> 1) * 32u;",
             "const unsigned mt_n0 = (wave & 1u) * 64u;",
             "const unsigned mt_row = mt_m0 + (lane & 31u);",
+            "mt_lost mt_cut = {};",
             "mt_f32x16 acc[1][2];",
             "mt_zero(acc[0][0]);",
             "mt_zero(acc[0][1]);",
@@ -875,7 +900,7 @@ class MatmulRowWavesFragment:
             f"ld_B.fetch({b}, {self.b_row_stride}u, 0u, threadIdx.x);",
             "#pragma unroll",
             "for (int s = 0; s < 4; ++s) mt_rw_load(mt_a[s], mt_arow, 0u, s);",
-            "ld_B.commit(&B_tile[0][0][0], &B_low[0][0][0], threadIdx.x);",
+            "ld_B.commit(&B_tile[0][0][0], &B_low[0][0][0], threadIdx.x, mt_cut);",
             "__syncthreads();",
             "const unsigned n_chunks = K / 64u;",
         ]
@@ -886,8 +911,11 @@ class MatmulRowWavesFragment:
         else:
             lines += self._loop("mt_pa")
         value = self.value_expr.format(a0="acc[0][j][v]") if self.value_expr else "acc[0][j][v]"
+        top_a = f"mt_largest({a}, {self.a_row_stride}u, mt_m0, mt_m0 + 32u, 0u, K, lane)" if pro is None else "__builtin_inff()"
         lines += [
-            "if (mt_mfma_retry<1, 2>(acc)) {",
+            "mt_cut.b = __syncthreads_or(mt_cut.b != 0ull ? 1 : 0) != 0 ? 1ull : 0ull;  // any lane's share of B",
+            "if (mt_mfma_retry<1, 2>(acc, mt_cut, K, 32u, 64u, lane, "
+            f"[&] {{ return {top_a}; }}, [&] {{ return mt_largest({b}, {self.b_row_stride}u, 0u, K, mt_n0, mt_n0 + 64u, lane); }})) {{",
             f"    const auto mt_fa = [=](unsigned r, unsigned k) -> float {{ return {value_at}; }};",
             f"    const auto mt_fb = [&](unsigned k, unsigned n) -> float {{ return {b}[(size_t)k * {self.b_row_stride}u + n]; }};",
             "    mt_mfma_exact<1, 2>(mt_fa, mt_fb, mt_m0, mt_n0, 0u, K, lane, acc);",

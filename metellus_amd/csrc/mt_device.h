@@ -980,9 +980,15 @@ MT_INLINE void mt_mfma_tile_f32(const float* __restrict__ As, const float* __res
 //
 // What a split cannot do: an infinite x, or one that rounds to an infinite x1
 // (from 0x1.ffp+127), leaves a NaN or an infinity of the wrong sign as its
-// remainder, which makes every sum it enters a NaN; and below 2^-110 the lower
-// parts fall under bf16's smallest number.  mt_mfma_retry finds such tiles by
-// their results.
+// remainder, which makes every sum it enters a NaN; mt_mfma_retry finds those by
+// their results.  And an x below 2^-110 may have bits below 2^-133, bf16's
+// smallest number (the MFMAs keep subnormals): the third part cuts them off, an
+// error of up to 2^-133 times whatever the other operand is.  Results do not show
+// that, so every split says whether it cut anything off (mt_lost): half a VALU
+// operation per element.  Measured on MI355X without and with it: 4096^3 674 -> 696
+// us, 1531 x 1000 x 3001 96 -> 103 us, C4 MLP 5.88 -> 6.07 ms.  Dearer were a
+// running minimum and maximum of the operands held by every wave (4096^3 737 us),
+// or taken by every lane of its share of the LDS tile (742 us).
 // ---------------------------------------------------------------------------
 
 typedef __bf16 mt_bf16x8 __attribute__((ext_vector_type(8)));
@@ -1002,8 +1008,14 @@ MT_INLINE unsigned mt_pack_hi16(float lo, float hi) {  // upper halves of two fl
 }
 MT_INLINE float mt_keep_hi16(unsigned x) { return __builtin_bit_cast(float, x & 0xffff0000u); }
 
-MT_INLINE mt_split8 mt_split(mt_f32x4 u, mt_f32x4 v) {
+// Lanes whose splits of A's and of B's elements cut off nonzero bits.
+struct mt_lost {
+    unsigned long long a, b;
+};
+
+MT_INLINE mt_split8 mt_split(mt_f32x4 u, mt_f32x4 v, unsigned long long& lost) {
     mt_split8 o;
+    unsigned low = 0u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const float x0 = q < 2 ? u[2 * q] : v[2 * q - 4], x1 = q < 2 ? u[2 * q + 1] : v[2 * q - 3];
@@ -1012,8 +1024,11 @@ MT_INLINE mt_split8 mt_split(mt_f32x4 u, mt_f32x4 v) {
         const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - mt_keep_hi16(h);
         const unsigned m = mt_cvt_pk_bf16(r0, r1);
         o.p2[q] = m;
-        o.p3[q] = mt_pack_hi16(r0 - __builtin_bit_cast(float, m << 16), r1 - mt_keep_hi16(m));
+        const float z0 = r0 - __builtin_bit_cast(float, m << 16), z1 = r1 - mt_keep_hi16(m);
+        o.p3[q] = mt_pack_hi16(z0, z1);
+        low |= __builtin_bit_cast(unsigned, z0) | __builtin_bit_cast(unsigned, z1);
     }
+    lost |= __ballot((low & 0xffffu) != 0u);
     return o;
 }
 
@@ -1037,8 +1052,9 @@ MT_INLINE mt_f32x16 mt_mfma_parts(const mt_split8& a, const mt_split8& b, mt_f32
 // an MFMA does not wait for the one before it (C4 X @ W1: 1840 us; block by
 // block 1924 us).
 template <int WN>
-MT_INLINE void mt_mfma_split(mt_f32x4 a0, mt_f32x4 a1, const mt_split8 (&b)[WN], mt_f32x16 (&acc)[WN]) {
-    const mt_split8 a = mt_split(a0, a1);
+MT_INLINE void mt_mfma_split(mt_f32x4 a0, mt_f32x4 a1, const mt_split8 (&b)[WN], unsigned long long& lost,
+                             mt_f32x16 (&acc)[WN]) {
+    const mt_split8 a = mt_split(a0, a1, lost);
 #pragma unroll
     for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p3, b[j].p1, acc[j]);
 #pragma unroll
@@ -1061,7 +1077,7 @@ struct mt_no_hook {
 
 // The chunk in the layouts of mt_mfma_tile_f32.
 template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false, typename H = mt_no_hook>
-MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restrict__ Bs,
+MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restrict__ Bs, mt_lost& lost,
                             mt_f32x16 (&acc)[WM][WN], unsigned lane, H hook = H{}) {
     static_assert(TK % 16 == 0, "TK must be a multiple of 16");
     static_assert(LDA % 4 == 0, "LDA must keep 16-byte alignment");
@@ -1085,12 +1101,12 @@ MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restric
         for (int j = 0; j < WN; ++j) {
             if constexpr (BNM) {
                 const float* row = b_base + j * 32 * TK;
-                b[j] = mt_split(mt_ld4(row + 4u * (slot0 ^ m)), mt_ld4(row + 4u * (slot1 ^ m)));
+                b[j] = mt_split(mt_ld4(row + 4u * (slot0 ^ m)), mt_ld4(row + 4u * (slot1 ^ m)), lost.b);
             } else {
                 mt_f32x4 q[2];
 #pragma unroll
                 for (int ss = 0; ss < 8; ++ss) q[ss / 4][ss % 4] = b_base[(s0 + ss) * LDB + j * 32];
-                b[j] = mt_split(q[0], q[1]);
+                b[j] = mt_split(q[0], q[1], lost.b);
             }
         }
 #pragma unroll
@@ -1099,7 +1115,7 @@ MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restric
             const float* row = a_base + i * 32 * LDA;
             const mt_f32x4 a0 = ASWZ ? mt_ld4(row + 4u * (slot0 ^ m)) : mt_ld4(row + s0);
             const mt_f32x4 a1 = ASWZ ? mt_ld4(row + 4u * (slot1 ^ m)) : mt_ld4(row + s0 + 4);
-            mt_mfma_split<WN>(a0, a1, b, acc[i]);
+            mt_mfma_split<WN>(a0, a1, b, lost.a, acc[i]);
         }
     }
     __builtin_amdgcn_s_setprio(0);
@@ -1117,20 +1133,63 @@ template <int WM, int WN>
 MT_INLINE void mt_mfma_group_run(const mt_mfma_group<WM, WN>&, mt_f32x16 (&)[WM][WN]) {}
 
 template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false>
-MT_INLINE void mt_mfma_tile_held(const float* __restrict__ As, const float* __restrict__ Bs,
+MT_INLINE void mt_mfma_tile_held(const float* __restrict__ As, const float* __restrict__ Bs, mt_lost& lost,
                                  mt_f32x16 (&acc)[WM][WN], unsigned lane, mt_mfma_group<WM, WN>&, bool) {
-    mt_mfma_tile<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, acc, lane);
+    mt_mfma_tile<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, lost, acc, lane);
+}
+
+// Row (within a 32x32 output block) of accumulator register v held by `lane`;
+// the column is lane % 32.
+MT_INLINE unsigned mt_acc_row(int v, unsigned lane) {
+    return 8u * (unsigned)(v >> 2) + 4u * (lane >> 5) + (unsigned)(v & 3);
+}
+
+// Largest magnitude of lines [l0, l1), elements [e0, e1) each, of a matrix whose
+// lines are contiguous and `pitch` apart: the whole wave, 4 lines of 64 elements a
+// load.
+MT_INLINE float mt_largest(const float* __restrict__ src, size_t pitch, unsigned l0, unsigned l1, unsigned e0,
+                           unsigned e1, unsigned lane) {
+    constexpr unsigned UNROLL = 8u;
+    float top = 0.0f;
+    for (unsigned e = e0 + 4u * (lane & 15u); e < e1; e += 64u)
+        for (unsigned l = l0 + (lane >> 4); l < l1; l += 4u * UNROLL) {
+            mt_f32x4 x[UNROLL];
+#pragma unroll
+            for (unsigned u = 0; u < UNROLL; ++u)
+                x[u] = l + 4u * u < l1 ? mt_ld_slot(src + (l + 4u * u) * pitch + e, e1 - e) : mt_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (unsigned u = 0; u < UNROLL; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) top = __builtin_fmaxf(top, __builtin_fabsf(x[u][q]));
+        }
+    return mt_wave_max(top);
 }
 
 // Whether the wave's accumulators may differ from the fp32 products' sums for
 // want of range: a value that is not finite (every sum an infinite or NaN operand
 // enters is a NaN here, where fp32 may give an infinity; and a part of a product
-// may pass the largest float where the product does not, as x1 is rounded up) or a
-// nonzero result below 2^-96, which takes operands small enough to have lost their
-// lower parts.  Wave uniform.
-template <int WM, int WN>
-MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN]) {
+// may pass the largest float where the product does not, as x1 is rounded up); a
+// nonzero one below 2^-96, whose smaller partial products may be subnormal; and,
+// where an operand's splits cut bits off, one these could matter to: K of them are
+// below K 2^-133 times the other operand's largest magnitude, which ta() and tb()
+// look up.  So the weights of a softmax may underflow beside ordinary ones.  Rows
+// and columns from `rows` and `cols` on are outside the matrix.  Wave uniform.
+template <int WM, int WN, typename TA, typename TB>
+MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN], const mt_lost& lost, unsigned K, unsigned rows,
+                             unsigned cols, unsigned lane, TA ta, TB tb) {
     bool odd = false;
+    if ((lost.a | lost.b) != 0ull) {
+        const float top = __builtin_fmaxf(lost.b != 0ull ? ta() : 0.0f, lost.a != 0ull ? tb() : 0.0f);
+        const float least = 0x1.0p-107f * (float)K * top;  // 2^25 times what both may have lost
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    odd |= !(__builtin_fabsf(acc[i][j][v]) >= least) &&
+                           32u * (unsigned)i + mt_acc_row(v, lane) < rows && 32u * (unsigned)j + (lane & 31u) < cols;
+    }
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -1203,8 +1262,8 @@ struct mt_rw_stage {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = p[(size_t)e * ldb];
     }
-    MT_INLINE void commit(float* hi, float* lo, unsigned tid) const {
-        const mt_split8 x = mt_split(mt_f32x4{v[0], v[1], v[2], v[3]}, mt_f32x4{v[4], v[5], v[6], v[7]});
+    MT_INLINE void commit(float* hi, float* lo, unsigned tid, mt_lost& lost) const {
+        const mt_split8 x = mt_split(mt_f32x4{v[0], v[1], v[2], v[3]}, mt_f32x4{v[4], v[5], v[6], v[7]}, lost.b);
         reinterpret_cast<mt_u32x4*>(hi)[tid] = x.p1;
         reinterpret_cast<mt_u32x4*>(hi)[1024u + tid] = x.p2;
         reinterpret_cast<mt_u32x4*>(lo)[tid] = x.p3;
@@ -1224,7 +1283,7 @@ MT_INLINE void mt_rw_load(mt_f32x4 (&a)[2], const float* __restrict__ arow, unsi
 template <typename P>
 MT_INLINE void mt_rw_chunk(mt_f32x4 (&a)[4][2], const float* __restrict__ arow, unsigned k_next, bool more,
                            const float* __restrict__ hi, const float* __restrict__ lo, unsigned n0, P pa, unsigned lane,
-                           mt_f32x16 (&acc)[1][2]) {
+                           mt_lost& lost, mt_f32x16 (&acc)[1][2]) {
     const mt_u32x4* __restrict__ h4 = reinterpret_cast<const mt_u32x4*>(hi) + n0 + (lane & 31u);
     const mt_u32x4* __restrict__ l4 = reinterpret_cast<const mt_u32x4*>(lo) + n0 + (lane & 31u);
     __builtin_amdgcn_s_setprio(1);
@@ -1235,7 +1294,7 @@ MT_INLINE void mt_rw_chunk(mt_f32x4 (&a)[4][2], const float* __restrict__ arow, 
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e / 4][e % 4] = pa(a[s][e / 4][e % 4]);
         if (more) mt_rw_load(a[s], arow, k_next, s);
-        const mt_split8 xa = mt_split(x[0], x[1]);
+        const mt_split8 xa = mt_split(x[0], x[1], lost.a);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const mt_split8 b = {h4[g + 32u * j], h4[1024u + g + 32u * j], l4[g + 32u * j]};
@@ -1568,12 +1627,6 @@ MT_INLINE void mt_buffer_store4(mt_f32x4 v, mt_u32x4 rs, unsigned voff, unsigned
                      :
                      : "v"(v), "v"(voff), "s"(rs), "s"(so)
                      : "memory");
-}
-
-// Row (within a 32x32 output block) of accumulator register v held by `lane`;
-// the column is lane % 32.
-MT_INLINE unsigned mt_acc_row(int v, unsigned lane) {
-    return 8u * (unsigned)(v >> 2) + 4u * (lane >> 5) + (unsigned)(v & 3);
 }
 
 MT_INLINE void mt_zero(mt_f32x16& a) {

@@ -440,7 +440,8 @@ def b_tile_for(tile: TileConfig, src_b: Tensor) -> TileConfig:
 
 
 def exact_retry(config: MatmulConfig, src_a: Tensor, src_b: Tensor, pro_a: ChainCode | None,
-                pro_b: ChainCode | None, suffix: str = "", persistent: bool = False) -> MatmulExactRetryFragment:
+                pro_b: ChainCode | None, suffix: str = "", persistent: bool = False,
+                check: bool = False) -> MatmulExactRetryFragment:
     """The fp32 fallback of a split mainloop over these operands."""
 
     def operand(src: Tensor, pro: ChainCode | None):
@@ -448,7 +449,7 @@ def exact_retry(config: MatmulConfig, src_a: Tensor, src_b: Tensor, pro_a: Chain
                 pro.lambda_transform() if pro is not None else None)
 
     return MatmulExactRetryFragment(config, a=operand(src_a, pro_a), b=operand(src_b, pro_b),
-                                    accumulator_suffix=suffix, persistent=persistent)
+                                    accumulator_suffix=suffix, persistent=persistent, check=check)
 
 
 # A 256x256 tile with bounds stores its 256 KiB after a short k loop with no
@@ -616,9 +617,10 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         MatmulTileMappingFragment(persistent, xcd_rows=xcd_rows(grid_for(M, N, tile)) if persistent is None else 0,
                                   split=(parts, tile.tile_K) if parts > 1 else None),
         ThreadIndexFragment(tile),
-        MatmulSetupFragment(config),
+        MatmulSetupFragment(config, split=True),
         mainloop,
-        exact_retry(config, src_a, src_b, pro_a, pro_b, persistent=persistent is not None or parts > 1),
+        exact_retry(config, src_a, src_b, pro_a, pro_b, persistent=persistent is not None or parts > 1,
+                    check=not aligned),
         *((MatmulSplitSumFragment(config, parts),) if parts > 1 else ()),
         *((StreamKFixupFragment(config),) if stream_k else ()),
         store,

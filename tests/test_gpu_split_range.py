@@ -1,6 +1,7 @@
 """Split matmuls at the ends of float32's range, in every kernel that splits
-its operands (``mt_split``): accumulators that pass the largest float inside a
-step although no sum of products does."""
+its operands (``mt_split``): operands too small for three bf16 parts against
+ones large enough that the products are of ordinary size, and accumulators
+that pass the largest float inside a step although no sum of products does."""
 
 from __future__ import annotations
 
@@ -62,6 +63,54 @@ def _product(name, a, b, text):
     assert text in g.kernel.source.split('extern "C"')[-1]
     got = run(ops).env[out]
     return got, {"d": 0.5, "p": 2.0}.get(name[0], 1.0) if name.startswith(("divided", "pair")) else 1.0
+
+
+def _spread(rng, shape, low, high):
+    return (rng.uniform(1.0, 2.0, shape) * rng.choice((-1.0, 1.0), shape)
+            * np.exp2(rng.integers(low, high, shape, endpoint=True))).astype(np.float32)
+
+
+@pytest.mark.parametrize("large", ["right", "left"])
+@pytest.mark.parametrize("rows", ["every", "some"])
+@pytest.mark.parametrize("low,high", [(-140, -112), (-117, -116), (-140, -140)])
+@pytest.mark.parametrize("name", list(FORMS))
+def test_small_against_large(name, low, high, rows, large, monkeypatch):
+    """Below 2^-110 a float is no sum of three bf16 numbers; products with 2^40
+    .. 2^100 are of ordinary size, so only the operands show it."""
+    (M, K, N), text = _form(name, monkeypatch)
+    print(f"split range {name} 2^{low}..2^{high} {rows} large={large}", flush=True)
+    rng = np.random.default_rng(31)
+    a, b = _spread(rng, (M, K), low, high), _spread(rng, (K, N), 40, 100)
+    if rows == "some":  # the others share their waves and tiles
+        a[np.arange(M) % 37 != 5] = 0.0
+    if large == "left":
+        flip = _spread(rng, (M, K), 40, 100), _spread(rng, (K, N), low, high)
+        a, b = flip
+        if rows == "some":
+            b[:, np.arange(N) % 41 != 7] = 0.0
+    if name.startswith("divided"):
+        a = (a * np.float32(0.5)) * np.float32(2.0)  # exact quotients, subnormal ones too
+    got, scale = _product(name, a, b, text)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    # K products and as many sums, each rounded by at most 2^-24 of the sum of
+    # magnitudes (a part, a merge and an underflow are within the 8)
+    bound = scale * (K + 8) * 2.0**-24 * (np.abs(a64) @ np.abs(b64)) + K * 2.0**-149
+    assert np.all(np.abs(got - scale * (a64 @ b64)) <= bound)
+
+
+@pytest.mark.parametrize("name", list(FORMS))
+def test_small_values_of_a_softmax(name, monkeypatch):
+    """Weights from 1 down to the smallest subnormal, as a row of exponentials has them."""
+    (M, K, N), text = _form(name, monkeypatch)
+    print(f"split range {name} softmax", flush=True)
+    rng = np.random.default_rng(32)
+    a = np.exp(-rng.uniform(0, 103, (M, K))).astype(np.float32)
+    a[:, 0] = 1.0
+    b = rng.standard_normal((K, N)).astype(np.float32)
+    got, scale = _product(name, a, b, text)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    bound = scale * (K + 8) * 2.0**-24 * (np.abs(a64) @ np.abs(b64)) + K * 2.0**-149
+    assert np.all(np.abs(got - scale * (a64 @ b64)) <= bound)
 
 
 @pytest.mark.parametrize("name", list(FORMS))
