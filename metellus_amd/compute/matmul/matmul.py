@@ -534,18 +534,17 @@ class MatmulExactRetryFragment:
     kind: str = "compute"
 
     @staticmethod
-    def _operand(label: str, operand: tuple, rows: str, cols: str) -> list[str]:
+    def _operand(label: str, operand: tuple, side: str, lines: str, ke: str) -> list[str]:
+        """``label``(line, k): four k's of a row of A or of a column of B."""
         src, rs, cs, transform = operand
-        at = f"{src}[(size_t)r * {rs}u + (size_t)c * {cs}u]"
-        lines = [f"const auto xf = {transform};"] if transform else []
-        value = f"xf({at}, r, c)" if transform else at
-        capture = "[=]" if transform else "[&]"
+        ls, ks = (rs, cs) if side == "a" else (cs, rs)
+        value = "raw" if not transform else "xf(raw, line, k)" if side == "a" else "xf(raw, k, line)"
         return [
-            f"const auto {label} = [&] {{",
-            *[f"    {x}" for x in lines],
-            f"    return {capture}(unsigned r, unsigned c) -> float "
-            f"{{ return r < {rows} && c < {cols} ? {value} : 0.0f; }};",
-            "}();",
+            f"const auto {label} = [&](unsigned line, unsigned k0) -> mt_f32x4 {{",
+            *([f"    const auto xf = {transform};"] if transform else ()),
+            f"    return mt_exact_quad<{'true' if ks == 1 else 'false'}>({src}, {ls}u, {ks}u, line, k0, {lines}, {ke},",
+            f"        [&](float raw, unsigned k) -> float {{ return {value}; }});",
+            "};",
         ]
 
     @staticmethod
@@ -576,8 +575,8 @@ class MatmulExactRetryFragment:
         lines = [
             f"if (mt_mfma_retry<{t.WM}, {t.WN}>({acc}, mt_cut{self.accumulator_suffix}, {k}, {rows}, {cols}, lane, "
             f"{top_a}, {top_b})) {{",
-            *["    " + x for x in self._operand("mt_fa", self.a, c.M_dim_var, k)],
-            *["    " + x for x in self._operand("mt_fb", self.b, k, c.N_dim_var)],
+            *["    " + x for x in self._operand("mt_fa", self.a, "a", c.M_dim_var, ke)],
+            *["    " + x for x in self._operand("mt_fb", self.b, "b", c.N_dim_var, ke)],
             f"    mt_mfma_exact<{t.WM}, {t.WN}>(mt_fa, mt_fb, tile_m0 + wave_m0, tile_n0 + wave_n0, {kb}, {ke}, lane, {acc});",
             "}",
         ]
@@ -878,20 +877,16 @@ class MatmulRowWavesFragment:
             "mt_f32x4 mt_a[4][2];",
         ]
         plain = False
-        raw = f"{a}[(size_t)r * {self.a_row_stride}u + k]"
         if pro is None:
             lines.append("const auto mt_pa = [](float raw) -> float { return raw; };")
-            value_at = raw
         elif pro[0] == "transform":
             lines += [f"const auto xt = {pro[1]};",
                       "const auto mt_pa = [=](float raw) -> float { return xt(raw, mt_row, 0u); };"]
-            value_at = f"xt({raw}, r, 0u)"
         else:
             _, gather, apply, plain_apply, plain_pred = pro
             lines += [f"const auto xg = {gather};", f"const auto xa = {apply};",
                       "const auto mt_e = xg(mt_row, 0u);  // the row's operands",
                       "const auto mt_pa = [=](float raw) -> float { return xa(raw, mt_e); };"]
-            value_at = f"xa({raw}, xg(r, 0u))"
             if plain_apply is not None:
                 plain = True
                 lines += [f"const auto xq = {plain_apply};", f"const auto xp = {plain_pred};",
@@ -916,8 +911,10 @@ class MatmulRowWavesFragment:
             "mt_cut.b = __syncthreads_or(mt_cut.b != 0ull ? 1 : 0) != 0 ? 1ull : 0ull;  // any lane's share of B",
             "if (mt_mfma_retry<1, 2>(acc, mt_cut, K, 32u, 64u, lane, "
             f"[&] {{ return {top_a}; }}, [&] {{ return mt_largest({b}, {self.b_row_stride}u, 0u, K, mt_n0, mt_n0 + 64u, lane); }})) {{",
-            f"    const auto mt_fa = [=](unsigned r, unsigned k) -> float {{ return {value_at}; }};",
-            f"    const auto mt_fb = [&](unsigned k, unsigned n) -> float {{ return {b}[(size_t)k * {self.b_row_stride}u + n]; }};",
+            f"    const auto mt_fa = [&](unsigned r, unsigned k0) {{ return mt_exact_quad<true>({a}, {self.a_row_stride}u, 1u, r, k0, "
+            "M, K, [&](float raw, unsigned) { return mt_pa(raw); }); };  // r is mt_row",
+            f"    const auto mt_fb = [&](unsigned n, unsigned k0) {{ return mt_exact_quad<false>({b}, 1u, {self.b_row_stride}u, n, k0, "
+            "N, K, [](float raw, unsigned) { return raw; }); };",
             "    mt_mfma_exact<1, 2>(mt_fa, mt_fb, mt_m0, mt_n0, 0u, K, lane, acc);",
             "}",
             "#pragma unroll",

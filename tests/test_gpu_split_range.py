@@ -25,6 +25,7 @@ FORMS = {
     "row waves": ((256, 1024, 128), {}, "mt_rw_chunk("),
     "divided row waves": ((256, 1024, 128), {}, "mt_rw_chunk("),
     "divided tile": ((129, 331, 195), {}, "mt_mfma_tile<"),
+    "transposed operands": ((129, 331, 195), {}, "mt_mfma_tile<"),
     "pair": ((130, 333, 200), {}, "acc_1"),
     "pair of two left operands": ((130, 333, 200), {}, "acc_1"),
 }
@@ -43,14 +44,20 @@ def _form(name, monkeypatch):
 def _product(name, a, b, text):
     """The product through the form's kernel; a pair's as the sum of two equal ones."""
     ops = Operations()
-    ops.from_numpy(a, "A")
-    ops.from_numpy(b, "B")
-    left = "A"
+    left, right = "A", "B"
+    if name.startswith("transposed"):
+        ops.from_numpy(np.ascontiguousarray(a.T), "At")
+        ops.from_numpy(np.ascontiguousarray(b.T), "Bt")
+        ops.transpose("At", out="A")
+        ops.transpose("Bt", out="B")
+    else:
+        ops.from_numpy(a, "A")
+        ops.from_numpy(b, "B")
     if name.startswith("divided"):
         ops.from_numpy(np.full((a.shape[0], 1), 2.0, np.float32), "s")
         ops.elementwise("div", out="P", operands=("A", "s"), y_broadcast="col")
         left = "P"
-    ops.matmul(a=left, b="B", out="C")
+    ops.matmul(a=left, b=right, out="C")
     out = "C"
     if name.startswith("pair"):
         ops.from_numpy(b, "B2")
