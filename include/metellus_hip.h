@@ -134,8 +134,9 @@ int mt_launch(uint64_t kernel, const uint64_t* buffers, int nbuf, const uint32_t
  * per dispatch (reference: src/runtime/program.py:179-196).  Launch n kernels in
  * order, untimed, in one call: each item is mt_launch's arguments, and
  * workspace > 0 appends the mt_workspace buffer (grown to at least that many
- * bytes) as the kernel's last parameter.  Stops at the first item that fails;
- * the ones before it are queued. */
+ * bytes) as the kernel's last parameter.  A workspace below its 4096-byte head
+ * is refused before anything is queued; otherwise stops at the first item that
+ * fails, the ones before it queued. */
 typedef struct mt_launch_item {
     uint64_t kernel;
     const uint64_t* buffers;

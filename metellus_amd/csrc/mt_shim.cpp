@@ -885,6 +885,10 @@ int mt_launch(uint64_t kernel, const uint64_t* buffers, int nbuf, const uint32_t
 
 int mt_launch_many(const mt_launch_item* items, int n) {
     if (n < 0 || (n > 0 && !items)) return fail("mt_launch_many: bad items");
+    for (int i = 0; i < n; ++i) {
+        if (items[i].workspace != 0 && items[i].workspace < kWsHeadBytes)
+            return fail("mt_launch_many: a workspace holds at least its 4096-byte head");
+    }
     State& s = state();
     std::lock_guard<std::mutex> lock(s.mu);
     if (init_locked(s)) return 1;

@@ -63,6 +63,15 @@ def test_device_calls_fail_loudly_without_gpu():
         hip_backend.create_buffer(16)
 
 
+def test_small_workspace_is_refused_before_device():
+    """A workspace starts with 4096 bytes of flags that are cleared when it is made."""
+    with pytest.raises(RuntimeError, match="4096-byte head"):
+        hip_backend.workspace_handle(4095)
+    small = [(1, 0, (), 0, (1, 1, 1), (64, 1, 1), size) for size in (0, 4096, 4095)]
+    with pytest.raises(RuntimeError, match="4096-byte head"):
+        hip_backend.LaunchSequence(small).launch([])
+
+
 def test_buffer_validation_before_device():
     with pytest.raises(RuntimeError, match="nbytes must be > 0"):
         hip_backend.create_buffer(0)
