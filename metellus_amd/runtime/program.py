@@ -261,6 +261,10 @@ class Runtime:
             object.__setattr__(self, "_made", made)
         return made
 
+    def __getstate__(self) -> dict:
+        """Copies and pickles lay their launches out anew."""
+        return {k: v for k, v in self.__dict__.items() if k != "_made"}
+
     def run(self, env: Env | None = None) -> Env:
         if env is None:
             env = {}

@@ -2,16 +2,19 @@
 dispatch / download / free order and the validation errors (the
 host-side assertions of the reference's tests/test_scheduler.py)."""
 
+import copy
+
 import numpy as np
 import pytest
 
+from metellus_amd.runtime import hip_backend
 from orchestrator import Operations
 from orchestrator.aliasing import alias_group
 from orchestrator.assembly import assemble
 from orchestrator.fusion import fuse
 from orchestrator.scheduler import schedule
 from metellus_amd.api import compile_program
-from runtime import Allocate, Dispatch, Download, Free, FromNumpy, Kernel
+from runtime import Allocate, Dispatch, Download, Free, FromNumpy, Kernel, Runtime
 
 
 def _groups(ops):
@@ -140,3 +143,29 @@ def test_outputs_must_be_materialised():
         schedule(ops, groups, outputs=["t1"])  # fused into the chain kernel
     with pytest.raises(ValueError, match="unknown output"):
         schedule(ops, groups, outputs=["nope"])
+
+
+class _NoLaunch:
+    """A native library whose launches are all right."""
+
+    def __getattr__(self, name):
+        return lambda *a: 0
+
+
+@pytest.mark.parametrize("copy_of", [copy.deepcopy, copy.copy])
+def test_runtime_is_copied_after_a_run(copy_of, monkeypatch):
+    """Its laid-out launches hold a lock and an address: a copy makes its own."""
+    monkeypatch.setattr(hip_backend, "_load", lambda: _NoLaunch())
+    ops = Operations()
+    _mm(ops)
+    ops.matmul(a="A", b="B", out="C")
+    (g,) = _groups(ops)
+    kernel = Kernel(g.kernel.fragments, g.kernel.ctx)
+    kernel._handle = 1
+    rt = Runtime((Dispatch(kernel, g.bindings, g.dims, g.grid, g.threads),))
+    env = {name: 7 for name in g.bindings}
+    rt.run(env)
+    again = copy_of(rt)
+    assert len(again.fragments) == 1 and again.fragments[0].grid == g.grid
+    again.run(env)
+    assert again._made[0][0].sequence is not rt._made[0][0].sequence
