@@ -75,9 +75,9 @@ class CodegenContext:
     # 0): its batched variant does.
     workspace_optional: bool = False
     # A workgroup may wait for another one's partial sums (stream-K) and reports
-    # a wait that gave up in the workspace's error word; other users of the
-    # workspace never wait.
-    workspace_waits: bool = False
+    # a wait that gave up in the workspace's error word, which is checked after a
+    # run; false for a kernel with a workspace whose workgroups never wait.
+    workspace_waits: bool = True
 
     @property
     def num_threads(self) -> int:

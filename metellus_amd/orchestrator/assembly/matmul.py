@@ -743,6 +743,7 @@ def _assemble_skinny(decision: DecisionView, function_name: str | None, src_a: T
         helpers=tuple(helpers),
         workspace_bytes=skinny_workspace_bytes(grid[0] // splits * grid[1], row_blocks, splits),
         workspace_optional=True,
+        workspace_waits=False,
     )
     return KernelGroup(
         kernel=Kernel(fragments=(frag,), ctx=ctx),

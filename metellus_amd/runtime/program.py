@@ -256,7 +256,8 @@ class Runtime:
                 steps.append(f)
             if run:
                 steps.append(_Launches(run))
-            waits = any(isinstance(f, Dispatch) and f.kernel.ctx.workspace_waits for f in self.fragments)
+            waits = any(isinstance(f, Dispatch) and f.kernel.workspace_bytes and f.kernel.ctx.workspace_waits
+                        for f in self.fragments)
             made = (tuple(steps), waits)
             object.__setattr__(self, "_made", made)
         return made

@@ -3,6 +3,7 @@ dispatch / download / free order and the validation errors (the
 host-side assertions of the reference's tests/test_scheduler.py)."""
 
 import copy
+import dataclasses
 
 import numpy as np
 import pytest
@@ -14,6 +15,7 @@ from orchestrator.assembly import assemble
 from orchestrator.fusion import fuse
 from orchestrator.scheduler import schedule
 from metellus_amd.api import compile_program
+from metellus_amd.compute.fragments import CodegenContext
 from runtime import Allocate, Dispatch, Download, Free, FromNumpy, Kernel, Runtime
 
 
@@ -169,3 +171,28 @@ def test_runtime_is_copied_after_a_run(copy_of, monkeypatch):
     assert len(again.fragments) == 1 and again.fragments[0].grid == g.grid
     again.run(env)
     assert again._made[0][0].sequence is not rt._made[0][0].sequence
+
+
+@pytest.mark.parametrize("flags,checked", [({}, True), ({"workspace_waits": False}, False)])
+def test_error_word_is_checked_unless_a_kernel_never_waits(flags, checked, monkeypatch):
+    """A kernel composed by hand says its workspace's size and no more."""
+    calls = []
+    monkeypatch.setattr(hip_backend, "_load", lambda: _NoLaunch())
+    monkeypatch.setattr(hip_backend, "check_workspace", lambda: calls.append(1))
+    ctx = CodegenContext(function_name="k", buffers=("float* __restrict__ x",), dims=(), tg_x=64, tg_y=1)
+    for size in (0, 8192):
+        kernel = Kernel((), dataclasses.replace(ctx, workspace_bytes=size, **flags))
+        kernel._handle = 1
+        Runtime((Dispatch(kernel, ("x",), (), (1, 1, 1), (64, 1, 1)),)).run({"x": 7})
+    assert calls == [1] * checked
+
+
+def test_which_kernels_wait():
+    from tests import gpu_cases
+
+    waits = [
+        compile_program(gpu_cases.plain_matmul(*shape))[0].kernel
+        for shape in ((4096, 4096, 11008), (8, 4096, 4096), (256, 2048, 256))
+    ]
+    assert all(k.workspace_bytes > 0 for k in waits)
+    assert [k.ctx.workspace_waits for k in waits] == [True, False, False]  # stream-K, skinny, in parts
