@@ -235,10 +235,8 @@ class LastAxisReductionComputeFragment:
         return "\n".join(L)
 
 
-STRIDED_ROWS = 32  # rows of a workgroup: 128 contiguous bytes per load and 32 lanes
 STRIDED_LANES = 512
-STRIDED_GROUPS = STRIDED_LANES // STRIDED_ROWS  # lanes that share a row
-STRIDED_LOADS = 16  # elements in flight per lane
+STRIDED_LOADS = 32  # elements in flight per lane (16: 8192 rows of 8192 61 instead of 49 us, 64: 53)
 
 
 @dataclass(frozen=True)
@@ -246,28 +244,29 @@ class StridedReductionFragment(LastAxisReductionComputeFragment):
     """The same reduction of rows that are contiguous across each other (row
     stride 1: the columns of a row-major matrix, e.g. a bias gradient), in the
     same order.  One wave per row would load one element per cache line; here a
-    workgroup takes STRIDED_ROWS rows, 32 lanes load one element of each at a
+    workgroup takes ``rows`` rows, as many lanes load one element of each at a
     time, and lane group G keeps the partial values of lanes t = J G .. J G + J - 1
-    of the wave-per-row order (J = T / 16).  They meet in LDS, where one lane per
-    row folds them along the butterfly's tree.  Bound by HBM; measured on MI355X,
-    4096 rows of 2048 (32 MiB): 47.3 us with a wave per row, 10.5 us this way
-    (3.2 TB/s: 128 workgroups).  Includes the store (``out_name``, ``epilogue``)."""
+    of the wave-per-row order (J = T rows / STRIDED_LANES).  They meet in LDS, where one lane per
+    row folds them along the butterfly's tree.  Bound by what the workgroups keep in
+    flight; measured on MI355X against a wave per row: 4096 rows of 4096 (64 MiB,
+    128 workgroups) 103 -> 15 us, 1000 rows of 16384 141 -> 31 us.  Includes the store (``out_name``, ``epilogue``)."""
 
     rows_dim: str = "M"
+    rows: int = 32
     out_name: str = ""
     epilogue: ValueTransform | None = None
     kind: str = "compute"
 
     @property
     def tgmem_accesses(self) -> tuple[TgmemAccess, ...]:
-        shape = strided_scratch_shape(self.W)
+        shape = strided_scratch_shape(self.W, self.rows)
         return (TgmemAccess(self.scratch_name, "readwrite", shape[0] * shape[1], shape),)
 
     def render(self, ctx: CodegenContext) -> str:
         _check_op(self.op)
-        W, R = self.W, STRIDED_ROWS
+        W, R = self.W, self.rows
         T = 64 * W
-        J = T // STRIDED_GROUPS
+        J = T * R // STRIDED_LANES
         U = max(1, STRIDED_LOADS // J)  # chunks of T elements in flight
         ident = _identity(self.op)
         tf = self.value_transform or (lambda raw: raw)
@@ -302,15 +301,19 @@ class StridedReductionFragment(LastAxisReductionComputeFragment):
             f"                mt_acc[j] = {_combine(self.op, 'mt_acc[j]', tf('x[u][j]'))};",
             "            }",
             "    }",
-            f"    for (; e < {self.reduce_dim}; e += {T}u)",
+            f"    for (; e < {self.reduce_dim}; e += {T}u) {{  // the rest: all loads of a chunk, then its sums",
+            f"        float x[{J}];",
             "#pragma unroll",
             f"        for (int j = 0; j < {J}; ++j) {{",
             "            const unsigned idx = e + (unsigned)j;",
-            f"            if (idx < {self.reduce_dim}) {{",
-            f"                const float xv = {at};",
-            f"                mt_acc[j] = {_combine(self.op, 'mt_acc[j]', tf('xv'))};",
-            "            }",
+            f"            x[j] = idx < {self.reduce_dim} ? {at} : 0.0f;",
             "        }",
+            "#pragma unroll",
+            f"        for (int j = 0; j < {J}; ++j) {{",
+            "            const unsigned idx = e + (unsigned)j;",
+            f"            if (idx < {self.reduce_dim}) mt_acc[j] = {_combine(self.op, 'mt_acc[j]', tf('x[j]'))};",
+            "        }",
+            "    }",
             "}",
             "#pragma unroll",
             f"for (int j = 0; j < {J}; ++j) {sc}[mt_g * {J}u + (unsigned)j][mt_r] = mt_acc[j];",
@@ -333,8 +336,8 @@ class StridedReductionFragment(LastAxisReductionComputeFragment):
         return "\n".join(lines)
 
 
-def strided_scratch_shape(waves_per_row: int) -> tuple[int, int]:
-    return (64 * waves_per_row, STRIDED_ROWS)
+def strided_scratch_shape(waves_per_row: int, rows: int) -> tuple[int, int]:
+    return (64 * waves_per_row, rows)
 
 
 @dataclass(frozen=True)

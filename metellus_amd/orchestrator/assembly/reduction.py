@@ -43,17 +43,36 @@ def reduction_waves_per_row(M: int, K: int) -> int:
     return W
 
 
+# A reduction of side-by-side rows from so many of them on, or of rows up to so
+# long: fewer and longer ones are a few workgroups, and a wave per row keeps more
+# loads in flight.  Measured on MI355X, this way against a wave per row: 256 rows of
+# 4096 6 against 9 us, 70 of 4096 6.8 against 6.2, 64 of 8192 8 against 10.5, 192 of
+# 16384 24 against 22, 32 of 65536 70 against 52, 320 of 65536 156 against 186.
+STRIDED_MIN_ROWS = 320
+STRIDED_MAX_LENGTH = 5120
+
+
 def strided_rows(src: Tensor) -> bool:
     """Rows lying side by side in memory (the columns of a row-major matrix), at
-    least a workgroup of them and a wave's 64 elements each: 32 lanes then load
-    128 contiguous bytes where a wave per row loads 64 cache lines."""
+    least 32 of them and a wave's 64 elements each: the lanes of a workgroup then
+    load contiguous bytes where a wave per row loads 64 cache lines."""
     M, K = src.shape
-    return src.row_stride == 1 and src.col_stride != 1 and M >= _red.STRIDED_ROWS and K >= 64
+    if src.row_stride != 1 or src.col_stride == 1 or M < 32 or K < 64:
+        return False
+    return M >= STRIDED_MIN_ROWS or K <= STRIDED_MAX_LENGTH
+
+
+def strided_rows_per_group(M: int) -> int:
+    """32 rows fill a 128-byte line; fewer where that leaves compute units without a
+    workgroup (1000 rows of 16384: 40 us with 32 rows, 31 with 16, 38 with 8; 3001
+    of 3000: 15, 18, 27; 70 of 5000: 15, 12, 9.6)."""
+    return 8 if M < 128 else 16 if M < 2560 else 32
 
 
 def _assemble_strided(decision: DecisionView, function_name: str | None, src: Tensor, final_out: Tensor,
                       extras: Extras, helpers: list[str], prologue, epilogue, M: int, K: int, W: int) -> KernelGroup:
     anchor = decision.anchor
+    rows = strided_rows_per_group(M)
     frag = StridedReductionFragment(
         op=anchor.op,
         input_name=param_name(src.buffer_key),
@@ -66,6 +85,7 @@ def _assemble_strided(decision: DecisionView, function_name: str | None, src: Te
         value_transform=prologue,
         waves_per_row=W,
         vectorized=False,
+        rows=rows,
         out_name=param_name(final_out.buffer_key),
         epilogue=epilogue,
     )
@@ -75,14 +95,14 @@ def _assemble_strided(decision: DecisionView, function_name: str | None, src: Te
         dims=("M", "K"),
         tg_x=_red.STRIDED_LANES,
         tg_y=1,
-        threadgroup_decls=(lds_decl("scratch", strided_scratch_shape(W)),),
+        threadgroup_decls=(lds_decl("scratch", strided_scratch_shape(W, rows)),),
         helpers=tuple(helpers),
     )
     return KernelGroup(
         kernel=Kernel(fragments=(frag,), ctx=ctx),
         bindings=(src.buffer_key, final_out.buffer_key, *extras.bindings),
         dims=(M, K),
-        grid=((M + _red.STRIDED_ROWS - 1) // _red.STRIDED_ROWS, 1, 1),
+        grid=((M + rows - 1) // rows, 1, 1),
         threads=(_red.STRIDED_LANES, 1, 1),
         ops=decision.ops,
         strategy=decision.strategy,

@@ -286,3 +286,21 @@ def test_asm_stores_keep_their_data_registers():
     stores = re.findall(r'asm volatile\(\s*"((?:global|buffer)_store[^"]*)"', src)
     assert len(stores) >= 3, stores
     assert all(st.endswith("\\n\\ts_nop 1") for st in stores), stores
+
+
+@pytest.mark.parametrize(
+    "M,K,groups",
+    [(31, 64, 0), (32, 64, 4), (127, 4096, 16), (128, 4096, 8), (319, 5120, 20), (319, 5121, 0), (32, 1 << 20, 0),
+     (320, 1 << 20, 20), (2559, 64, 160), (2560, 64, 80)],
+)
+def test_reductions_of_side_by_side_rows(M, K, groups):
+    """Column sums: a workgroup takes 8, 16 or 32 columns; few long ones (and
+    fewer than 32) keep a wave each."""
+    ops = Operations()
+    ops.input("X", (K, M))
+    ops.transpose("X", out="Xt")
+    ops.reduction("sum", out="r", x="Xt")
+    (g,) = compile_program(ops)
+    assert ("mt_acc[" in g.kernel.source.split('extern "C"')[-1]) == (groups > 0)
+    if groups:
+        assert g.grid == (groups, 1, 1) and g.threads == (512, 1, 1)
