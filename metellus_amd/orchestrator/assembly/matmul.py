@@ -536,6 +536,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         aligned = is_aligned_shape(M, K, N, tile)
     if not aligned and K <= SHORT_K and (tile.tile_M, tile.tile_N) == (256, 256) and _config.FORCE_TILE is None:
         tile = b_tile_for(SHORT_K_TILE, src_b)
+        aligned = is_aligned_shape(M, K, N, tile)
     if decision.reduction is not None and (tile.tile_N, tile.sg_M, tile.sg_N) == (256, 4, 4):
         # each wave reduces its rows over its own columns: 2x8 waves leave
         # half as many rows to every wave's lane exchanges

@@ -304,3 +304,15 @@ def test_reductions_of_side_by_side_rows(M, K, groups):
     assert ("mt_acc[" in g.kernel.source.split('extern "C"')[-1]) == (groups > 0)
     if groups:
         assert g.grid == (groups, 1, 1) and g.threads == (512, 1, 1)
+
+
+@pytest.mark.parametrize("M,K,N", [(17920, 512, 1152), (8192, 256, 4224)])
+def test_short_products_that_divide_into_256x128_tiles_need_no_bounds(M, K, N):
+    """Ragged for 256x256 tiles, whole for the ones they take: direct-to-LDS loads."""
+    ops = Operations()
+    ops.input("A", (M, K))
+    ops.input("B", (K, N))
+    ops.matmul(a="A", b="B", out="C")
+    (g,) = compile_program(ops)
+    body = g.kernel.source.split('extern "C"')[-1]
+    assert "mt_tile_dma<" in body and "tile_m0 + wave_m0 < M" not in body
