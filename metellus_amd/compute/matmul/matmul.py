@@ -573,8 +573,8 @@ class MatmulExactRetryFragment:
         top_a = self._largest(self.a, (m0, f"{m0} + {rows}"), (kb, ke))
         top_b = self._largest(self.b, (kb, ke), (n0, f"{n0} + {cols}"))
         lines = [
-            f"if (mt_mfma_retry<{t.WM}, {t.WN}>({acc}, mt_cut{self.accumulator_suffix}, {k}, {rows}, {cols}, lane, "
-            f"{top_a}, {top_b})) {{",
+            f"if (__builtin_expect(mt_mfma_retry<{t.WM}, {t.WN}>({acc}, mt_cut{self.accumulator_suffix}, {k}, {rows}, {cols}, lane, "
+            f"{top_a}, {top_b}), 0)) {{",
             *["    " + x for x in self._operand("mt_fa", self.a, "a", c.M_dim_var, ke)],
             *["    " + x for x in self._operand("mt_fb", self.b, "b", c.N_dim_var, ke)],
             f"    mt_mfma_exact<{t.WM}, {t.WN}>(mt_fa, mt_fb, tile_m0 + wave_m0, tile_n0 + wave_n0, {kb}, {ke}, lane, {acc});",
@@ -909,8 +909,8 @@ class MatmulRowWavesFragment:
         top_a = f"mt_largest({a}, {self.a_row_stride}u, mt_m0, mt_m0 + 32u, 0u, K, lane)" if pro is None else "__builtin_inff()"
         lines += [
             "mt_cut.b = __syncthreads_or(mt_cut.b != 0ull ? 1 : 0) != 0 ? 1ull : 0ull;  // any lane's share of B",
-            "if (mt_mfma_retry<1, 2>(acc, mt_cut, K, 32u, 64u, lane, "
-            f"[&] {{ return {top_a}; }}, [&] {{ return mt_largest({b}, {self.b_row_stride}u, 0u, K, mt_n0, mt_n0 + 64u, lane); }})) {{",
+            "if (__builtin_expect(mt_mfma_retry<1, 2>(acc, mt_cut, K, 32u, 64u, lane, "
+            f"[&] {{ return {top_a}; }}, [&] {{ return mt_largest({b}, {self.b_row_stride}u, 0u, K, mt_n0, mt_n0 + 64u, lane); }}), 0)) {{",
             f"    const auto mt_fa = [&](unsigned r, unsigned k0) {{ return mt_exact_quad<true>({a}, {self.a_row_stride}u, 1u, r, k0, "
             "M, K, [&](float raw, unsigned) { return mt_pa(raw); }); };  // r is mt_row",
             f"    const auto mt_fb = [&](unsigned n, unsigned k0) {{ return mt_exact_quad<false>({b}, 1u, {self.b_row_stride}u, n, k0, "

@@ -1144,6 +1144,13 @@ MT_INLINE unsigned mt_acc_row(int v, unsigned lane) {
     return 8u * (unsigned)(v >> 2) + 4u * (lane >> 5) + (unsigned)(v & 3);
 }
 
+// The lane, as a value the compiler computes nothing from ahead of its use: what a
+// rare path needs of it must not take registers from the k loop before.
+MT_INLINE unsigned mt_late(unsigned lane) {
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // Largest magnitude of lines [l0, l1), elements [e0, e1) each, of a matrix whose
 // lines are contiguous and `pitch` apart: the whole wave, 4 lines of 64 elements a
 // load.
@@ -1151,6 +1158,7 @@ MT_INLINE float mt_largest(const float* __restrict__ src, size_t pitch, unsigned
                            unsigned e1, unsigned lane) {
     constexpr unsigned UNROLL = 8u;
     float top = 0.0f;
+    lane = mt_late(lane);
     for (unsigned e = e0 + 4u * (lane & 15u); e < e1; e += 64u)
         for (unsigned l = l0 + (lane >> 4); l < l1; l += 4u * UNROLL) {
             mt_f32x4 x[UNROLL];
@@ -1178,9 +1186,10 @@ template <int WM, int WN, typename TA, typename TB>
 MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN], const mt_lost& lost, unsigned K, unsigned rows,
                              unsigned cols, unsigned lane, TA ta, TB tb) {
     bool odd = false;
-    if ((lost.a | lost.b) != 0ull) {
+    if (__builtin_expect((lost.a | lost.b) != 0ull, 0)) {
         const float top = __builtin_fmaxf(lost.b != 0ull ? ta() : 0.0f, lost.a != 0ull ? tb() : 0.0f);
         const float least = 0x1.0p-107f * (float)K * top;  // 2^25 times what both may have lost
+        lane = mt_late(lane);
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -1199,7 +1208,7 @@ MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN], const mt_lost& lost
                 const float x = __builtin_fabsf(acc[i][j][v]);
                 odd |= !(x >= 0x1.0p-96f && x <= 0x1.fffffep+127f) && x != 0.0f;
             }
-    return __ballot(odd) != 0ull;
+    return __builtin_expect(__ballot(odd) != 0ull, 0);
 }
 
 // The wave's blocks at (m0, n0) over k in [kb, ke) again, with fp32 MFMAs on
@@ -1212,6 +1221,7 @@ MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN], const mt_lost& lost
 template <int WM, int WN, typename FA, typename FB>
 MT_INLINE void mt_mfma_exact(FA fa, FB fb, unsigned m0, unsigned n0, unsigned kb, unsigned ke, unsigned lane,
                              mt_f32x16 (&acc)[WM][WN]) {
+    lane = mt_late(lane);
     const unsigned li = lane & 31u, lh = lane >> 5;
 #pragma unroll
     for (int i = 0; i < WM; ++i)
