@@ -455,7 +455,11 @@ def exact_retry(config: MatmulConfig, src_a: Tensor, src_b: Tensor, pro_a: Chain
 # A 256x256 tile with bounds stores its 256 KiB after a short k loop with no
 # other workgroup on the unit to work meanwhile; two 256x128 ones overlap.
 # Measured on MI355X: 17872 x 64 x 1117 47.6 -> 39.0 us, 4000 x 333 x 7001 232.8 ->
-# 198.9 us; 2049 x 1111 x 3333 and longer k's are as fast or faster on 256x256.
+# 198.9 us; 2049 x 1111 x 3333 and longer k's are as fast or faster on 256x256, as
+# long as they are one round: the persistent loop with bounds spills (352 bytes a
+# lane), so several rounds take 256x128 tiles too (4095 x 4096 x 8192 1920 -> 1628
+# us, 3500 x 1500 x 5500 552 -> 487, 2600 x 700 x 8100 349 -> 297; 4001 x 600 x 8001,
+# two whole rounds, 362 -> 376).
 SHORT_K = 512
 SHORT_K_TILE = TileConfig(256, 128, 32, 4, 2)
 
@@ -534,7 +538,9 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         # 16-wave tiles only without bounds checks (their masks cost registers)
         tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b)
         aligned = is_aligned_shape(M, K, N, tile)
-    if not aligned and K <= SHORT_K and (tile.tile_M, tile.tile_N) == (256, 256) and _config.FORCE_TILE is None:
+    if not aligned and (tile.tile_M, tile.tile_N) == (256, 256) and _config.FORCE_TILE is None and (
+        K <= SHORT_K or (decision.reduction is None and persistent_workgroups(M, N, tile, batch) is not None)
+    ):
         tile = b_tile_for(SHORT_K_TILE, src_b)
         aligned = is_aligned_shape(M, K, N, tile)
     if decision.reduction is not None and (tile.tile_N, tile.sg_M, tile.sg_N) == (256, 4, 4):
