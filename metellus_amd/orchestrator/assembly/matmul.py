@@ -452,14 +452,13 @@ def exact_retry(config: MatmulConfig, src_a: Tensor, src_b: Tensor, pro_a: Chain
                                     accumulator_suffix=suffix, persistent=persistent, check=check)
 
 
-# A 256x256 tile with bounds stores its 256 KiB after a short k loop with no
-# other workgroup on the unit to work meanwhile; two 256x128 ones overlap.
-# Measured on MI355X: 17872 x 64 x 1117 47.6 -> 39.0 us, 4000 x 333 x 7001 232.8 ->
-# 198.9 us; 2049 x 1111 x 3333 and longer k's are as fast or faster on 256x256, as
-# long as they are one round: the persistent loop with bounds spills (352 bytes a
-# lane), so several rounds take 256x128 tiles too (4095 x 4096 x 8192 1920 -> 1628
-# us, 3500 x 1500 x 5500 552 -> 487, 2600 x 700 x 8100 349 -> 297; 4001 x 600 x 8001,
-# two whole rounds, 362 -> 376).
+# Several rounds of 256x256 tiles with bounds: each stores its 256 KiB with no other
+# workgroup on the unit to work meanwhile, and the persistent loop spills (352 bytes a
+# lane).  Two 256x128 workgroups a unit overlap.  Measured on MI355X: 17872 x 64 x 1117
+# 47.6 -> 39.0 us, 4000 x 333 x 7001 232.8 -> 198.9, 4095 x 4096 x 8192 1920 -> 1628,
+# 3500 x 1500 x 5500 552 -> 487 (4001 x 600 x 8001, two whole rounds, 362 -> 376).  One
+# round keeps its tiles: 1576 x 304 x 7121, 196 of them, 80 us against 113.  With a row
+# reduction, which wants few column tiles, only for short k loops.
 SHORT_K = 512
 SHORT_K_TILE = TileConfig(256, 128, 32, 4, 2)
 
@@ -538,8 +537,9 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         # 16-wave tiles only without bounds checks (their masks cost registers)
         tile = b_tile_for(select_tile_config(M, K, N, batch=batch), src_b)
         aligned = is_aligned_shape(M, K, N, tile)
-    if not aligned and (tile.tile_M, tile.tile_N) == (256, 256) and _config.FORCE_TILE is None and (
-        K <= SHORT_K or (decision.reduction is None and persistent_workgroups(M, N, tile, batch) is not None)
+    if (
+        not aligned and (tile.tile_M, tile.tile_N) == (256, 256) and _config.FORCE_TILE is None
+        and persistent_workgroups(M, N, tile, batch) is not None and (decision.reduction is None or K <= SHORT_K)
     ):
         tile = b_tile_for(SHORT_K_TILE, src_b)
         aligned = is_aligned_shape(M, K, N, tile)

@@ -316,3 +316,26 @@ def test_short_products_that_divide_into_256x128_tiles_need_no_bounds(M, K, N):
     (g,) = compile_program(ops)
     body = g.kernel.source.split('extern "C"')[-1]
     assert "mt_tile_dma<" in body and "tile_m0 + wave_m0 < M" not in body
+
+
+@pytest.mark.parametrize(
+    "M,K,N,tile,grid",
+    [
+        (1576, 304, 7121, (256, 256), (28, 7, 1)),  # ragged, one round of 256x256 tiles
+        (3500, 1500, 5500, (256, 128), None),  # ragged, more: persistent
+        (512, 256, 384, (32, 32), (12, 16, 1)),  # whole 32x32 tiles, three to four a unit
+        (256, 2048, 256, (32, 32), (128, 8, 1)),  # in 16 parts
+    ],
+)
+def test_tiles_of_plain_products(M, K, N, tile, grid):
+    ops = Operations()
+    ops.input("A", (M, K))
+    ops.input("B", (K, N))
+    ops.matmul(a="A", b="B", out="C")
+    (g,) = compile_program(ops)
+    body = g.kernel.source.split('extern "C"')[-1]
+    assert f"tile_m0 = tg.y * {tile[0]}u" in body and f"tile_n0 = tg.x * {tile[1]}u" in body
+    if grid is None:
+        assert "mt_t += gridDim.x" in body or "mt_sk" in body
+    else:
+        assert g.grid == grid
