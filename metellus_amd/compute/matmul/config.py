@@ -204,10 +204,14 @@ class FillTile:
     """A tile for problems whose best-scored tile leaves compute units idle, with
     what one 32-wide k-chunk of it costs on MI355X in microseconds: ``alone`` with
     at most one workgroup on every other compute unit, where it waits for its own
-    loads and barriers; ``base + each * n`` with n workgroups on every unit, but
-    not below ``shared * n``, the unit's rate.  ``registers``: factor when an operand goes through registers (no direct-to-LDS
-    loads).  Fitted to 10 shapes from 256^3 to 2048 x 4096 x 1024, every tile in 1
-    to 16 parts; the pick is within 10 % of the best of all measured ones."""
+    loads and barriers; ``base + each * n`` with n workgroups on every unit, but not
+    below ``shared * n``, the unit's rate.  ``registers``: factor when an operand of
+    sizes it divides, or of a product in parts, goes through registers (no
+    direct-to-LDS loads); ``odd``: the factors for other sizes (bounds, masked loads)
+    with up to one workgroup a unit and with more.  Fitted to 10 whole shapes from
+    256^3 to 2048 x 4096 x 1024, every tile in 1 to 16 parts (the pick within 10 % of
+    the best), and ``odd`` to 90 more of 65 to 4096 rows, 128 to 4096 k's and 64 to
+    8192 columns, where one wave of 32x32 is the worst off (2145 of them 37 us, 561 tiles of 64x64 26 us)."""
 
     tile: TileConfig
     alone: float
@@ -215,18 +219,19 @@ class FillTile:
     each: float
     registers: float = 1.05
     shared: float = 0.0
+    odd: tuple[float, float] = (1.0, 1.0)
 
 
 FILL_TILES = (
-    FillTile(TileConfig(256, 256, 32, 4, 4), 4.0, 0.0, 5.2, 1.4),
-    FillTile(TileConfig(256, 128, 32, 4, 4), 2.5, 0.2, 3.4, 1.1),
-    FillTile(TileConfig(128, 256, 32, 4, 4), 2.5, 0.2, 3.4, 1.1),
-    FillTile(TileConfig(128, 128, 32, 2, 2), 1.5, 0.25, 1.55, 1.1),
-    FillTile(TileConfig(128, 64, 32, 2, 2), 1.0, 0.3, 0.85),
-    FillTile(TileConfig(64, 128, 32, 2, 2), 1.0, 0.25, 0.83),
-    FillTile(TileConfig(64, 64, 32, 2, 2), 0.65, 0.3, 0.43, 1.25, shared=0.5),
-    FillTile(TileConfig(32, 64, 32, 1, 2), 0.5, 0.45, 0.165, shared=0.32),
-    FillTile(TileConfig(32, 32, 32, 1, 1), 0.5, 0.42, 0.07, shared=0.175),
+    FillTile(TileConfig(256, 256, 32, 4, 4), 4.0, 0.0, 5.2, 1.4, odd=(1.75, 1.5)),
+    FillTile(TileConfig(256, 128, 32, 4, 4), 2.5, 0.2, 3.4, 1.1, odd=(1.25, 1.0)),
+    FillTile(TileConfig(128, 256, 32, 4, 4), 2.5, 0.2, 3.4, 1.1, odd=(1.3, 1.0)),
+    FillTile(TileConfig(128, 128, 32, 2, 2), 1.5, 0.25, 1.55, 1.1, odd=(1.65, 1.15)),
+    FillTile(TileConfig(128, 64, 32, 2, 2), 1.0, 0.3, 0.85, odd=(1.65, 1.3)),
+    FillTile(TileConfig(64, 128, 32, 2, 2), 1.0, 0.25, 0.83, odd=(1.7, 1.2)),
+    FillTile(TileConfig(64, 64, 32, 2, 2), 0.65, 0.3, 0.43, 1.25, shared=0.5, odd=(1.55, 1.25)),
+    FillTile(TileConfig(32, 64, 32, 1, 2), 0.5, 0.45, 0.165, shared=0.32, odd=(2.1, 1.4)),
+    FillTile(TileConfig(32, 32, 32, 1, 1), 0.5, 0.42, 0.07, shared=0.175, odd=(2.25, 1.75)),
 )
 FILL_MAX_PARTS = 16
 # Products of fewer k's keep one sum in one order: as the product of a pair or
@@ -235,14 +240,15 @@ FILL_PARTS_MIN_K = 1024
 FILL_WORKSPACE = 64 << 20  # bytes of partial sums a split may need (both anchors' of a pair)
 
 
-def fill_time(tiles: int, chunks: int, parts: int, f: FillTile, registers: bool) -> float:
+def fill_time(tiles: int, chunks: int, parts: int, f: FillTile, slow: tuple[float, float] = (1.0, 1.0)) -> float:
     """Microseconds of ``tiles`` tiles in ``parts`` parts each: the chunks the
-    busiest compute unit walks, and for a split the partial sums (5 TB/s out, and
-    the last workgroup reads its tile's at about 80 GB/s; 2 us to meet)."""
+    busiest compute unit walks (``slow``: factors with up to one workgroup a unit and
+    with more), and for a split the partial sums (5 TB/s out, and the last workgroup
+    reads its tile's at about 80 GB/s; 2 us to meet)."""
     groups = tiles * parts
     n = ceil_div(groups, NUM_CUS)
     chunk = f.alone if 2 * groups <= NUM_CUS else max(f.base + f.each * n, f.shared * n)
-    time = ceil_div(chunks, parts) * chunk * (f.registers if registers else 1.0)
+    time = ceil_div(chunks, parts) * chunk * slow[n > 1]
     if parts == 1:
         return time
     tile_bytes = 4 * f.tile.tile_M * f.tile.tile_N
@@ -271,7 +277,7 @@ def filled_parts(M: int, K: int, N: int, batch: int = 1) -> int:
                 or 2 * tiles * parts * t.tile_M * t.tile_N * 4 > FILL_WORKSPACE
             ):
                 break
-            best = min(best, (fill_time(batch * tiles, chunks, parts, f, False), parts))
+            best = min(best, (fill_time(batch * tiles, chunks, parts, f), parts))
     return best[1]
 
 
@@ -290,7 +296,9 @@ def select_filled(M: int, K: int, N: int, batch: int = 1, splittable: bool = Tru
         if parts > 1 and (tiles >= STREAM_K_MAX_WORKGROUPS
                           or anchors * tiles * parts * t.tile_M * t.tile_N * 4 > FILL_WORKSPACE):
             return float("inf")
-        return fill_time(batch * tiles, chunks, parts, f, registers)
+        whole = parts > 1 or is_aligned_shape(M, K, N, t)
+        slow = f.odd if not whole else (f.registers, f.registers) if registers else (1.0, 1.0)
+        return fill_time(batch * tiles, chunks, parts, f, slow)
 
     return min(_fill_candidates(M, N, min_waves, anchors), key=time).tile, parts
 

@@ -323,6 +323,8 @@ def test_short_products_that_divide_into_256x128_tiles_need_no_bounds(M, K, N):
     [
         (1576, 304, 7121, (256, 256), (28, 7, 1)),  # ragged, one round of 256x256 tiles
         (3500, 1500, 5500, (256, 128), None),  # ragged, more: persistent
+        (950, 427, 2296, (64, 64), (36, 15, 1)),  # ragged for every tile: no one-wave tiles by the thousand
+        (3000, 900, 700, (64, 64), (11, 47, 1)),
         (512, 256, 384, (32, 32), (12, 16, 1)),  # whole 32x32 tiles, three to four a unit
         (256, 2048, 256, (32, 32), (128, 8, 1)),  # in 16 parts
     ],
