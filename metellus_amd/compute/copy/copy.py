@@ -12,9 +12,10 @@ transposed views and other irregular strides.  Two forms:
   ``ld``), i.e. a transposed view: tiles staged through LDS, read along the
   source's contiguous axis and written along the output's, both coalesced;
   128-bit nontemporal loads and device-scope stores: aligned when the sizes
-  and ``ld`` are multiples of 4, at any element address otherwise (4099x3001
-  35.6 -> 22.4 us, 14110x1024 40 -> 24.7 us against one element per lane;
-  ordinary loads and stores 24.0 and 29.6 us), one element per lane for small
+  and ``ld`` are multiples of 4, at any element address otherwise (out of HBM,
+  buffers larger than the caches taken in turn: 4099x3001 37.1 -> 31.0 us,
+  14110x1024 41.9 -> 33.5, 2001x16000 82.0 -> 74.9 against one element per lane;
+  ordinary loads and stores 30.7, 34.9 and 78.9), one element per lane for small
   odd ones.  Measured on
   MI355X, a transposed 4096x4096 view (64 MiB each way): 79.3 us with one
   lane per output element gathering through the strides, 35.1 us with
