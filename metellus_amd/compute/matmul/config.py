@@ -228,8 +228,8 @@ FILL_TILES = (
     FillTile(TileConfig(128, 256, 32, 4, 4), 2.5, 0.2, 3.4, 1.1, odd=(1.3, 1.0)),
     FillTile(TileConfig(128, 128, 32, 2, 2), 1.5, 0.25, 1.55, 1.1, odd=(1.65, 1.15)),
     FillTile(TileConfig(128, 64, 32, 2, 2), 1.0, 0.3, 0.85, odd=(1.65, 1.3)),
-    FillTile(TileConfig(64, 128, 32, 2, 2), 1.0, 0.25, 0.83, odd=(1.7, 1.2)),
-    FillTile(TileConfig(64, 64, 32, 2, 2), 0.65, 0.3, 0.43, 1.25, shared=0.5, odd=(1.55, 1.25)),
+    FillTile(TileConfig(64, 128, 32, 2, 2), 1.0, 0.25, 0.83, odd=(1.7, 1.15)),
+    FillTile(TileConfig(64, 64, 32, 2, 2), 0.65, 0.3, 0.43, 1.25, shared=0.5, odd=(1.55, 1.3)),
     FillTile(TileConfig(32, 64, 32, 1, 2), 0.5, 0.45, 0.165, shared=0.32, odd=(2.1, 1.4)),
     FillTile(TileConfig(32, 32, 32, 1, 1), 0.5, 0.42, 0.07, shared=0.175, odd=(2.25, 1.75)),
 )

@@ -40,6 +40,9 @@ class MatmulConfig:
     b_tile_name: str
     c_tile_name: str = "C_tile"
     c_col_stride: str = "1"
+    # a split mainloop's waves may look at what is lost for each other
+    # (``looking_wave``)
+    look_together: bool = True
 
     def validate(self) -> None:
         self.tile.validate()
@@ -404,24 +407,58 @@ class ThreadIndexFragment:
         return ()
 
 
+def cut_words(first: str | None = None) -> list[str]:
+    """The LDS words of ``mt_cut``, zeroed by the first wave if the code ``first``
+    holds; a barrier follows before the first split."""
+    guard = f"{first} && threadIdx.x < 32u" if first else "threadIdx.x < 32u"
+    return ["__shared__ unsigned mt_cut_words[32];", f"if ({guard}) mt_cut_words[threadIdx.x] = 0u;"]
+
+
+def cut_of(tile: TileConfig, look: str) -> str:
+    """This wave's ``mt_cut``: the words of its row and its column of waves."""
+    n = tile.sg_N
+    return f"mt_cut<{look}>{{&mt_cut_words[wave / {n}u], &mt_cut_words[16u + wave % {n}u]}}"
+
+
+def looking_wave(config: MatmulConfig) -> str | None:
+    """Code: whether this wave looks at what its splits lose, one in every row and
+    every column of waves and as many on each SIMD (the k loop is instantiated for
+    both kinds, every barrier in both): 4096^3 698 -> 676 us, 668 without the look.
+    None: each for itself.  With loads through registers, which both would keep,
+    (h1*s*h2) @ W3 spills (MLP block 6.15 against 6.94 ms), 2049 x 1111 x 3333 takes
+    137 against 160 us; a persistent loop of 16 waves, out of registers with one
+    instance, 1993 against 2040 us (4096 x 4096 x 11008)."""
+    tile = config.tile
+    m, n = tile.sg_M, tile.sg_N
+    if not config.look_together or min(m, n) == 1 or "pad" in (tile.a_layout, tile.b_layout) or tile.stages != 2:
+        return None
+    if n >= m:
+        return f"wave % {n}u % {m}u == wave / {n}u"
+    return f"wave % {n}u == wave / {n * (m // n)}u"
+
+
 @dataclass(frozen=True)
 class MatmulSetupFragment:
-    """Zeroed accumulators ``acc{suffix}[WM][WN]``, and for a split mainloop what
-    its splits cut off (``mt_cut{suffix}``)."""
+    """Zeroed accumulators ``acc{suffix}[WM][WN]``; ``split``: and the note of what a
+    split mainloop's splits lost (the workgroup's is kept over ``persistent`` tiles)."""
 
     config: MatmulConfig
     accumulator_suffix: str = ""
     emit_thread_coords: bool = True
     split: bool = False
+    persistent: bool = False
     name: str = "matmul_setup"
     kind: str = "setup"
 
     def render(self, ctx: CodegenContext) -> str:
         t = self.config.tile
         a = f"acc{self.accumulator_suffix}"
+        note = []
+        if self.split:
+            note = cut_words("mt_first_tile" if self.persistent else None) if looking_wave(self.config) else ["mt_lost mt_own_lost = {};"]
         return "\n".join(
             [
-                *([f"mt_lost mt_cut{self.accumulator_suffix} = {{}};"] if self.split else ()),
+                *note,
                 f"mt_f32x16 {a}[{t.WM}][{t.WN}];",
                 "#pragma unroll",
                 f"for (int i = 0; i < {t.WM}; ++i)",
@@ -483,12 +520,12 @@ class MatmulComputeFragment:
                 raise ValueError("a held group and a load hook do not combine")
             return (
                 f"mt_mfma_tile_held<{t.WM}, {t.WN}, {t.tile_K}, {t.lda}, {t.ldb}{flags}>"
-                f"({a_ptr}, {b_ptr}, mt_cut{sfx}, acc{sfx}, lane, {held[0]}, {held[1]});"
+                f"({a_ptr}, {b_ptr}, mt_notes, acc{sfx}, lane, {held[0]}, {held[1]});"
             )
         hook_arg = f", {hook}" if hook is not None else ""
         return (
             f"mt_mfma_tile<{t.WM}, {t.WN}, {t.tile_K}, {t.lda}, {t.ldb}{flags}>"
-            f"({a_ptr}, {b_ptr}, mt_cut{sfx}, acc{sfx}, lane{hook_arg});"
+            f"({a_ptr}, {b_ptr}, mt_notes, acc{sfx}, lane{hook_arg});"
         )
 
     def render_held_decl(self, var: str) -> str:
@@ -572,8 +609,9 @@ class MatmulExactRetryFragment:
             rows, cols = f"min({rows}, {t.wave_M}u)", f"min({cols}, {t.wave_N}u)"
         top_a = self._largest(self.a, (m0, f"{m0} + {rows}"), (kb, ke))
         top_b = self._largest(self.b, (kb, ke), (n0, f"{n0} + {cols}"))
+        lost = f"{cut_of(t, 'true')}.told()" if looking_wave(self.config) else "mt_own_lost"
         lines = [
-            f"if (__builtin_expect(mt_mfma_retry<{t.WM}, {t.WN}>({acc}, mt_cut{self.accumulator_suffix}, {k}, {rows}, {cols}, lane, "
+            f"if (__builtin_expect(mt_mfma_retry<{t.WM}, {t.WN}>({acc}, {lost}, {k}, {rows}, {cols}, lane, "
             f"{top_a}, {top_b}), 0)) {{",
             *["    " + x for x in self._operand("mt_fa", self.a, "a", c.M_dim_var, ke)],
             *["    " + x for x in self._operand("mt_fb", self.b, "b", c.N_dim_var, ke)],
@@ -654,6 +692,8 @@ class MatmulMainloopFragment:
         if stages == 1 and any(getattr(ld, "is_dma", False) for ld in loads):
             raise ValueError("direct-to-LDS loads need double-buffered LDS tiles")
         if stages == 1:
+            if computes and computes[0].split:
+                body.append("const mt_own mt_notes = {mt_own_lost};")
             body += [
                 f"for (unsigned k_chunk = 0; k_chunk < {kvar}; k_chunk += {tk}u) {{",
                 *[f"    {ld.render_fetch()}" for ld in loads],
@@ -675,7 +715,7 @@ class MatmulMainloopFragment:
         plain_lds = [ld for ld in loads if getattr(ld, "plain_invariant", False)]
 
         def loop(plain: bool | None) -> list[str]:
-            return [
+            return self._looking(computes, [
                 *[c.render_held_decl(f"mt_held{i}") for i, c in enumerate(computes) if held],
                 "for (unsigned kt = 0; kt < n_chunks; ++kt) {",
                 "    const unsigned cur = kt & 1u;",
@@ -688,7 +728,7 @@ class MatmulMainloopFragment:
                 *[f"    {x}" for x in sync],
                 "}",
                 *self._held_flush(computes, held),
-            ]
+            ])
 
         body += [
             f"const unsigned n_chunks = ({kvar} + {tk - 1}u) / {tk}u;",
@@ -730,6 +770,22 @@ class MatmulMainloopFragment:
             return [f"    {c.render_stage('cur', held=(f'mt_held{i}', f'kt > {k_begin}'))}"
                     for i, c in enumerate(computes)]
         return [f"    {c.render_stage('cur', 'mt_hook' if spread and i == 0 else None)}" for i, c in enumerate(computes)]
+
+    @staticmethod
+    def _looking(computes, loop: list[str]) -> list[str]:
+        """The k loop of split computes with its ``mt_notes`` (``looking_wave``)."""
+        if not computes or not computes[0].split:
+            return loop
+        tile = computes[0].config.tile
+        look = looking_wave(computes[0].config)
+        if look is None:
+            return ["const mt_own mt_notes = {mt_own_lost};", *loop]
+        return [
+            "const auto mt_k_loop = [&](const auto mt_notes) __attribute__((always_inline)) {",
+            *[f"    {x}" for x in loop],
+            "};",
+            f"if ({look}) mt_k_loop({cut_of(tile, 'true')}); else mt_k_loop({cut_of(tile, 'false')});",
+        ]
 
     @staticmethod
     def _held_flush(computes, held: bool) -> list[str]:
@@ -785,18 +841,20 @@ class MatmulMainloopFragment:
             *[f"    {c}" for c in _nonempty(ld.render_commit("mt_stage") for ld in loads)],
             *[f"    {x}" for x in sync],
             "}",
-            *[c.render_held_decl(f"mt_held{i}") for i, c in enumerate(computes) if held],
-            "for (unsigned kt = mt_kb; kt < mt_ke; ++kt) {",
-            "    const unsigned cur = mt_stage;",
-            "    const bool more = kt + 1u < mt_ke;",
-            *self._next_loads(loads, spread, persistent=True),
-            *self._computes_lines(computes, spread, held, "mt_kb"),
-            *_guarded("    if (more || mt_has_next) {",
-                      [f"        {c}" for c in _nonempty(ld.render_commit("cur ^ 1u") for ld in loads)]),
-            *[f"    {x}" for x in sync],
-            "    mt_stage ^= 1u;",
-            "}",
-            *self._held_flush(computes, held),
+            *self._looking(computes, [
+                *[c.render_held_decl(f"mt_held{i}") for i, c in enumerate(computes) if held],
+                "for (unsigned kt = mt_kb; kt < mt_ke; ++kt) {",
+                "    const unsigned cur = mt_stage;",
+                "    const bool more = kt + 1u < mt_ke;",
+                *self._next_loads(loads, spread, persistent=True),
+                *self._computes_lines(computes, spread, held, "mt_kb"),
+                *_guarded("    if (more || mt_has_next) {",
+                          [f"        {c}" for c in _nonempty(ld.render_commit("cur ^ 1u") for ld in loads)]),
+                *[f"    {x}" for x in sync],
+                "    mt_stage ^= 1u;",
+                "}",
+                *self._held_flush(computes, held),
+            ]),
         ]
         return "{\n" + textwrap.indent("\n".join(body), "    ") + "\n}"
 
@@ -847,16 +905,20 @@ class MatmulRowWavesFragment:
             return [
                 f"    if ({more}) ld_B.fetch({b}, {brs}u, (kt + {ahead}u) * 64u, threadIdx.x);",
                 f"    mt_rw_chunk(mt_a, mt_arow, (kt + {ahead}u) * 64u, {more}, &B_tile[{stage}][0][0], "
-                f"&B_low[{stage}][0][0], mt_n0, {pa}, lane, mt_cut, acc);",
-                f"    if ({more}) ld_B.commit(&B_tile[{stage ^ 1}][0][0], &B_low[{stage ^ 1}][0][0], threadIdx.x, mt_cut);",
+                f"&B_low[{stage}][0][0], mt_n0, {pa}, lane, mt_notes, acc);",
+                f"    if ({more}) ld_B.commit(&B_tile[{stage ^ 1}][0][0], &B_low[{stage ^ 1}][0][0], threadIdx.x, mt_told);",
                 "    __syncthreads();",
             ]
 
+        # two waves share rows of A: one of them looks, as many on each SIMD
         return [
-            "for (unsigned kt = 0; kt < n_chunks; kt += 2u) {",
-            *chunk(0, 1, "true"),
-            *chunk(1, 2, "kt + 2u < n_chunks"),
-            "}",
+            "const auto mt_k_loop = [&](const auto mt_notes) __attribute__((always_inline)) {",
+            "    for (unsigned kt = 0; kt < n_chunks; kt += 2u) {",
+            *[f"    {x}" for x in (*chunk(0, 1, "true"), *chunk(1, 2, "kt + 2u < n_chunks"))],
+            "    }",
+            "};",
+            "if ((wave & 1u) == (wave >> 2 & 1u)) mt_k_loop(mt_told);",
+            "else mt_k_loop(mt_cut<false>{mt_told.a, mt_told.b});",
         ]
 
     def render(self, ctx: CodegenContext) -> str:
@@ -868,7 +930,6 @@ class MatmulRowWavesFragment:
             "const unsigned mt_m0 = blockIdx.y * 256u + (wave >> 1) * 32u;",
             "const unsigned mt_n0 = (wave & 1u) * 64u;",
             "const unsigned mt_row = mt_m0 + (lane & 31u);",
-            "mt_lost mt_cut = {};",
             "mt_f32x16 acc[1][2];",
             "mt_zero(acc[0][0]);",
             "mt_zero(acc[0][1]);",
@@ -895,7 +956,10 @@ class MatmulRowWavesFragment:
             f"ld_B.fetch({b}, {self.b_row_stride}u, 0u, threadIdx.x);",
             "#pragma unroll",
             "for (int s = 0; s < 4; ++s) mt_rw_load(mt_a[s], mt_arow, 0u, s);",
-            "ld_B.commit(&B_tile[0][0][0], &B_low[0][0][0], threadIdx.x, mt_cut);",
+            *cut_words(),
+            "const mt_cut<true> mt_told = {&mt_cut_words[wave >> 1], &mt_cut_words[16]};",
+            "__syncthreads();",
+            "ld_B.commit(&B_tile[0][0][0], &B_low[0][0][0], threadIdx.x, mt_told);",
             "__syncthreads();",
             "const unsigned n_chunks = K / 64u;",
         ]
@@ -908,8 +972,7 @@ class MatmulRowWavesFragment:
         value = self.value_expr.format(a0="acc[0][j][v]") if self.value_expr else "acc[0][j][v]"
         top_a = f"mt_largest({a}, {self.a_row_stride}u, mt_m0, mt_m0 + 32u, 0u, K, lane)" if pro is None else "__builtin_inff()"
         lines += [
-            "mt_cut.b = __syncthreads_or(mt_cut.b != 0ull ? 1 : 0) != 0 ? 1ull : 0ull;  // any lane's share of B",
-            "if (__builtin_expect(mt_mfma_retry<1, 2>(acc, mt_cut, K, 32u, 64u, lane, "
+            "if (__builtin_expect(mt_mfma_retry<1, 2>(acc, mt_told.told(), K, 32u, 64u, lane, "
             f"[&] {{ return {top_a}; }}, [&] {{ return mt_largest({b}, {self.b_row_stride}u, 0u, K, mt_n0, mt_n0 + 64u, lane); }}), 0)) {{",
             f"    const auto mt_fa = [&](unsigned r, unsigned k0) {{ return mt_exact_quad<true>({a}, {self.a_row_stride}u, 1u, r, k0, "
             "M, K, [&](float raw, unsigned) { return mt_pa(raw); }); };  // r is mt_row",

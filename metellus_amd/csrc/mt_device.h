@@ -993,11 +993,14 @@ MT_INLINE void mt_mfma_tile_f32(const float* __restrict__ As, const float* __res
 // their results.  And an x below 2^-110 may have bits below 2^-133, bf16's
 // smallest number (the MFMAs keep subnormals): the third part cuts them off, an
 // error of up to 2^-133 times whatever the other operand is.  Results do not show
-// that, so every split says whether it cut anything off (mt_lost): half a VALU
-// operation per element.  Measured on MI355X without and with it: 4096^3 674 -> 696
-// us, 1531 x 1000 x 3001 96 -> 103 us, C4 MLP 5.88 -> 6.07 ms.  Dearer were a
-// running minimum and maximum of the operands held by every wave (4096^3 737 us),
-// or taken by every lane of its share of the LDS tile (742 us).
+// that, so a split says whether it cut anything off (mt_lost): half a VALU operation
+// per element, in every wave or in one of each row and column of waves (mt_own,
+// mt_cut).  Measured on MI355X without and with it: 4096^3 686 -> 699 us, 4096 x
+// 4096 x 11008 1874 -> 1979, 1531 x 1000 x 3001 98 -> 104, C4 MLP 5.92 -> 6.04 ms.
+// Dearer were a running minimum and maximum of the operands held by every wave
+// (4096^3 737 us where the look in every wave took 712), or taken by every lane of
+// its share of the LDS tile (742), or a look at every fourth chunk branched to inside
+// the asm of the split (691, but 2252 instead of 2103 for 4096 x 4096 x 8191).
 // ---------------------------------------------------------------------------
 
 typedef __bf16 mt_bf16x8 __attribute__((ext_vector_type(8)));
@@ -1022,6 +1025,38 @@ struct mt_lost {
     unsigned long long a, b;
 };
 
+// A wave's note of what its own splits lost.
+struct mt_own {
+    static constexpr bool LOOK = true;
+    mt_lost& lost;
+
+    MT_INLINE mt_lost& open(mt_lost&) const { return lost; }
+    MT_INLINE void tell(const mt_lost&) const {}
+};
+
+// Or the workgroup's: words in LDS, one for the waves that split the same rows of A
+// and one for those that split the same columns of B, zeroed before the k loop and
+// read after it.  One wave of each row and column of waves looks, the same one
+// through the loop.
+template <bool WAVE_LOOKS>
+struct mt_cut {
+    static constexpr bool LOOK = WAVE_LOOKS;
+    unsigned* a;
+    unsigned* b;
+
+    MT_INLINE mt_lost& open(mt_lost& chunk) const { return chunk; }
+    MT_INLINE void tell(const mt_lost& lost) const {
+        if constexpr (LOOK) {
+            if (__builtin_expect(lost.a != 0ull, 0)) *a = 1u;
+            if (__builtin_expect(lost.b != 0ull, 0)) *b = 1u;
+        }
+    }
+    MT_INLINE mt_lost told() const {
+        return {(unsigned)__builtin_amdgcn_readfirstlane(*a), (unsigned)__builtin_amdgcn_readfirstlane(*b)};
+    }
+};
+
+template <bool LOOK>
 MT_INLINE mt_split8 mt_split(mt_f32x4 u, mt_f32x4 v, unsigned long long& lost) {
     mt_split8 o;
     unsigned low = 0u;
@@ -1035,9 +1070,9 @@ MT_INLINE mt_split8 mt_split(mt_f32x4 u, mt_f32x4 v, unsigned long long& lost) {
         o.p2[q] = m;
         const float z0 = r0 - __builtin_bit_cast(float, m << 16), z1 = r1 - mt_keep_hi16(m);
         o.p3[q] = mt_pack_hi16(z0, z1);
-        low |= __builtin_bit_cast(unsigned, z0) | __builtin_bit_cast(unsigned, z1);
+        if constexpr (LOOK) low |= __builtin_bit_cast(unsigned, z0) | __builtin_bit_cast(unsigned, z1);
     }
-    lost |= __ballot((low & 0xffffu) != 0u);
+    if constexpr (LOOK) lost |= __ballot((low & 0xffffu) != 0u);
     return o;
 }
 
@@ -1060,10 +1095,10 @@ MT_INLINE mt_f32x16 mt_mfma_parts(const mt_split8& a, const mt_split8& b, mt_f32
 // b[j] column block j's parts.  Product by product over the column blocks, so
 // an MFMA does not wait for the one before it (C4 X @ W1: 1840 us; block by
 // block 1924 us).
-template <int WN>
+template <int WN, bool LOOK>
 MT_INLINE void mt_mfma_split(mt_f32x4 a0, mt_f32x4 a1, const mt_split8 (&b)[WN], unsigned long long& lost,
                              mt_f32x16 (&acc)[WN]) {
-    const mt_split8 a = mt_split(a0, a1, lost);
+    const mt_split8 a = mt_split<LOOK>(a0, a1, lost);
 #pragma unroll
     for (int j = 0; j < WN; ++j) acc[j] = mt_mfma_bf16(a.p3, b[j].p1, acc[j]);
 #pragma unroll
@@ -1085,9 +1120,13 @@ struct mt_no_hook {
 };
 
 // The chunk in the layouts of mt_mfma_tile_f32.
-template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false, typename H = mt_no_hook>
-MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restrict__ Bs, mt_lost& lost,
+template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false, typename N,
+          typename H = mt_no_hook>
+MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restrict__ Bs, N notes,
                             mt_f32x16 (&acc)[WM][WN], unsigned lane, H hook = H{}) {
+    constexpr bool LOOK = N::LOOK;
+    mt_lost chunk = {};
+    mt_lost& lost = notes.open(chunk);
     static_assert(TK % 16 == 0, "TK must be a multiple of 16");
     static_assert(LDA % 4 == 0, "LDA must keep 16-byte alignment");
     static_assert(!ASWZ || LDA == TK, "a swizzled A tile is dense");
@@ -1110,12 +1149,12 @@ MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restric
         for (int j = 0; j < WN; ++j) {
             if constexpr (BNM) {
                 const float* row = b_base + j * 32 * TK;
-                b[j] = mt_split(mt_ld4(row + 4u * (slot0 ^ m)), mt_ld4(row + 4u * (slot1 ^ m)), lost.b);
+                b[j] = mt_split<LOOK>(mt_ld4(row + 4u * (slot0 ^ m)), mt_ld4(row + 4u * (slot1 ^ m)), lost.b);
             } else {
                 mt_f32x4 q[2];
 #pragma unroll
                 for (int ss = 0; ss < 8; ++ss) q[ss / 4][ss % 4] = b_base[(s0 + ss) * LDB + j * 32];
-                b[j] = mt_split(q[0], q[1], lost.b);
+                b[j] = mt_split<LOOK>(q[0], q[1], lost.b);
             }
         }
 #pragma unroll
@@ -1124,9 +1163,10 @@ MT_INLINE void mt_mfma_tile(const float* __restrict__ As, const float* __restric
             const float* row = a_base + i * 32 * LDA;
             const mt_f32x4 a0 = ASWZ ? mt_ld4(row + 4u * (slot0 ^ m)) : mt_ld4(row + s0);
             const mt_f32x4 a1 = ASWZ ? mt_ld4(row + 4u * (slot1 ^ m)) : mt_ld4(row + s0 + 4);
-            mt_mfma_split<WN>(a0, a1, b, lost.a, acc[i]);
+            mt_mfma_split<WN, LOOK>(a0, a1, b, lost.a, acc[i]);
         }
     }
+    notes.tell(lost);
     __builtin_amdgcn_s_setprio(0);
 }
 
@@ -1141,10 +1181,10 @@ struct mt_mfma_group {};
 template <int WM, int WN>
 MT_INLINE void mt_mfma_group_run(const mt_mfma_group<WM, WN>&, mt_f32x16 (&)[WM][WN]) {}
 
-template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false>
-MT_INLINE void mt_mfma_tile_held(const float* __restrict__ As, const float* __restrict__ Bs, mt_lost& lost,
+template <int WM, int WN, int TK, int LDA, int LDB, bool ASWZ = false, bool BNM = false, typename N>
+MT_INLINE void mt_mfma_tile_held(const float* __restrict__ As, const float* __restrict__ Bs, N notes,
                                  mt_f32x16 (&acc)[WM][WN], unsigned lane, mt_mfma_group<WM, WN>&, bool) {
-    mt_mfma_tile<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, lost, acc, lane);
+    mt_mfma_tile<WM, WN, TK, LDA, LDB, ASWZ, BNM>(As, Bs, notes, acc, lane);
 }
 
 // Row (within a 32x32 output block) of accumulator register v held by `lane`;
@@ -1308,11 +1348,13 @@ struct mt_rw_stage {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = p[(size_t)e * ldb];
     }
-    MT_INLINE void commit(float* hi, float* lo, unsigned tid, mt_lost& lost) const {
-        const mt_split8 x = mt_split(mt_f32x4{v[0], v[1], v[2], v[3]}, mt_f32x4{v[4], v[5], v[6], v[7]}, lost.b);
+    MT_INLINE void commit(float* hi, float* lo, unsigned tid, mt_cut<true> cut) const {
+        mt_lost lost = {};
+        const mt_split8 x = mt_split<true>(mt_f32x4{v[0], v[1], v[2], v[3]}, mt_f32x4{v[4], v[5], v[6], v[7]}, lost.b);
         reinterpret_cast<mt_u32x4*>(hi)[tid] = x.p1;
         reinterpret_cast<mt_u32x4*>(hi)[1024u + tid] = x.p2;
         reinterpret_cast<mt_u32x4*>(lo)[tid] = x.p3;
+        cut.tell(lost);
     }
 };
 
@@ -1326,10 +1368,11 @@ MT_INLINE void mt_rw_load(mt_f32x4 (&a)[2], const float* __restrict__ arow, unsi
 // One 64-wide chunk: a holds its raw A values (pa applies the prologue) and,
 // step by step, receives those of the chunk at k_next (`more`): a step's loads
 // have the rest of this chunk and the steps before theirs in the next to land.
-template <typename P>
+template <bool LOOK, typename P>
 MT_INLINE void mt_rw_chunk(mt_f32x4 (&a)[4][2], const float* __restrict__ arow, unsigned k_next, bool more,
                            const float* __restrict__ hi, const float* __restrict__ lo, unsigned n0, P pa, unsigned lane,
-                           mt_lost& lost, mt_f32x16 (&acc)[1][2]) {
+                           mt_cut<LOOK> cut, mt_f32x16 (&acc)[1][2]) {
+    mt_lost lost = {};
     const mt_u32x4* __restrict__ h4 = reinterpret_cast<const mt_u32x4*>(hi) + n0 + (lane & 31u);
     const mt_u32x4* __restrict__ l4 = reinterpret_cast<const mt_u32x4*>(lo) + n0 + (lane & 31u);
     __builtin_amdgcn_s_setprio(1);
@@ -1340,13 +1383,14 @@ MT_INLINE void mt_rw_chunk(mt_f32x4 (&a)[4][2], const float* __restrict__ arow, 
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e / 4][e % 4] = pa(a[s][e / 4][e % 4]);
         if (more) mt_rw_load(a[s], arow, k_next, s);
-        const mt_split8 xa = mt_split(x[0], x[1], lost.a);
+        const mt_split8 xa = mt_split<LOOK>(x[0], x[1], lost.a);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const mt_split8 b = {h4[g + 32u * j], h4[1024u + g + 32u * j], l4[g + 32u * j]};
             acc[0][j] = mt_mfma_parts(xa, b, acc[0][j]);
         }
     }
+    cut.tell(lost);
     __builtin_amdgcn_s_setprio(0);
 }
 

@@ -598,6 +598,8 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         n_persistent = min(ceil_div(M, tile.tile_M), max(1, NUM_CUS * rr_resident_workgroups(tile) // batch))
     persistent = PersistentTiles(tile.tile_M, tile.tile_N, stream_k=stream_k, tile_K=tile.tile_K,
                                  row_blocks=local_rr) if n_persistent else None
+    if persistent is not None and tile.num_threads > 512:
+        config = dataclasses.replace(config, look_together=False)
     spread = load_spread(pro_a, pro_b)
     mainloop = MatmulMainloopFragment(
         tile_K=tile.tile_K,
@@ -624,7 +626,7 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         MatmulTileMappingFragment(persistent, xcd_rows=xcd_rows(grid_for(M, N, tile)) if persistent is None else 0,
                                   split=(parts, tile.tile_K) if parts > 1 else None),
         ThreadIndexFragment(tile),
-        MatmulSetupFragment(config, split=True),
+        MatmulSetupFragment(config, split=True, persistent=persistent is not None),
         mainloop,
         exact_retry(config, src_a, src_b, pro_a, pro_b, persistent=persistent is not None or parts > 1,
                     check=not aligned),

@@ -181,8 +181,8 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
     fragments = (
         MatmulTileMappingFragment(persistent, split=(parts, tile.tile_K) if parts > 1 else None),
         ThreadIndexFragment(tile),
-        MatmulSetupFragment(configs[0], accumulator_suffix=suffixes[0], split=True),
-        MatmulSetupFragment(configs[1], accumulator_suffix=suffixes[1], emit_thread_coords=False, split=True),
+        MatmulSetupFragment(configs[0], accumulator_suffix=suffixes[0], split=True, persistent=persistent is not None),
+        MatmulSetupFragment(configs[1], accumulator_suffix=suffixes[1], emit_thread_coords=False),
         *mainloops,
         *(
             exact_retry(configs[i], src_a[0 if shared else i], src_b[i], tf_a[0 if shared else i], tf_b[i],

@@ -20,7 +20,9 @@ FORMS = {
     "short": ((129, 8, 195), {}, "mt_mfma_tile<"),
     "ragged tile": ((129, 331, 195), {}, "mt_mfma_tile<"),
     "long k loop": ((512, 1024, 256), {"FILL": False}, "mt_mfma_tile_held<"),
+    "looking together": ((256, 512, 512), {"FILL": False}, "mt_k_loop(mt_cut<true>"),
     "summed in parts": ((256, 1024, 256), {}, "mt_part_i"),
+    "in parts, looking together": ((512, 1024, 1024), {}, "mt_k_loop(mt_cut<true>"),
     "stream-K": ((384, 512, 640), {"FILL": False}, "mt_sk_wait("),
     "row waves": ((256, 1024, 128), {}, "mt_rw_chunk("),
     "divided row waves": ((256, 1024, 128), {}, "mt_rw_chunk("),
@@ -28,6 +30,7 @@ FORMS = {
     "transposed operands": ((129, 331, 195), {}, "mt_mfma_tile<"),
     "pair": ((130, 333, 200), {}, "acc_1"),
     "pair of two left operands": ((130, 333, 200), {}, "acc_1"),
+    "pair, looking together": ((512, 512, 512), {"FILL": False}, "mt_k_loop(mt_cut<true>"),
 }
 
 
@@ -120,13 +123,11 @@ def test_small_values_of_a_softmax(name, monkeypatch):
     assert np.all(np.abs(got - scale * (a64 @ b64)) <= bound)
 
 
-@pytest.mark.parametrize("name", list(FORMS))
+@pytest.mark.parametrize("name", [f for f in FORMS if not f.startswith("pair")])  # (twice the sum is infinite)
 def test_largest_accumulators(name, monkeypatch):
     """-1.00586 is -1.0078 + 0.00195 in bf16 parts: added to 0.9995 of the largest
     float, the second part alone passes it, the product does not."""
     (M, K, N), text = _form(name, monkeypatch)
-    if name.startswith("pair"):
-        pytest.skip("twice the sum is infinite")
     print(f"split range {name} largest", flush=True)
     half = 0.5 if name.startswith("divided") else 1.0
     a, b = np.zeros((M, K), np.float32), np.zeros((K, N), np.float32)
