@@ -18,7 +18,7 @@ time, so the clocks have settled before the timed steps.  ``value`` =
 1.108 TFLOP / mean step time; ``roofline`` is the dominant kernel's (the one
 taking the largest share of the step).
 
-Also measured (``per_kernel``): C2 (one fused elementwise kernel), C3
+Also measured (``per_kernel``; whole records on stderr): C2 (one fused elementwise kernel), C3
 softmax (4 kernels), the 4096^3 matmul, C4 literal and the fused diamond
 variant, C5 attention (32 heads; each of the 5 per-head kernels launched
 once for all heads, ``api.run_batch``), each kernel against its roofline.
@@ -1026,7 +1026,8 @@ def headline_c4(args, flush, info) -> tuple[dict, dict]:
             "step_ms_min": round(float(np.min(step_ms)), 5),
             "step_ms_median": round(float(np.median(step_ms)), 5),
             "arithmetic": "fp32 products and sums; each factor as three bf16 parts (RNE), six exact products per "
-            "multiply-add on the bf16 matrix cores, accumulated in fp32 (error no larger than the fp32 MFMA's)",
+            "multiply-add on the bf16 matrix cores, accumulated in fp32 (error no larger than the fp32 MFMA's; fp32 "
+            "MFMAs where operands or sums leave the range this holds for)",
             "fraction_of_fp32_mfma_peak": round(tflops / FP32_MFMA_PEAK_TFLOPS, 4),
             "cache_flush_between_steps": flush is not None,
             "wall_ms_per_step_incl_flush": round(wall * 1e3 / args.steps, 4),
@@ -1058,6 +1059,14 @@ def headline_c4(args, flush, info) -> tuple[dict, dict]:
     made = prep.ops
     prep.release()
     return line, {"records": records, "made": made}
+
+
+def brief(line: dict) -> dict:
+    """The line with a few values per kernel: whoever captures stdout may keep only
+    its last 12000 characters.  Everything goes to stderr."""
+    keys = ("kernel", "config", "source_sha16", "ms_mean", "achieved", "unit", "frac")
+    kernels = [{k: r[k] for k in keys if k in r} for r in line["per_kernel"]]
+    return {**line, "per_kernel": kernels}
 
 
 def main() -> int:
@@ -1183,7 +1192,8 @@ def main() -> int:
         line["hbm_sweep"] = sweep_fits
     if only is None and not args.no_extra:
         line["end_to_end"] = end_to_end_runs()
-    print(json.dumps(line), flush=True)
+    log("[bench] details: " + json.dumps({"per_kernel": per_config}))
+    print(json.dumps(brief(line)), flush=True)
     return 0
 
 

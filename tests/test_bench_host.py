@@ -1,6 +1,8 @@
 """Host-side pieces of bench.py: the size-sweep fit and the read-ceiling
 kernel's launch contract (no GPU needed)."""
 
+import json
+
 import pytest
 
 import bench
@@ -93,3 +95,16 @@ def test_sensor_parsing_and_absence(tmp_path):
     with s:
         pass
     assert s.paths == {} and s.summary() is None
+
+
+def test_the_line_fits_what_is_kept_of_stdout():
+    """27 kernels with sensors were 24000 characters; 12000 are kept."""
+    sensor = {"min": 1715.0, "mean": 1753.8, "max": 1786.0, "samples": 32}
+    record = {"kernel": "elementwise_out_fused_longest", "config": "C4 MLP literal, gate fused (extension)",
+              "source_sha16": "5f01579684b4f1a4", "strategy": "matmul_epilogue_register", "grid": [1, 8, 1],
+              "threads": [1024, 1, 1], "ms_mean": 2.02421, "ms_min": 1.99672, "ms_median": 2.02468, "bound": "mfma",
+              "work": 369367187456.0, "achieved": 182.47, "peak": 416.66, "unit": "TFLOP/s", "frac": 0.4379,
+              "sensors": {name: sensor for name in ("power_w", "temp_c", "temp_mem_c", "sclk_mhz", "mclk_mhz")}}
+    line = {"value": 1.0, "config": "x" * 1500, "cpu_baseline": "x" * 3000, "per_kernel": [dict(record) for _ in range(27)]}
+    assert len(json.dumps(line)) > 20000 and len(json.dumps(bench.brief(line))) < 11500
+    assert bench.brief(line)["per_kernel"][0]["achieved"] == 182.47 and line["per_kernel"][0] == record
