@@ -427,7 +427,7 @@ def looking_wave(config: MatmulConfig) -> str | None:
     None: each for itself.  With loads through registers, which both would keep,
     (h1*s*h2) @ W3 spills (MLP block 6.15 against 6.94 ms), 2049 x 1111 x 3333 takes
     137 against 160 us; a persistent loop of 16 waves, out of registers with one
-    instance, 1993 against 2040 us (4096 x 4096 x 11008)."""
+    instance, 1932 against 2051 us (4096 x 4096 x 11008)."""
     tile = config.tile
     m, n = tile.sg_M, tile.sg_N
     if not config.look_together or min(m, n) == 1 or "pad" in (tile.a_layout, tile.b_layout) or tile.stages != 2:

@@ -29,9 +29,12 @@
 //   * mt_mfma_tile            one LDS k-chunk for a wave's WM x WN grid of 32x32
 //                             blocks: fp32 operands split into three bf16 parts
 //                             in registers (mt_split), six bf16 MFMAs per step
+//   * mt_own / mt_cut         what of the operands' low bits the split cut off,
+//                             noticed by each wave or by some for the others
 //   * mt_mfma_retry / mt_mfma_exact
-//                             the fp32 MFMAs a wave falls back to when the
-//                             split cannot represent its operands
+//                             the fp32 MFMAs a wave falls back to when its
+//                             results are not finite or too small for the
+//                             split, or the bits cut off could matter
 //   * mt_mfma_tile_f32        the same chunk on fp32 MFMAs (hand-composed kernels)
 //   * mt_rw_*                 row-owning waves for matmuls 128 columns wide
 //                             (split MFMAs, A in registers, B's parts in LDS)
@@ -425,7 +428,7 @@ struct mt_tile_rowvec {
             const unsigned idx = tid + i * NT;
             if (TOTAL % NT == 0 || idx < (unsigned)TOTAL) {
                 unsigned c;
-            const unsigned r = slot(tid, i, c);
+                const unsigned r = slot(tid, i, c);
                 lds[(r + 0u) * LD + c] = v[i].x;
                 lds[(r + 1u) * LD + c] = v[i].y;
                 lds[(r + 2u) * LD + c] = v[i].z;
@@ -967,6 +970,9 @@ MT_INLINE void mt_mfma_tile_f32(const float* __restrict__ As, const float* __res
 // cutting it off) gives x2 a sign of its own: the MFMA drops what lies far
 // below the accumulator's last bit, and with x2 y2 always of the product's
 // sign that added up (all-positive operands, K = 4096: 3.4e-6 instead of 5.9e-7).
+// (Three-part bf16 products: G. Henry, P. Tang, A. Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations",
+// ARITH 2019.)
 //
 // Why: the fp32 MFMA does 64 multiply-adds per cycle and SIMD, the bf16 one
 // 1024, so six of them have 2.7 times its rate.  Measured on MI355X, 4096^3:
@@ -995,8 +1001,8 @@ MT_INLINE void mt_mfma_tile_f32(const float* __restrict__ As, const float* __res
 // error of up to 2^-133 times whatever the other operand is.  Results do not show
 // that, so a split says whether it cut anything off (mt_lost): half a VALU operation
 // per element, in every wave or in one of each row and column of waves (mt_own,
-// mt_cut).  Measured on MI355X without and with it: 4096^3 686 -> 699 us, 4096 x
-// 4096 x 11008 1874 -> 1979, 1531 x 1000 x 3001 98 -> 104, C4 MLP 5.92 -> 6.04 ms.
+// mt_cut).  Measured on MI355X without and with it: 4096^3 661 -> 671 us, 4096 x
+// 4096 x 11008 1850 -> 1932, 1531 x 1000 x 3001 96 -> 102, C4 MLP 5.86 -> 5.99 ms.
 // Dearer were a running minimum and maximum of the operands held by every wave
 // (4096^3 737 us where the look in every wave took 712), or taken by every lane of
 // its share of the LDS tile (742), or a look at every fourth chunk branched to inside
@@ -1244,9 +1250,14 @@ MT_INLINE bool mt_mfma_retry(const mt_f32x16 (&acc)[WM][WN], const mt_lost& lost
 #pragma unroll
             for (int j = 0; j < WN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    odd |= !(__builtin_fabsf(acc[i][j][v]) >= least) &&
-                           32u * (unsigned)i + mt_acc_row(v, lane) < rows && 32u * (unsigned)j + (lane & 31u) < cols;
+                for (int v = 0; v < 16; ++v) {
+                    float x = acc[i][j][v];
+                    // else |x| is computed ahead for this and the check below: 29 spills
+                    // a tile (4096 x 4096 x 11008: 1993 us with them, 1932 without)
+                    asm volatile("" : "+v"(x));
+                    odd |= !(__builtin_fabsf(x) >= least) && 32u * (unsigned)i + mt_acc_row(v, lane) < rows &&
+                           32u * (unsigned)j + (lane & 31u) < cols;
+                }
     }
 #pragma unroll
     for (int i = 0; i < WM; ++i)
