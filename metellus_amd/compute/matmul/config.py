@@ -264,8 +264,11 @@ def _fill_candidates(M: int, N: int, min_waves: int, anchors: int) -> list[FillT
 @functools.lru_cache(maxsize=1024)
 def filled_parts(M: int, K: int, N: int, batch: int = 1) -> int:
     """Workgroups per tile of the least ``fill_time`` (one for batched programs and
-    fewer than FILL_PARTS_MIN_K k's).  It depends on the sizes alone: however a
-    product of these sizes is fused, its terms are added in the same order."""
+    fewer than FILL_PARTS_MIN_K k's).  It depends on the sizes alone, so that a
+    product adds its terms in the same order with any epilogue and as one of a pair
+    that shares its left operand.  Not where another kernel takes it: up to 64 rows
+    alone (skinny) but not as one of a pair, a prologue that divides by rows (never
+    in parts), a batch, 128 columns on row waves."""
     chunks = ceil_div(K, 32)
     best = (float("inf"), 1)
     for f in _fill_candidates(M, N, 1, 1):

@@ -114,6 +114,30 @@ def test_pair_sharing_a(parts, monkeypatch):
     np.testing.assert_allclose(z, ref, rtol=1e-4, atol=1e-2)
 
 
+def test_pair_of_few_rows():
+    """Alone, a product of up to 64 rows takes the skinny kernel (fp32 MFMAs, k's in
+    other groups); in a pair the tiles: both within an fp32 sum's rounding."""
+    rng = np.random.default_rng(18)
+    M, K, N = 48, 1040, 200
+    x, w1, w2 = (rng.standard_normal(s).astype(np.float32) for s in ((M, K), (K, N), (K, N)))
+    pair, one = Operations(), Operations()
+    for o in (pair, one):
+        o.from_numpy(x, "X")
+        o.from_numpy(w1, "W1")
+        o.matmul(a="X", b="W1", out="h1")
+    pair.from_numpy(w2, "W2")
+    pair.matmul(a="X", b="W2", out="h2")
+    pair.elementwise("add", out="z", operands=("h1", "h2"))
+    print("pair of few rows", flush=True)
+    (g,), (s,) = compile_program(pair), compile_program(one)
+    assert "mt_mfma_tile" in g.kernel.source.split('extern "C"')[-1]
+    assert "mt_sn_mainloop<" in s.kernel.source.split('extern "C"')[-1]
+    x64, a64 = x.astype(np.float64), np.abs(x.astype(np.float64))
+    unit = (K + 8) * 2.0**-24
+    assert np.all(np.abs(run(one).env["h1"] - x64 @ w1) <= unit * (a64 @ np.abs(w1)))
+    assert np.all(np.abs(run(pair).env["z"] - x64 @ (w1.astype(np.float64) + w2)) <= unit * (a64 @ (np.abs(w1) + np.abs(w2))))
+
+
 @pytest.mark.parametrize("a_view", [False, True])
 @pytest.mark.parametrize("kind", ["recip", "none", "row", "col"])
 def test_odd_prologues(kind, a_view):

@@ -1,8 +1,9 @@
-"""The held-group mainloop on the GPU: carrying each chunk's last group of 4
-k-steps over the barrier adds every product in the same k order, so every
-output is bit-identical to the plain mainloop's -- aligned, ragged (a
-partial last chunk, bounds checks), persistent with stream-K, a prologue
-division taking either of its two k loops, and batched attention."""
+"""The two renderings of the mainloop, ``mt_mfma_tile_held`` for long k loops and
+``mt_mfma_tile``, on the GPU: the same products in the same k order (a chunk
+leaves nothing to the next since the split's parts took the registers), so every
+output is bit-identical, and within the rounding of an fp32 sum of float64 --
+aligned, ragged (a partial last chunk, bounds checks), persistent with stream-K,
+a prologue division taking either of its two k loops, and batched attention."""
 
 from __future__ import annotations
 
@@ -13,6 +14,7 @@ from metellus_amd.api import run, run_batch
 from metellus_amd.orchestrator import Operations
 from metellus_amd.orchestrator.assembly import matmul as mm
 from tests import gpu_cases
+from tests.matmul_check import U32, accumulation_bound
 
 pytestmark = pytest.mark.gpu
 
@@ -65,6 +67,13 @@ def test_held_matches_plain_mainloop(case, monkeypatch):
             assert "mt_sk_wait(" in body
         got[held] = res.env[out]
     np.testing.assert_array_equal(got[True], got[False], err_msg=case)
+    if "stream-K" not in case and "per-element" not in case:  # (the whole stream-K output: test_gpu_full_size)
+        up = _CASES[case]().uploads
+        a, b = (up["E"].astype(np.float64) / up["s"].astype(np.float64)[:, None], up["V"]) if out == "Y" else (up["A"], up["B"])
+        a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+        # a divided operand within 2 ulp, the products and sums of matmul_check
+        bound = (accumulation_bound(a.shape[1]) + 4 * U32) * (np.abs(a) @ np.abs(b))
+        assert np.all(np.abs(got[True] - a @ b) <= bound)
     if "per-element" not in case:
         assert np.all(np.isfinite(got[True]))
 

@@ -1,7 +1,7 @@
-"""The held-group mainloop (``MatmulMainloopFragment.held``): each k-chunk's
-last group of 4 k-steps is carried over the barrier into the next chunk.
-Checked on the CPU: which kernels get it, the code it renders, and that the
-kernels compile."""
+"""The long mainloop's rendering (``MatmulMainloopFragment.held``,
+``mt_mfma_tile_held``) on the CPU: which kernels get it, the code around each
+k-chunk, and that the kernels compile.  With fp32 MFMAs a chunk left its last
+group of 4 k-steps to the next; with split products it leaves nothing."""
 
 from __future__ import annotations
 
