@@ -335,6 +335,17 @@ def resident_workgroups(t: TileConfig, anchors: int = 1, extra_lds: int = 0) -> 
     return max(1, min(by_lds, by_vgpr))
 
 
+LOOK_LDS_BYTES = 512  # the words of waves looking for each other, as LDS is allocated
+
+
+def look_words_fit(t: TileConfig, anchors: int = 1, extra_lds: int = 0) -> bool:
+    """Whether those words leave a compute unit as many workgroups of tile ``t``: the
+    operand tiles of 64x64 fill its LDS five times, a pair's of 64x128 twice and of
+    128x256 once."""
+    lds = tile_lds_bytes(t, anchors) + extra_lds
+    return LDS_BYTES // lds == LDS_BYTES // (lds + LOOK_LDS_BYTES)
+
+
 def persistent_workgroups(M: int, N: int, t: TileConfig, batch: int = 1, anchors: int = 1) -> int | None:
     """Workgroups per problem for a persistent tile loop, or None when every
     tile of every problem gets a resident workgroup in one round anyway."""

@@ -22,6 +22,7 @@ kernel parameter.
 from __future__ import annotations
 
 import dataclasses
+import math
 
 from metellus_amd.compute.fragments import BarrierFragment, CodegenContext, lds_decl
 from metellus_amd.compute.matmul import config as _config
@@ -35,6 +36,7 @@ from metellus_amd.compute.matmul.config import (
     fills,
     grid_for,
     is_aligned_shape,
+    look_words_fit,
     persistent_workgroups,
     resident_workgroups,
     select_filled,
@@ -598,7 +600,8 @@ def assemble_matmul(decision: DecisionView, function_name: str | None, batch: in
         n_persistent = min(ceil_div(M, tile.tile_M), max(1, NUM_CUS * rr_resident_workgroups(tile) // batch))
     persistent = PersistentTiles(tile.tile_M, tile.tile_N, stream_k=stream_k, tile_K=tile.tile_K,
                                  row_blocks=local_rr) if n_persistent else None
-    if persistent is not None and tile.num_threads > 512:
+    rr_lds = 4 * math.prod(rr_lds_shape(tile)) if red is not None else 0
+    if persistent is not None and tile.num_threads > 512 or not look_words_fit(tile, extra_lds=rr_lds):
         config = dataclasses.replace(config, look_together=False)
     spread = load_spread(pro_a, pro_b)
     mainloop = MatmulMainloopFragment(

@@ -22,6 +22,7 @@ from metellus_amd.compute.fragments import BarrierFragment, CodegenContext, lds_
 from metellus_amd.compute.matmul.config import (
     grid_for,
     is_aligned_shape,
+    look_words_fit,
     persistent_workgroups,
     select_filled,
     select_tile_config,
@@ -121,6 +122,7 @@ def assemble_multi_anchor(decision: DecisionView, function_name: str | None, bat
             c_buffer_name=param_name(out_key),
             a_tile_name="A_tile" if shared else f"A{i}_tile",
             b_tile_name=f"B{i}_tile",
+            look_together=look_words_fit(tile, 2),
         )
         for i in range(2)
     )

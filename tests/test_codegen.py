@@ -9,6 +9,7 @@ import pytest
 import numpy as np
 
 from metellus_amd.api import compile_program
+from metellus_amd.compute.matmul import config
 from metellus_amd.orchestrator import Operations
 from metellus_amd.runtime import hip_backend
 from tests import gpu_cases
@@ -341,3 +342,30 @@ def test_tiles_of_plain_products(M, K, N, tile, grid):
         assert "mt_t += gridDim.x" in body or "mt_sk" in body
     else:
         assert g.grid == grid
+
+
+@pytest.mark.parametrize("pair", [False, True])
+def test_looking_for_each_other_costs_no_resident_workgroup(pair, monkeypatch):
+    # the words of waves that look for each other are no LDS plan's: a tile whose
+    # operands fill a compute unit's LDS a whole number of times does without
+    shared = []
+    for tile in dict.fromkeys((*config.SINGLE_ANCHOR_TILES, *config.DUAL_ANCHOR_TILES, *config.WIDE_TILES)):
+        monkeypatch.setattr(config, "FORCE_TILE", tile)
+        ops = Operations()
+        ops.input("A", (1024, 256))
+        for i in range(1 + pair):
+            ops.input(f"B{i}", (256, 1024))
+            ops.matmul(a="A", b=f"B{i}", out=f"C{i}")
+        if pair:
+            ops.elementwise("add", out="E", operands=("C0", "C1"))
+        if config.tile_lds_bytes(tile, 1 + pair) > config.LDS_BYTES:
+            continue
+        (g,) = compile_program(ops)
+        body = g.kernel.source.split('extern "C"')[-1]
+        arrays = re.findall(r"__shared__ (?:alignas\(16\) )?(?:float|unsigned) (\w+)((?:\[\d+\])+);", body)
+        lds = {name: 4 * int(np.prod([int(d) for d in re.findall(r"\d+", dims)])) for name, dims in arrays}
+        tiles = sum(n for name, n in lds.items() if name.endswith("_tile"))
+        used = -(-sum(lds.values()) // 512) * 512
+        assert used <= config.LDS_BYTES and config.LDS_BYTES // used == config.LDS_BYTES // tiles, (tile, lds)
+        shared.append("mt_cut_words" in lds)
+    assert any(shared) and not all(shared)
