@@ -22,7 +22,7 @@ FORMS = {
     "long k loop": ((512, 1024, 256), {"FILL": False}, "mt_mfma_tile_held<"),
     "looking together": ((256, 512, 512), {"FILL": False}, "mt_k_loop(mt_cut<true>"),
     "summed in parts": ((256, 1024, 256), {}, "mt_part_i"),
-    "in parts, looking together": ((512, 1024, 1024), {}, "mt_k_loop(mt_cut<true>"),
+    "in parts, looking together": ((1024, 1024, 1024), {}, "mt_k_loop(mt_cut<true>"),
     "stream-K": ((384, 512, 640), {"FILL": False}, "mt_sk_wait("),
     "row waves": ((256, 1024, 128), {}, "mt_rw_chunk("),
     "divided row waves": ((256, 1024, 128), {}, "mt_rw_chunk("),
